@@ -24,6 +24,8 @@ struct Scene {
     uint32_t* obj_xf = nullptr;
     float4* xf_ps = nullptr;
     float4* xf_q = nullptr;
+    float4* world = nullptr;           // world-space bounding spheres' centres and the scale, per object
+    uint32_t* xf_stamp = nullptr;      // [n_transforms] xf_version of each transform's last update (shared transforms)
     float4* surf_sphere = nullptr;
     uint2* surf_lod = nullptr;
     float* lod_error = nullptr;
@@ -53,8 +55,8 @@ struct Scene {
     // transform-update staging (bz_scene_transform_staging, also behind bz_scene_update_transforms): two pinned slots
     // [ids | 32-byte MeshTransforms], used in turn
     struct XfSlot {
-        uint8_t* host = nullptr;       // pinned, read by the scatter kernel: cap ids, then cap transforms at xf_offset
-        uint32_t* dev_ids = nullptr;   // [cap] device copy of the committed ids
+        uint8_t* host = nullptr;       // pinned, read by a kernel: cap ids, then cap transforms at xf_offset
+        float4* dev = nullptr;         // device copy of the committed updates: 2 cap float4 of transforms, then cap ids
         uint32_t cap = 0;
         size_t xf_offset = 0;
         hipEvent_t done = nullptr;     // the last commit from this slot completed

@@ -69,14 +69,14 @@ Pyramid* Ctx::pyramid(bz_pyramid h)
 
 Scene::~Scene()
 {
-    void* ps[] = { obj_surf, obj_surf16, obj_xf, xf_ps, xf_q, surf_sphere, surf_lod, lod_error, lod_draw, lod_cluster, vis,
+    void* ps[] = { obj_surf, obj_surf16, obj_xf, xf_ps, xf_q, world, xf_stamp, surf_sphere, surf_lod, lod_error, lod_draw, lod_cluster, vis,
                    cl_sphere, cl_cone, cl_draw, cache.sph, cache.meta, cache.counts, xf_winner };
     for (XfSlot& x : xf_slot)
         if (x.done) (void)hipEventSynchronize(x.done);
     for (void* p : ps)
         if (p) (void)hipFree(p);
     for (XfSlot& x : xf_slot) {
-        if (x.dev_ids) (void)hipFree(x.dev_ids);
+        if (x.dev) (void)hipFree(x.dev);
         if (x.host) (void)hipHostFree(x.host);
         if (x.done) (void)hipEventDestroy(x.done);
     }
@@ -191,6 +191,7 @@ SceneDev Scene::dev() const
     d.obj_xf = obj_xf;
     d.xf_ps = xf_ps;
     d.xf_q = xf_q;
+    d.world = world;
     d.surf_sphere = surf_sphere;
     d.surf_lod = surf_lod;
     d.lod_error = lod_error;
@@ -456,6 +457,7 @@ bz_status bz_scene_create(bz_ctx* ctx, const bz_RenderObject* objects, uint32_t 
     if (!identity && (st = up((void**)&s->obj_xf, xf_ids.data(), xf_ids.size() * 4))) return st;
     if ((st = up((void**)&s->xf_ps, ps.data(), ps.size() * sizeof(float4)))) return st;
     if ((st = up((void**)&s->xf_q, q.data(), q.size() * sizeof(float4)))) return st;
+    if ((st = up((void**)&s->world, nullptr, (size_t)n_objects * sizeof(float4)))) return st;
     if ((st = up((void**)&s->surf_sphere, sph.data(), sph.size() * sizeof(float4)))) return st;
     if ((st = up((void**)&s->surf_lod, slod.data(), slod.size() * sizeof(uint2)))) return st;
     if ((st = up((void**)&s->lod_error, lerr.data(), lerr.size() * 4))) return st;
@@ -464,8 +466,9 @@ bz_status bz_scene_create(bz_ctx* ctx, const bz_RenderObject* objects, uint32_t 
     if ((st = up((void**)&s->vis, nullptr, (size_t)std::max<uint32_t>(n_objects, 1u) * 4))) return st;
     // visibility starts at zero (vulkanRendererSetup.cpp:349)
     hipError_t e = launch_fill_u32(s->vis, 0u, std::max<uint32_t>(n_objects, 1u), nullptr);
+    if (e == hipSuccess) e = launch_world_spheres(s->dev(), s->world, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (e != hipSuccess) return ctx->hip_fail(e, "visibility fill");
+    if (e != hipSuccess) return ctx->hip_fail(e, "visibility fill, world-space spheres");
     const bz_scene h = ++ctx->next_handle;
     ctx->scenes[h] = std::move(s);
     *out = h;
@@ -558,14 +561,14 @@ bz_status bz_scene_transform_staging(bz_ctx* ctx, bz_scene scene, uint32_t capac
     }
     if (x.cap < capacity) {
         if (x.host) (void)hipHostFree(x.host);
-        if (x.dev_ids) (void)hipFree(x.dev_ids);
+        if (x.dev) (void)hipFree(x.dev);
         x.host = nullptr;
-        x.dev_ids = nullptr;
+        x.dev = nullptr;
         x.cap = 0;
         const size_t off = ((size_t)capacity * 4 + 255) / 256 * 256;
         const size_t bytes = off + (size_t)capacity * sizeof(bz_MeshTransform);
         hipError_t e = hipHostMalloc((void**)&x.host, bytes, hipHostMallocDefault);  // pinned, device-readable
-        if (e == hipSuccess) e = hipMalloc((void**)&x.dev_ids, (size_t)capacity * 4);
+        if (e == hipSuccess) e = hipMalloc((void**)&x.dev, (size_t)capacity * (sizeof(bz_MeshTransform) + 4));
         if (e == hipSuccess && !s->xf_winner) {
             e = hipMalloc((void**)&s->xf_winner, (size_t)s->n_transforms * 4);
             if (e == hipSuccess) e = hipMemset(s->xf_winner, 0, (size_t)s->n_transforms * 4);
@@ -574,6 +577,15 @@ bz_status bz_scene_transform_staging(bz_ctx* ctx, bz_scene scene, uint32_t capac
                 s->xf_winner = nullptr;
             }
         }
+        if (e == hipSuccess && s->obj_xf && !s->xf_stamp) {  // zero is no update's stamp
+            e = hipMalloc((void**)&s->xf_stamp, (size_t)s->n_transforms * 4);
+            if (e == hipSuccess) e = hipMemset(s->xf_stamp, 0, (size_t)s->n_transforms * 4);
+            if (e != hipSuccess && s->xf_stamp) {
+                (void)hipFree(s->xf_stamp);
+                s->xf_stamp = nullptr;
+            }
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the clears, before a commit on any stream
         if (e == hipSuccess && !x.done) e = hipEventCreateWithFlags(&x.done, hipEventDisableTiming);
         if (e != hipSuccess) return ctx->hip_fail(e, "transform staging slot");
         x.cap = capacity;
@@ -600,11 +612,13 @@ bz_status bz_scene_commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, vo
     ++s->xf_version;  // frame-cache survivors recorded before this update no longer apply
     hipError_t e = hipSuccess;
     if (n) {
-        // the kernels read the pinned slot directly over the host link (ids once, records once; no staging copy)
+        // a kernel reads the pinned slot over the host link, ids and records once
+        // (a stamp repeats after 2^32 - 1 updates, and then only has spheres recomputed that need not be)
+        const uint32_t stamp = (uint32_t)(s->xf_version % 0xffffffffull) + 1u;
+        const XfTarget to{ s->dev(), s->xf_ps, s->xf_q, s->world, s->xf_winner, s->xf_stamp, stamp };
         e = launch_scatter_staged_transforms(reinterpret_cast<const uint32_t*>(x.host),
-                                             reinterpret_cast<const float4*>(x.host + x.xf_offset), n,
-                                             s->n_transforms, x.dev_ids, s->xf_winner, s->xf_ps, s->xf_q, sc->err,
-                                             st);
+                                             reinterpret_cast<const float4*>(x.host + x.xf_offset), n, to, x.dev,
+                                             reinterpret_cast<uint32_t*>(x.dev + 2 * (size_t)x.cap), sc->err, st);
     }
     if (e == hipSuccess) e = hipEventRecord(x.done, st);
     if (e != hipSuccess) return ctx->hip_fail(e, "staged transform update");

@@ -32,14 +32,14 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, uint32_t lane)
     return v;
 }
 
-// Small tables staged in LDS per workgroup when they fit: surface spheres and LOD ranges (512 surfaces, 12 KiB),
+// Small tables staged in LDS per workgroup when they fit: surface radii and LOD ranges (512 surfaces, 6 KiB),
 // LOD errors (2048 LODs, 8 KiB) and the pyramid's level offsets. Larger tables are gathered from global memory.
 constexpr uint32_t kLdsSurfaces = 512;
 constexpr uint32_t kLdsLods = 2048;
 
 template <int BLOCK, int ITEMS>
 struct TileSmem {
-    float4 surf[kLdsSurfaces];
+    float surf_rad[kLdsSurfaces];
     uint2 surf_lod[kLdsSurfaces];
     float lod_err[kLdsLods];
     float4 cand[BLOCK];               // per-wave compaction area: one chunk of 64 entries per wave
@@ -86,7 +86,7 @@ template <int ITEMS>
 struct Streams {
     uint32_t gi[ITEMS], vis[ITEMS], surf[ITEMS];
     bool valid[ITEMS], active[ITEMS];
-    float4 ps[ITEMS], q[ITEMS];
+    float4 w[ITEMS];  // world-space centre, scale
 };
 
 // Loads of the per-object streams. NT: marked non-temporal (streaming, evicted first), for the passes that read each
@@ -132,10 +132,10 @@ __device__ __forceinline__ void issue_vis(const CullJob& J, uint32_t tile_in_job
     }
 }
 
-// The surface-id and transform streams: for every object, or in EARLY only for last-frame-visible ones (which waits
+// The surface-id and world-space sphere streams: for every object, or in EARLY only for last-frame-visible ones (which waits
 // for the visibility stream first).
 // ALL (EARLY recording a frame cache): every object's streams are loaded, not only the last-frame-visible ones.
-template <int ITEMS, int MODE, bool XF_ID, bool ALL = false, bool NT = false>
+template <int ITEMS, int MODE, bool ALL = false, bool NT = false>
 __device__ __forceinline__ void issue_objects(const CullJob& J, Streams<ITEMS>& s)
 {
     const SceneDev& S = J.scene;
@@ -143,28 +143,26 @@ __device__ __forceinline__ void issue_objects(const CullJob& J, Streams<ITEMS>& 
     for (int k = 0; k < ITEMS; ++k) {
         s.active[k] = s.valid[k] && (MODE != MODE_EARLY || s.vis[k] != 0u);
         s.surf[k] = 0u;
-        s.ps[k] = s.q[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s.w[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         if (MODE != MODE_EARLY || ALL || s.active[k]) {
-            const uint32_t x = XF_ID ? s.gi[k] : stream_load<NT>(S.obj_xf + s.gi[k]);
             s.surf[k] = S.obj_surf16 ? (uint32_t)stream_load<NT>(S.obj_surf16 + s.gi[k])
                                      : stream_load<NT>(S.obj_surf + s.gi[k]);
-            s.ps[k] = stream_load<NT>(S.xf_ps + x);
-            s.q[k] = stream_load<NT>(S.xf_q + x);
+            s.w[k] = stream_load<NT>(S.world + s.gi[k]);
         }
     }
 }
 
-template <int BLOCK, int ITEMS, int MODE, bool XF_ID, bool ALL = false, bool NT = false>
+template <int BLOCK, int ITEMS, int MODE, bool ALL = false, bool NT = false>
 __device__ __forceinline__ void issue_tile(const CullJob& J, uint32_t tile_in_job, Streams<ITEMS>& s)
 {
     issue_vis<BLOCK, ITEMS, MODE, NT>(J, tile_in_job, s);
-    issue_objects<ITEMS, MODE, XF_ID, ALL, NT>(J, s);
+    issue_objects<ITEMS, MODE, ALL, NT>(J, s);
 }
 
-// Small tables into LDS (surface spheres and LOD ranges, LOD errors) plus the pyramid's level offsets. All loads of a
+// Small tables into LDS (surface radii and LOD ranges, LOD errors) plus the pyramid's level offsets. All loads of a
 // thread are issued before its first LDS write. The caller places the barrier.
 template <int BLOCK, int ITEMS>
 __device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, ITEMS>& sm, bool lds_tab)
@@ -173,14 +171,14 @@ __device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, I
     const SceneDev& S = J.scene;
     if (lds_tab) {
         constexpr int SPT = (kLdsSurfaces + BLOCK - 1) / BLOCK, LPT = (kLdsLods + BLOCK - 1) / BLOCK;
-        float4 t_sph[SPT];
+        float t_rad[SPT];
         uint2 t_lod[SPT];
         float t_err[LPT];
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             const uint32_t t = tid + (uint32_t)j * BLOCK;
             const uint32_t tt = t < S.n_surfaces ? t : 0u;
-            t_sph[j] = S.surf_sphere[tt];
+            t_rad[j] = S.surf_sphere[tt].w;
             t_lod[j] = S.surf_lod[tt];
         }
 #pragma unroll
@@ -192,7 +190,7 @@ __device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, I
         for (int j = 0; j < SPT; ++j) {
             const uint32_t t = tid + (uint32_t)j * BLOCK;
             if (t < S.n_surfaces) {
-                sm.surf[t] = t_sph[j];
+                sm.surf_rad[t] = t_rad[j];
                 sm.surf_lod[t] = t_lod[j];
             }
         }
@@ -234,22 +232,21 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
     const uint32_t pass = J.pass;
     const SceneDev& S = J.scene;
 
-    float4 sph[ITEMS];
+    float cx[ITEMS], cy[ITEMS], cz[ITEMS], rad[ITEMS];
     if (lds_tab) {
 #pragma unroll
-        for (int k = 0; k < ITEMS; ++k) sph[k] = sm.surf[s.surf[k]];
+        for (int k = 0; k < ITEMS; ++k) rad[k] = sm.surf_rad[s.surf[k]];
     } else {
 #pragma unroll
-        for (int k = 0; k < ITEMS; ++k) sph[k] = S.surf_sphere[s.surf[k]];
+        for (int k = 0; k < ITEMS; ++k) rad[k] = S.surf_sphere[s.surf[k]].w;
     }
 
     // ---- sphere -> view space + frustum for every object
-    float cx[ITEMS], cy[ITEMS], cz[ITEMS], rad[ITEMS];
     bool vis_new[ITEMS], emit[ITEMS], frus[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-        sphere_to_view(J.view, sph[k].x, sph[k].y, sph[k].z, sph[k].w, s.ps[k].x, s.ps[k].y, s.ps[k].z, s.ps[k].w,
-                       s.q[k].x, s.q[k].y, s.q[k].z, s.q[k].w, cx[k], cy[k], cz[k], rad[k]);
+        world_to_view(J.view, s.w[k].x, s.w[k].y, s.w[k].z, cx[k], cy[k], cz[k]);
+        rad[k] = rad[k] * s.w[k].w;
         if constexpr (CACHE) {
             frus[k] = s.valid[k] && frustum_visible(J.view, cx[k], cy[k], cz[k], rad[k]);
             vis_new[k] = frus[k] && s.active[k];
@@ -324,7 +321,7 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
         for (int k = 0; k < ITEMS; ++k)
             if (lsel[k] && eslot[k] - c0 < 64u) {
                 cand[eslot[k] - c0] = make_float4(cx[k], cy[k], cz[k], rad[k]);
-                cand2[eslot[k] - c0] = make_uint2(__float_as_uint(s.ps[k].w), s.surf[k]);
+                cand2[eslot[k] - c0] = make_uint2(__float_as_uint(s.w[k].w), s.surf[k]);
             }
         wave_lds_sync();
         if (c0 + lane < ne) {
@@ -430,7 +427,7 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
 }
 
 // One tile, loads and decision (non-persistent form, used by the batched kernel and the cluster object pass).
-template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool XF_ID, bool LDS_TAB, bool CL = false>
+template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false>
 __device__ __forceinline__ void decide_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t* counts,
                                             uint2* staging, TileSmem<BLOCK, ITEMS>& sm, uint32_t* ccounts = nullptr)
 {
@@ -438,9 +435,9 @@ __device__ __forceinline__ void decide_tile(const CullJob& J, uint32_t tile_in_j
     constexpr bool NT = MODE == MODE_OTHER && !HIZ;  // PLAIN / ONPC: streamed once, no Hi-Z
     Streams<ITEMS> s;
     issue_vis<BLOCK, ITEMS, MODE, NT>(J, tile_in_job, s);
-    if (MODE != MODE_EARLY) issue_objects<ITEMS, MODE, XF_ID, false, NT>(J, s);
+    if (MODE != MODE_EARLY) issue_objects<ITEMS, MODE, false, NT>(J, s);
     stage_tables<BLOCK, ITEMS>(J, sm, lds_tab);
-    if (MODE == MODE_EARLY) issue_objects<ITEMS, MODE, XF_ID, false, NT>(J, s);
+    if (MODE == MODE_EARLY) issue_objects<ITEMS, MODE, false, NT>(J, s);
     __syncthreads();  // staged tables visible
     process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, CL>(J, gtile, s, counts, staging, ccounts, sm, NoPrefetch{});
 }
@@ -450,7 +447,7 @@ __device__ __forceinline__ void decide_tile(const CullJob& J, uint32_t tile_in_j
 // decided (two register sets, alternating, so no register copy waits on a load in flight).
 // INST: workgroup b takes the contiguous tiles of chunk b instead (chunk_range), counts
 // its emitting objects per LOD in LDS and writes the counts to row b of ih.hist.
-template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool XF_ID, bool LDS_TAB, bool CACHE = false, bool INST = false>
+template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CACHE = false, bool INST = false>
 __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* counts, uint2* staging, FrameCacheDev fc,
                                                        InstHistDev ih)
 {
@@ -469,7 +466,7 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
         step = gridDim.x;
     }
     Streams<ITEMS> A, B;
-    issue_tile<BLOCK, ITEMS, MODE, XF_ID, CACHE, NT>(J, t, A);
+    issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, t, A);
     stage_tables<BLOCK, ITEMS>(J, sm, lds_tab);
     __syncthreads();
     while (true) {
@@ -481,7 +478,7 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
             // fetched again).
             process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, A, counts, staging, nullptr, sm,
                                                                                 [&]() {
-                issue_tile<BLOCK, ITEMS, MODE, XF_ID, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, B);
+                issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, B);
             }, fc, s_hist);
             t = tn;
             if (t >= t_end) break;
@@ -490,7 +487,7 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
             const uint32_t tn = t + step;
             process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, B, counts, staging, nullptr, sm,
                                                                                 [&]() {
-                issue_tile<BLOCK, ITEMS, MODE, XF_ID, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, A);
+                issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, A);
             }, fc, s_hist);
             t = tn;
             if (t >= t_end) break;
@@ -545,55 +542,35 @@ __global__ __launch_bounds__(BLOCK) void decide_batch_kernel(const CullJob* __re
     }
     const CullJob& sjob = jobs[__builtin_amdgcn_readfirstlane(jb)];
     const uint32_t tt = t - sjob.tile_start;
-    const bool xf_id = sjob.scene.obj_xf == nullptr;
-    // identity scenes have no transform-index stream (obj_xf == nullptr): XF_ID must follow it in every variant
-#define BZ_DECIDE_TILE(M, HZ)                                                                                     \
-    if (xf_id) decide_tile<BLOCK, ITEMS, M, HZ, true, false>(sjob, tt, t, counts, staging, sm);                  \
-    else decide_tile<BLOCK, ITEMS, M, HZ, false, false>(sjob, tt, t, counts, staging, sm);
-    if (sjob.pass == PASS_LATE) {
-        BZ_DECIDE_TILE(MODE_LATE, true)
-    } else if (sjob.hiz) {
-        BZ_DECIDE_TILE(MODE_OTHER, true)
-    } else {
-        BZ_DECIDE_TILE(MODE_OTHER, false)
-    }
-#undef BZ_DECIDE_TILE
+    if (sjob.pass == PASS_LATE) decide_tile<BLOCK, ITEMS, MODE_LATE, true, false>(sjob, tt, t, counts, staging, sm);
+    else if (sjob.hiz) decide_tile<BLOCK, ITEMS, MODE_OTHER, true, false>(sjob, tt, t, counts, staging, sm);
+    else decide_tile<BLOCK, ITEMS, MODE_OTHER, false, false>(sjob, tt, t, counts, staging, sm);
 }
 
 // Cluster object pass (PreClusterDrawCull.comp.glsl:13-47): the PLAIN (or, with a pyramid, TEMPORAL) decision of
 // every object, its LOD, and per tile the number of emitting objects (counts), their (objectId, LOD) list (staging)
 // and the sum of their LOD cluster counts (ccounts). One workgroup per tile.
-template <int BLOCK, int ITEMS, bool HIZ, bool XF_ID, bool LDS_TAB>
+template <int BLOCK, int ITEMS, bool HIZ, bool LDS_TAB>
 __global__ __launch_bounds__(BLOCK) void decide_cluster_kernel(CullJob J, uint32_t* counts, uint2* staging,
                                                                uint32_t* ccounts)
 {
     __shared__ TileSmem<BLOCK, ITEMS> sm;
-    decide_tile<BLOCK, ITEMS, MODE_OTHER, HIZ, XF_ID, LDS_TAB, true>(J, blockIdx.x, blockIdx.x, counts, staging, sm,
-                                                                     ccounts);
+    decide_tile<BLOCK, ITEMS, MODE_OTHER, HIZ, LDS_TAB, true>(J, blockIdx.x, blockIdx.x, counts, staging, sm, ccounts);
 }
 
 template <int BLOCK, int ITEMS>
 hipError_t launch_cluster_objects_t(const CullJob& job, const CompactScratch& s, uint32_t* ccounts, hipStream_t st)
 {
     const bool lds = job.scene.n_surfaces <= kLdsSurfaces && job.scene.n_lods <= kLdsLods;
-    const bool xf_id = job.scene.obj_xf == nullptr;
     const dim3 g(job.n_tiles), b(BLOCK);
-#define BZ_CL_LAUNCH(HZ)                                                                                           \
-    if (xf_id) {                                                                                                   \
-        if (lds) hipLaunchKernelGGL((decide_cluster_kernel<BLOCK, ITEMS, HZ, true, true>), g, b, 0, st, job,      \
-                                    s.counts, s.staging, ccounts);                                                 \
-        else hipLaunchKernelGGL((decide_cluster_kernel<BLOCK, ITEMS, HZ, true, false>), g, b, 0, st, job,         \
-                                s.counts, s.staging, ccounts);                                                     \
-    } else {                                                                                                       \
-        if (lds) hipLaunchKernelGGL((decide_cluster_kernel<BLOCK, ITEMS, HZ, false, true>), g, b, 0, st, job,     \
-                                    s.counts, s.staging, ccounts);                                                 \
-        else hipLaunchKernelGGL((decide_cluster_kernel<BLOCK, ITEMS, HZ, false, false>), g, b, 0, st, job,        \
-                                s.counts, s.staging, ccounts);                                                     \
-    }
+#define BZ_CL_LAUNCH(HZ, LT) \
+    hipLaunchKernelGGL((decide_cluster_kernel<BLOCK, ITEMS, HZ, LT>), g, b, 0, st, job, s.counts, s.staging, ccounts)
     if (job.hiz) {
-        BZ_CL_LAUNCH(true)
+        if (lds) BZ_CL_LAUNCH(true, true);
+        else BZ_CL_LAUNCH(true, false);
     } else {
-        BZ_CL_LAUNCH(false)
+        if (lds) BZ_CL_LAUNCH(false, true);
+        else BZ_CL_LAUNCH(false, false);
     }
 #undef BZ_CL_LAUNCH
     return hipGetLastError();
@@ -911,7 +888,7 @@ hipError_t launch_late_cached_t(const CullJob& job, const CompactScratch& s, con
 }
 
 // Persistent grid: `per_cu` workgroups per CU, or (per_cu == 0) as many as are resident at once per CU.
-template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool XF_ID, bool LDS_TAB, bool CACHE = false, bool INST = false>
+template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CACHE = false, bool INST = false>
 void launch_decide(const CullJob& job, uint32_t n_cu, uint32_t per_cu, uint32_t* counts, uint2* staging, hipStream_t st,
                    const FrameCacheDev& fc = FrameCacheDev{}, const InstHistDev& ih = InstHistDev{})
 {
@@ -919,7 +896,7 @@ void launch_decide(const CullJob& job, uint32_t n_cu, uint32_t per_cu, uint32_t*
     if (resident == 0) {
         int r = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &r, decide_kernel<BLOCK, ITEMS, MODE, HIZ, XF_ID, LDS_TAB, CACHE, INST>, BLOCK, 0) != hipSuccess ||
+                &r, decide_kernel<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, CACHE, INST>, BLOCK, 0) != hipSuccess ||
             r < 1)
             r = 1;
         resident = r;
@@ -928,7 +905,7 @@ void launch_decide(const CullJob& job, uint32_t n_cu, uint32_t per_cu, uint32_t*
     if (grid > job.n_tiles) grid = job.n_tiles;
     if (grid == 0) grid = 1;
     if (INST) grid = job.n_tiles ? (job.n_tiles - ih.n_long) / ih.tiles_per_chunk : 1;  // one chunk per workgroup
-    hipLaunchKernelGGL((decide_kernel<BLOCK, ITEMS, MODE, HIZ, XF_ID, LDS_TAB, CACHE, INST>), dim3((uint32_t)grid),
+    hipLaunchKernelGGL((decide_kernel<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, CACHE, INST>), dim3((uint32_t)grid),
                        dim3(BLOCK), 0, st, job, counts, staging, fc, ih);
 }
 
@@ -940,7 +917,7 @@ uint32_t inst_resident()
     if (resident == 0) {
         int r = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &r, decide_kernel<BLOCK, ITEMS, MODE_OTHER, false, true, true, false, true>, BLOCK, 0) != hipSuccess ||
+                &r, decide_kernel<BLOCK, ITEMS, MODE_OTHER, false, true, false, true>, BLOCK, 0) != hipSuccess ||
             r < 1)
             r = 1;
         resident = r;
@@ -955,17 +932,10 @@ hipError_t launch_decide_inst_t(const CullJob& job, const CompactScratch& s, uin
 {
     const bool lds = job.scene.n_surfaces <= kLdsSurfaces && job.scene.n_lods <= kLdsLods;
     const FrameCacheDev none{};
-    if (job.scene.obj_xf == nullptr) {
-        if (lds) launch_decide<BLOCK, ITEMS, MODE_OTHER, false, true, true, false, true>(job, n_cu, per_cu, s.counts,
-                                                                                      s.staging, st, none, ih);
-        else launch_decide<BLOCK, ITEMS, MODE_OTHER, false, true, false, false, true>(job, n_cu, per_cu, s.counts,
-                                                                                   s.staging, st, none, ih);
-    } else {
-        if (lds) launch_decide<BLOCK, ITEMS, MODE_OTHER, false, false, true, false, true>(job, n_cu, per_cu, s.counts,
-                                                                                       s.staging, st, none, ih);
-        else launch_decide<BLOCK, ITEMS, MODE_OTHER, false, false, false, false, true>(job, n_cu, per_cu, s.counts,
-                                                                                    s.staging, st, none, ih);
-    }
+    if (lds) launch_decide<BLOCK, ITEMS, MODE_OTHER, false, true, false, true>(job, n_cu, per_cu, s.counts, s.staging,
+                                                                               st, none, ih);
+    else launch_decide<BLOCK, ITEMS, MODE_OTHER, false, false, false, true>(job, n_cu, per_cu, s.counts, s.staging, st,
+                                                                            none, ih);
     return hipGetLastError();
 }
 
@@ -973,16 +943,9 @@ template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool CACHE = false>
 void launch_mode(const CullJob& job, uint32_t n_cu, uint32_t per_cu, uint32_t* counts, uint2* staging, hipStream_t st,
                  const FrameCacheDev& fc = FrameCacheDev{})
 {
-    // identity scenes have no transform-index stream (obj_xf == nullptr): XF_ID must follow it in every variant
     const bool lds = job.scene.n_surfaces <= kLdsSurfaces && job.scene.n_lods <= kLdsLods;
-    const bool xf_id = job.scene.obj_xf == nullptr;
-    if (xf_id) {
-        if (lds) launch_decide<BLOCK, ITEMS, MODE, HIZ, true, true, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
-        else launch_decide<BLOCK, ITEMS, MODE, HIZ, true, false, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
-    } else {
-        if (lds) launch_decide<BLOCK, ITEMS, MODE, HIZ, false, true, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
-        else launch_decide<BLOCK, ITEMS, MODE, HIZ, false, false, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
-    }
+    if (lds) launch_decide<BLOCK, ITEMS, MODE, HIZ, true, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
+    else launch_decide<BLOCK, ITEMS, MODE, HIZ, false, CACHE>(job, n_cu, per_cu, counts, staging, st, fc);
 }
 
 template <int BLOCK, int ITEMS>
@@ -1209,50 +1172,101 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t 
 
 // Transform updates, in two launches so that an id named more than once in one commit takes its last occurrence
 // (UpdateObjectTransform copies updates into the staging buffer in call order, vulkanDraw.cpp:816-820):
-//   mark:    update i copies its id from the pinned slot into device memory and raises winner[id] to i + 1;
+//   stage:   copies ids and records from the pinned slot into device memory, one coalesced 16-byte word per thread, and
+//            update i raises winner[id] to i + 1;
 //   scatter: update i writes its 32-byte record into the position/scale and quaternion streams only if it is the
 //            winner, which then clears winner[id] (the array is all zero between commits; a non-winner compares its
 //            own i + 1 and never matches, whether it reads before or after that clear).
 // Ids >= n_xf are skipped and set err[2].
-__global__ void mark_staged_transforms_kernel(const uint32_t* __restrict__ ids, uint32_t n, uint32_t n_xf,
-                                              uint32_t* dev_ids, uint32_t* winner, uint32_t* err)
+// The host link bounds the first launch, and everything that has to cross it does so there, in one round trip: reading
+// the records in the scatter, 32 bytes apart per lane and after its ids and winners had come back, cost a second one
+// (10 485 updates: 11.2 + 5.2 us with the objects' world-space spheres written too, against 4.1 + 9.6 us without them).
+__global__ __launch_bounds__(256) void stage_transforms_kernel(const uint32_t* __restrict__ ids,
+                                                               const float4* __restrict__ records, uint32_t n,
+                                                               uint32_t n_xf, float4* __restrict__ dev_records,
+                                                               uint32_t* __restrict__ dev_ids, uint32_t* winner,
+                                                               uint32_t* err)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = ids[i];
-    dev_ids[i] = id;
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;  // grid: 2n threads (n < 2^31 transforms fit the host's memory)
+    const bool own = j < n;
+    const uint32_t id = own ? ids[j] : 0u;
+    if (j < 2ull * n) dev_records[j] = records[j];
+    if (!own) return;
+    dev_ids[j] = id;
     if (id >= n_xf) {
         atomicOr(&err[2], 1u);
         return;
     }
-    atomicMax(&winner[id], i + 1u);
+    atomicMax(&winner[id], j + 1u);
 }
 
-__global__ void scatter_staged_transforms_kernel(const uint32_t* __restrict__ dev_ids,
-                                                 const float4* __restrict__ records, uint32_t n, uint32_t n_xf,
-                                                 uint32_t* winner, float4* xf_ps, float4* xf_q)
+// World-space bounding sphere of an object, and its transform's scale.
+__device__ __forceinline__ float4 world_sphere(const float4& sph, const float4& ps, const float4& q)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    float4 w;
+    sphere_to_world(sph.x, sph.y, sph.z, ps.x, ps.y, ps.z, ps.w, q.x, q.y, q.z, q.w, w.x, w.y, w.z);
+    w.w = ps.w;
+    return w;
+}
+
+__device__ __forceinline__ float4 object_surface(const SceneDev& S, uint32_t obj)
+{
+    return S.surf_sphere[S.obj_surf16 ? (uint32_t)S.obj_surf16[obj] : S.obj_surf[obj]];
+}
+
+__global__ __launch_bounds__(256) void scatter_staged_transforms_kernel(const uint32_t* __restrict__ dev_ids,
+                                                                        const float4* __restrict__ records, uint32_t n,
+                                                                        XfTarget to)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
     const uint32_t id = dev_ids[i];
-    if (id >= n_xf || winner[id] != i + 1u) return;
     const float4 ps = records[2u * i], q = records[2u * i + 1u];
-    xf_ps[id] = ps;
-    xf_q[id] = q;
-    winner[id] = 0u;
+    if (id >= to.scene.n_transforms || to.winner[id] != i + 1u) return;
+    to.xf_ps[id] = ps;
+    to.xf_q[id] = q;
+    to.winner[id] = 0u;
+    if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
+    else if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), ps, q);
 }
 
-hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n, uint32_t n_xf,
-                                            uint32_t* dev_ids, uint32_t* winner, float4* xf_ps, float4* xf_q,
-                                            uint32_t* err, hipStream_t st)
+// World-space spheres of the scene's objects: all of them (stamp == nullptr), or those whose transform carries the
+// stamp of the update just scattered. One thread per object, so that the cost does not depend on how many objects
+// share one transform (a list of objects per transform would be walked serially by the transform's thread).
+__global__ __launch_bounds__(256) void world_spheres_kernel(SceneDev S, float4* __restrict__ world,
+                                                            const uint32_t* __restrict__ stamp, uint32_t version)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= S.n_objects) return;
+    const uint32_t x = S.obj_xf ? S.obj_xf[i] : i;
+    if (stamp && stamp[x] != version) return;
+    world[i] = world_sphere(object_surface(S, i), S.xf_ps[x], S.xf_q[x]);
+}
+
+hipError_t launch_world_spheres(const SceneDev& scene, float4* world, hipStream_t st)
+{
+    if (scene.n_objects == 0) return hipSuccess;
+    hipLaunchKernelGGL(world_spheres_kernel, dim3((scene.n_objects + 255u) / 256u), dim3(256), 0, st, scene, world,
+                       (const uint32_t*)nullptr, 0u);
+    return hipGetLastError();
+}
+
+hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n,
+                                            const XfTarget& to, float4* dev_records, uint32_t* dev_ids, uint32_t* err,
+                                            hipStream_t st)
 {
     if (n == 0) return hipSuccess;
-    const dim3 g((n + 255) / 256), b(256);
-    hipLaunchKernelGGL(mark_staged_transforms_kernel, g, b, 0, st, ids, n, n_xf, dev_ids, winner, err);
+    const dim3 g((n + 255u) / 256u), b(256);
+    hipLaunchKernelGGL(stage_transforms_kernel, dim3((uint32_t)((2ull * n + 255u) / 256u)), b, 0, st, ids, records, n,
+                       to.scene.n_transforms, dev_records, dev_ids, to.winner, err);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(scatter_staged_transforms_kernel, g, b, 0, st, (const uint32_t*)dev_ids, records, n, n_xf,
-                       winner, xf_ps, xf_q);
+    hipLaunchKernelGGL(scatter_staged_transforms_kernel, g, b, 0, st, (const uint32_t*)dev_ids,
+                       (const float4*)dev_records, n, to);
+    e = hipGetLastError();
+    if (e != hipSuccess || !to.scene.obj_xf || to.scene.n_objects == 0) return e;
+    hipLaunchKernelGGL(world_spheres_kernel, dim3((to.scene.n_objects + 255u) / 256u), b, 0, st, to.scene, to.world,
+                       (const uint32_t*)to.stamp, to.version);
     return hipGetLastError();
 }
 

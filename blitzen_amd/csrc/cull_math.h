@@ -3,13 +3,13 @@
 // fp32 only, compiled with -ffp-contract=off (no contraction by the compiler), IEEE denormals, correctly rounded
 // sqrt and division, so every result is bit-identical to a CPU build of the same expressions. A product is fused
 // into the add or subtract that follows it (one rounding: v_fma_f32) exactly where an expression is written with
-// fma_f: in rotate_quat, sphere_to_view, frustum_visible and project_sphere. GLSL lets a compiler
+// fma_f: in rotate_quat, sphere_to_world, frustum_visible and project_sphere. GLSL lets a compiler
 // contract a*b+c in the reference's shaders (they declare nothing `precise`), so both forms are the reference's
 // arithmetic; this one is fixed here and in the oracle, point for point, and takes about 14 fewer VALU instructions per
 // object in the transform and frustum test.
 // Sources of the arithmetic (GLSL, Blitzen):
 //   rotate_quat        src/Renderer/VulkanShaderHeaders/ShaderBuffers.glsl:197-200
-//   sphere_to_view     src/Renderer/VulkanShaderHeaders/CullingShaderData.glsl:44-46
+//   sphere_to_world, world_to_view, sphere_to_view  src/Renderer/VulkanShaderHeaders/CullingShaderData.glsl:44-46
 //   frustum_visible    CullingShaderData.glsl:52-55
 //   project_sphere     CullingShaderData.glsl:8-33
 //   occlusion_visible  CullingShaderData.glsl:60-73 (+ sampler rules below)
@@ -62,20 +62,34 @@ BZ_HD void rotate_quat(float vx, float vy, float vz, float qx, float qy, float q
     oz = vz + 2.0f * fma_f(qx, ty, -(qy * tx));
 }
 
+// Bounding sphere centre (surface) -> world space, through the object transform. It does not depend on the view, so the
+// scene keeps the result per object (SceneDev::world).
+BZ_HD void sphere_to_world(float cx, float cy, float cz, float px, float py, float pz, float scale, float qx, float qy,
+                           float qz, float qw, float& wx, float& wy, float& wz)
+{
+    float rx, ry, rz;
+    rotate_quat(cx, cy, cz, qx, qy, qz, qw, rx, ry, rz);
+    wx = fma_f(rx, scale, px);
+    wy = fma_f(ry, scale, py);
+    wz = fma_f(rz, scale, pz);
+}
+
+BZ_HD void world_to_view(const ViewConsts& v, float wx, float wy, float wz, float& ox, float& oy, float& oz)
+{
+    // column-major view * vec4(w, 1): ((m0*x + m4*y) + m8*z) + m12, unfused (the reference's mat * vec order)
+    ox = ((v.m[0] * wx + v.m[1] * wy) + v.m[2] * wz) + v.m[3];
+    oy = ((v.m[4] * wx + v.m[5] * wy) + v.m[6] * wz) + v.m[7];
+    oz = ((v.m[8] * wx + v.m[9] * wy) + v.m[10] * wz) + v.m[11];
+}
+
 // Bounding sphere (surface centre/radius) -> view space, through the object transform.
 BZ_HD void sphere_to_view(const ViewConsts& v, float cx, float cy, float cz, float r, float px, float py, float pz,
                           float scale, float qx, float qy, float qz, float qw, float& ox, float& oy, float& oz,
                           float& orad)
 {
-    float rx, ry, rz;
-    rotate_quat(cx, cy, cz, qx, qy, qz, qw, rx, ry, rz);
-    const float wx = fma_f(rx, scale, px);
-    const float wy = fma_f(ry, scale, py);
-    const float wz = fma_f(rz, scale, pz);
-    // column-major view * vec4(w, 1): ((m0*x + m4*y) + m8*z) + m12, unfused (the reference's mat * vec order)
-    ox = ((v.m[0] * wx + v.m[1] * wy) + v.m[2] * wz) + v.m[3];
-    oy = ((v.m[4] * wx + v.m[5] * wy) + v.m[6] * wz) + v.m[7];
-    oz = ((v.m[8] * wx + v.m[9] * wy) + v.m[10] * wz) + v.m[11];
+    float wx, wy, wz;
+    sphere_to_world(cx, cy, cz, px, py, pz, scale, qx, qy, qz, qw, wx, wy, wz);
+    world_to_view(v, wx, wy, wz, ox, oy, oz);
     orad = r * scale;
 }
 
