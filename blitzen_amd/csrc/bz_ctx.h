@@ -156,6 +156,8 @@ struct Ctx {
     std::unordered_map<uint64_t, std::unique_ptr<ExtSem>> extsems;
     std::unordered_map<uintptr_t, std::unique_ptr<StreamScratch>> scratch;
     bz_tuning tune[2] = {};
+    // The tuning of one single-view pass over n objects: tune[0], or where that is the built-in one, the choice by n.
+    bz_tuning pass_tuning(uint32_t n) const;
     std::unique_ptr<Server> server;
     void* noalloc_scratch = nullptr;  // device address of this device's fixed scratch (bz_cull_noalloc)
 

@@ -253,6 +253,21 @@ uint32_t tiles_for(uint32_t n, uint32_t block, uint32_t items)
     return t ? (uint32_t)t : 1u;
 }
 
+constexpr bz_tuning kBuiltInTuning{ 512, 2, 0, 0 };
+
+// Up to 2^19 objects a pass is a few rounds of dependent latencies: tiles of 512 objects give every CU two workgroups or
+// more (65 536 objects, EARLY + pyramid + LATE: 27.8 us against 29.4 us with 1024-object tiles of 512 threads; 262 161:
+// 28.2 against 28.8; 500 009 TEMPORAL: 34.3 against 34.3-38). Above it the streams bound it and four objects a thread
+// are better: a wave's compacted LOD selection then runs on twice the lanes (1 048 576: 40.1 against 41.9 us; 4 194 304
+// with the frame cache: 59.2 against 62.1; PLAIN of 16 777 216: 83.1 against 84.3).
+bz_tuning Ctx::pass_tuning(uint32_t n) const
+{
+    const bz_tuning& t = tune[0];
+    const bz_tuning& d = kBuiltInTuning;
+    if (t.block != d.block || t.items != d.items || t.grid_per_cu != d.grid_per_cu) return t;
+    return n <= (1u << 19) ? bz_tuning{ 256, 2, 0, 0 } : bz_tuning{ 256, 4, 0, 0 };
+}
+
 // Validates one view's cull and fills a CullJob (without tile_start).
 bz_status Ctx::make_job(uint32_t pass, uint32_t flags, bz_scene sh, bz_pyramid ph, const bz_CameraViewData& view,
                         uint32_t begin, uint32_t count, const uint32_t* vis_in, uint32_t* vis_out, void* cmds,
@@ -348,7 +363,7 @@ bz_status bz_create(const bz_config* cfg, bz_ctx** out)
     c->n_cu = (uint32_t)prop.multiProcessorCount;
     c->hbm_bytes = (uint64_t)prop.totalGlobalMem;
     std::snprintf(c->device_name, sizeof c->device_name, "%s", prop.gcnArchName);
-    c->tune[0] = bz_tuning{ 512, 2, 0, 0 };
+    c->tune[0] = kBuiltInTuning;
     c->tune[1] = bz_tuning{ 256, 4, 8, 0 };
     *out = c.release();
     return BZ_OK;
@@ -891,7 +906,10 @@ namespace bz {
 // range that needs more, or a frame cache not yet allocated large enough, is refused.
 bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch* fixed)
 {
-    const bz_tuning& t = tune[0];
+    Scene* scn = scene(a->scene);
+    if (!scn) return fail(BZ_E_INVALID, "unknown scene handle");
+    const bool all = a->object_begin == 0 && a->object_count == 0;
+    const bz_tuning t = pass_tuning(all ? scn->n_objects : a->object_count);
     CullJob job;
     bz_status s = make_job(a->pass, a->flags, a->scene, a->pyramid, *a->view, a->object_begin, a->object_count,
                            a->visibility_in_dev, a->visibility_out_dev, a->cmds_dev, a->count_dev, a->capacity, t.block,
@@ -915,7 +933,6 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
         if (r == BZ_OK) *out = sc->cs;
         return r;
     };
-    Scene* scn = scene(a->scene);
     const bool cache = (a->flags & BZ_CULL_FRAME_CACHE) != 0;
     float key[19];
     std::memcpy(key, job.view.m, sizeof job.view.m);

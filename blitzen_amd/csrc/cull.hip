@@ -37,18 +37,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, uint32_t lane)
 constexpr uint32_t kLdsSurfaces = 512;
 constexpr uint32_t kLdsLods = 2048;
 
-template <int BLOCK, int ITEMS>
+template <int BLOCK, int ITEMS, bool LDS_TAB>
 struct TileSmem {
-    float surf_rad[kLdsSurfaces];
-    uint2 surf_lod[kLdsSurfaces];
-    float lod_err[kLdsLods];
+    float surf_rad[LDS_TAB ? kLdsSurfaces : 1];
+    uint2 surf_lod[LDS_TAB ? kLdsSurfaces : 1];
+    float lod_err[LDS_TAB ? kLdsLods : 1];
     float4 cand[BLOCK];               // per-wave compaction area: one chunk of 64 entries per wave
     uint2 cand2[BLOCK];
     uint32_t lvl[kMaxMips];
-    uint32_t woff[ITEMS][BLOCK / 64];
+    uint32_t wtot[2][BLOCK / 64];     // per-wave totals of the emitting objects, by the tile's parity
+    uint32_t ctot[2][BLOCK / 64];     // frame cache: per-wave totals of the survivors
     uint32_t csum[BLOCK / 64];        // cluster mode: per-wave sums of the emitting objects' cluster counts
-    uint32_t cwoff[ITEMS][BLOCK / 64];  // frame cache: survivor offsets in (item, wave) order
-    uint32_t job;
 };
 
 // Pass families compiled separately so the visibility stream is loaded unconditionally where it is used.
@@ -81,13 +80,26 @@ __device__ __forceinline__ uint32_t wave_compact(const bool (&pred)[ITEMS], uint
 }
 
 // Object streams of one tile held in registers. Indices are clamped into the job so every load is issued without
-// waiting on another; out-of-range lanes are discarded afterwards.
+// waiting on another; out-of-range lanes are discarded afterwards. Item k of a thread is object tile_object + 64 k of the
+// job: a wave's objects are consecutive, so that their order within the tile is (wave, item, lane) and a wave ranks its
+// own without its neighbours. The indices are recomputed from the tile's number where they are needed, not kept: two
+// tiles' streams are live at once, and 64 registers a thread is what a fourth workgroup per CU fits in.
 template <int ITEMS>
 struct Streams {
-    uint32_t gi[ITEMS], vis[ITEMS], surf[ITEMS];
-    bool valid[ITEMS], active[ITEMS];
+    uint32_t vis[ITEMS], surf[ITEMS];
     float4 w[ITEMS];  // world-space centre, scale
 };
+
+template <int BLOCK, int ITEMS>
+__device__ __forceinline__ uint32_t tile_object(uint32_t tile_in_job)
+{
+    return tile_in_job * (uint32_t)(BLOCK * ITEMS) + (threadIdx.x >> 6) * (64u * ITEMS) + (threadIdx.x & 63u);
+}
+// Item k's object, clamped into the job (jobs always hold at least one object).
+__device__ __forceinline__ uint32_t clamped_object(const CullJob& J, uint32_t i)
+{
+    return J.begin + (i < J.n ? i : J.n - 1u);
+}
 
 // Loads of the per-object streams. NT: marked non-temporal (streaming, evicted first), for the passes that read each
 // stream once and gather no Hi-Z texels: an EARLY pass recording a frame cache (its LATE pass reads the records, not
@@ -112,45 +124,35 @@ __device__ __forceinline__ T stream_load(const T* p)
     else return *p;
 }
 
-// Tile indices and the visibility stream (EARLY, LATE). Jobs always hold at least one object (empty ranges are
-// answered on the host), so clamped indices are always valid.
+// The visibility stream (EARLY, LATE).
 template <int BLOCK, int ITEMS, int MODE, bool NT = false>
 __device__ __forceinline__ void issue_vis(const CullJob& J, uint32_t tile_in_job, Streams<ITEMS>& s)
 {
-    const uint32_t base = tile_in_job * (uint32_t)(BLOCK * ITEMS);
-    const uint32_t nmax = J.n ? J.n - 1u : 0u;
+    const uint32_t i0 = tile_object<BLOCK, ITEMS>(tile_in_job);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-        const uint32_t i = base + (uint32_t)k * BLOCK + threadIdx.x;
-        s.valid[k] = i < J.n;
-        s.gi[k] = J.begin + (s.valid[k] ? i : nmax);
         s.vis[k] = 0u;
-    }
-    if (MODE == MODE_EARLY || MODE == MODE_LATE) {  // J.n >= 1: clamped indices are in range
-#pragma unroll
-        for (int k = 0; k < ITEMS; ++k) s.vis[k] = stream_load<NT>(J.vis_in + s.gi[k]);
+        if (MODE == MODE_EARLY || MODE == MODE_LATE)
+            s.vis[k] = stream_load<NT>(J.vis_in + clamped_object(J, i0 + 64u * k));
     }
 }
 
-// The surface-id and world-space sphere streams: for every object, or in EARLY only for last-frame-visible ones (which waits
-// for the visibility stream first).
+// The surface-id and world-space sphere streams: for every object, or in EARLY only for last-frame-visible ones (which
+// waits for the visibility stream first).
 // ALL (EARLY recording a frame cache): every object's streams are loaded, not only the last-frame-visible ones.
-template <int ITEMS, int MODE, bool ALL = false, bool NT = false>
-__device__ __forceinline__ void issue_objects(const CullJob& J, Streams<ITEMS>& s)
+template <int BLOCK, int ITEMS, int MODE, bool ALL = false, bool NT = false>
+__device__ __forceinline__ void issue_objects(const CullJob& J, uint32_t tile_in_job, Streams<ITEMS>& s)
 {
     const SceneDev& S = J.scene;
+    const uint32_t i0 = tile_object<BLOCK, ITEMS>(tile_in_job);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-        s.active[k] = s.valid[k] && (MODE != MODE_EARLY || s.vis[k] != 0u);
+        const uint32_t g = clamped_object(J, i0 + 64u * k);
         s.surf[k] = 0u;
         s.w[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        if (MODE != MODE_EARLY || ALL || s.active[k]) {
-            s.surf[k] = S.obj_surf16 ? (uint32_t)stream_load<NT>(S.obj_surf16 + s.gi[k])
-                                     : stream_load<NT>(S.obj_surf + s.gi[k]);
-            s.w[k] = stream_load<NT>(S.world + s.gi[k]);
+        if (MODE != MODE_EARLY || ALL || (i0 + 64u * k < J.n && s.vis[k] != 0u)) {
+            s.surf[k] = S.obj_surf16 ? (uint32_t)stream_load<NT>(S.obj_surf16 + g) : stream_load<NT>(S.obj_surf + g);
+            s.w[k] = stream_load<NT>(S.world + g);
         }
     }
 }
@@ -159,17 +161,17 @@ template <int BLOCK, int ITEMS, int MODE, bool ALL = false, bool NT = false>
 __device__ __forceinline__ void issue_tile(const CullJob& J, uint32_t tile_in_job, Streams<ITEMS>& s)
 {
     issue_vis<BLOCK, ITEMS, MODE, NT>(J, tile_in_job, s);
-    issue_objects<ITEMS, MODE, ALL, NT>(J, s);
+    issue_objects<BLOCK, ITEMS, MODE, ALL, NT>(J, tile_in_job, s);
 }
 
 // Small tables into LDS (surface radii and LOD ranges, LOD errors) plus the pyramid's level offsets. All loads of a
 // thread are issued before its first LDS write. The caller places the barrier.
-template <int BLOCK, int ITEMS>
-__device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, ITEMS>& sm, bool lds_tab)
+template <int BLOCK, int ITEMS, bool LDS_TAB>
+__device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, ITEMS, LDS_TAB>& sm)
 {
     const uint32_t tid = threadIdx.x;
     const SceneDev& S = J.scene;
-    if (lds_tab) {
+    if constexpr (LDS_TAB) {
         constexpr int SPT = (kLdsSurfaces + BLOCK - 1) / BLOCK, LPT = (kLdsLods + BLOCK - 1) / BLOCK;
         float t_rad[SPT];
         uint2 t_lod[SPT];
@@ -219,17 +221,18 @@ struct NoPrefetch {
 // INST (LOD-instanced output): each emitting object also adds 1 to its LOD's bin of the workgroup's LDS histogram.
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false, bool CACHE = false, bool INST = false,
           class Prefetch>
-__device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, const Streams<ITEMS>& s,
-                                             uint32_t* counts, uint2* staging, uint32_t* ccounts,
-                                             TileSmem<BLOCK, ITEMS>& sm, Prefetch&& prefetch,
+__device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t parity,
+                                             const Streams<ITEMS>& s, uint32_t* counts, uint2* staging, uint32_t* ccounts,
+                                             TileSmem<BLOCK, ITEMS, LDS_TAB>& sm, Prefetch&& prefetch,
                                              FrameCacheDev fc = FrameCacheDev{}, uint32_t* lds_hist = nullptr)
 {
     constexpr bool lds_tab = LDS_TAB;
     constexpr int NW = BLOCK / 64;
     constexpr uint32_t TILE = BLOCK * ITEMS;
     constexpr bool late = MODE == MODE_LATE;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t pass = J.pass;
+    const uint32_t i0 = tile_object<BLOCK, ITEMS>(tile_in_job);  // item k: object i0 + 64 k of the job
     const SceneDev& S = J.scene;
 
     float cx[ITEMS], cy[ITEMS], cz[ITEMS], rad[ITEMS];
@@ -247,12 +250,8 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
     for (int k = 0; k < ITEMS; ++k) {
         world_to_view(J.view, s.w[k].x, s.w[k].y, s.w[k].z, cx[k], cy[k], cz[k]);
         rad[k] = rad[k] * s.w[k].w;
-        if constexpr (CACHE) {
-            frus[k] = s.valid[k] && frustum_visible(J.view, cx[k], cy[k], cz[k], rad[k]);
-            vis_new[k] = frus[k] && s.active[k];
-        } else {
-            vis_new[k] = s.active[k] && frustum_visible(J.view, cx[k], cy[k], cz[k], rad[k]);
-        }
+        frus[k] = i0 + 64u * k < J.n && frustum_visible(J.view, cx[k], cy[k], cz[k], rad[k]);
+        vis_new[k] = frus[k] && (MODE != MODE_EARLY || s.vis[k] != 0u);
     }
     float4* cand = sm.cand + wave * 64u;
     uint2* cand2 = sm.cand2 + wave * 64u;
@@ -332,13 +331,18 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
             const float len = sqrtf((c.x * c.x + c.y * c.y) + c.z * c.z);
             const float distance = glsl_max(len - c.w, 0.0f);
             const float threshold = (distance * J.view.lodTarget) / scale;
-            uint32_t idx = 0;
-            if (lds_tab) {
-                for (uint32_t l = 1; l < lo.y; ++l)
-                    if (sm.lod_err[lo.x + l] < threshold) idx = l;
-            } else {
-                for (uint32_t l = 1; l < lo.y; ++l)
-                    if (S.lod_error[lo.x + l] < threshold) idx = l;
+            uint32_t idx = 0;  // the last LOD whose error is below the threshold: four errors read at a time
+            for (uint32_t l0 = 1; l0 < lo.y; l0 += 4u) {
+                uint32_t l[4];
+                float err[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) {
+                    l[j] = l0 + j < lo.y ? l0 + j : lo.y - 1u;
+                    err[j] = lds_tab ? sm.lod_err[lo.x + l[j]] : S.lod_error[lo.x + l[j]];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j)
+                    if (err[j] < threshold) idx = l[j];
             }
             cand2[lane].x = (pass == PASS_ONPC) ? idx : idx + lo.x;
         }
@@ -365,81 +369,73 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t gtile, c
         if (lane == 0) sm.csum[wave] = cc;
     }
 
-    // ---- visibility; ranks in (item, wave) order -> staging
+    // ---- visibility; ranks in (wave, item, lane) order -> staging
     if (late) {
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k)
-            if (s.valid[k]) J.vis_out[s.gi[k]] = vis_new[k] ? 1u : 0u;
+            if (i0 + 64u * k < J.n) J.vis_out[J.begin + i0 + 64u * k] = vis_new[k] ? 1u : 0u;
     }
-    uint32_t rank[ITEMS], crank[ITEMS];
+    // A wave's ranks come from its own ballots (without a frame cache those of the LOD compaction); the waves' totals go
+    // through LDS, and each wave adds up the totals before its own. One barrier per tile: the totals alternate between
+    // two sets by the tile's parity, so a wave that is a tile ahead does not overwrite what a slower one still reads.
+    uint32_t erank[ITEMS], etot = ne;
+    if constexpr (CACHE) etot = wave_compact<ITEMS>(emit, erank, lane);
+    if (lane == 0) {
+        sm.wtot[parity][wave] = etot;
+        if constexpr (CACHE) sm.ctot[parity][wave] = ne;
+    }
+    __syncthreads();
+    uint32_t before = 0, total = 0, cbefore = 0, ctotal = 0;
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        const unsigned long long m = __ballot(emit[k]);
-        rank[k] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if (lane == 0) sm.woff[k][wave] = (uint32_t)__popcll(m);
+    for (uint32_t w = 0; w < (uint32_t)NW; ++w) {
+        const uint32_t x = sm.wtot[parity][w];
+        before += w < wave ? x : 0u;
+        total += x;
         if constexpr (CACHE) {
-            const unsigned long long mc = __ballot(frus[k]);
-            crank[k] = (uint32_t)__popcll(mc & ((1ull << lane) - 1ull));
-            if (lane == 0) sm.cwoff[k][wave] = (uint32_t)__popcll(mc);
+            const uint32_t y = sm.ctot[parity][w];
+            cbefore += w < wave ? y : 0u;
+            ctotal += y;
         }
     }
-    __syncthreads();
-    if constexpr (CACHE) {
-        if (wave == (uint32_t)NW - 1u) {  // the cache's survivor offsets, scanned by another wave than the commands'
-            constexpr uint32_t E = ITEMS * NW;
-            const uint32_t c = lane < E ? (&sm.cwoff[0][0])[lane] : 0u;
-            const uint32_t incl = wave_incl_scan(c, lane);
-            if (lane < E) (&sm.cwoff[0][0])[lane] = incl - c;
-            if (lane == 63) fc.counts[gtile] = incl;
-        }
-    }
-    if (wave == 0) {
-        constexpr uint32_t E = ITEMS * NW;  // <= 64
-        const uint32_t c = lane < E ? (&sm.woff[0][0])[lane] : 0u;
-        const uint32_t incl = wave_incl_scan(c, lane);
-        if (lane < E) (&sm.woff[0][0])[lane] = incl - c;
-        if (lane == 63) counts[gtile] = incl;
+    if (tid == 0) {
+        counts[gtile] = total;
+        if constexpr (CACHE) fc.counts[gtile] = ctotal;
         if constexpr (CL) {
-            if (lane == 0) {
-                uint32_t tot = 0;
+            uint32_t tot = 0;
 #pragma unroll
-                for (int w = 0; w < NW; ++w) tot += sm.csum[w];
-                ccounts[gtile] = tot;
-            }
+            for (int w = 0; w < NW; ++w) tot += sm.csum[w];
+            ccounts[gtile] = tot;
         }
     }
-    __syncthreads();
-    uint2* stage = staging + (size_t)gtile * TILE;
+    uint2* stage = staging + (size_t)gtile * TILE + before;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k)
-        if (emit[k]) stage[sm.woff[k][wave] + rank[k]] = make_uint2(s.gi[k], lod_abs[k]);
+        if (emit[k]) stage[CACHE ? erank[k] : eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
     if constexpr (CACHE) {
-        const size_t cb = (size_t)gtile * TILE;
+        const size_t cb = (size_t)gtile * TILE + cbefore;
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k)
             if (frus[k]) {
-                const uint32_t pos = sm.cwoff[k][wave] + crank[k];
-                fc.sph[cb + pos] = make_float4(cx[k], cy[k], cz[k], rad[k]);
-                fc.meta[cb + pos] = make_uint2(s.gi[k], lod_abs[k]);
+                fc.sph[cb + eslot[k]] = make_float4(cx[k], cy[k], cz[k], rad[k]);
+                fc.meta[cb + eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
             }
     }
-    __syncthreads();  // woff / cwoff are rewritten by the next tile
 }
 
 // One tile, loads and decision (non-persistent form, used by the batched kernel and the cluster object pass).
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false>
 __device__ __forceinline__ void decide_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t* counts,
-                                            uint2* staging, TileSmem<BLOCK, ITEMS>& sm, uint32_t* ccounts = nullptr)
+                                            uint2* staging, TileSmem<BLOCK, ITEMS, LDS_TAB>& sm, uint32_t* ccounts = nullptr)
 {
-    constexpr bool lds_tab = LDS_TAB;
     constexpr bool NT = MODE == MODE_OTHER && !HIZ;  // PLAIN / ONPC: streamed once, no Hi-Z
     Streams<ITEMS> s;
     issue_vis<BLOCK, ITEMS, MODE, NT>(J, tile_in_job, s);
-    if (MODE != MODE_EARLY) issue_objects<ITEMS, MODE, false, NT>(J, s);
-    stage_tables<BLOCK, ITEMS>(J, sm, lds_tab);
-    if (MODE == MODE_EARLY) issue_objects<ITEMS, MODE, false, NT>(J, s);
+    if (MODE != MODE_EARLY) issue_objects<BLOCK, ITEMS, MODE, false, NT>(J, tile_in_job, s);
+    stage_tables<BLOCK, ITEMS>(J, sm);
+    if (MODE == MODE_EARLY) issue_objects<BLOCK, ITEMS, MODE, false, NT>(J, tile_in_job, s);
     __syncthreads();  // staged tables visible
-    process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, CL>(J, gtile, s, counts, staging, ccounts, sm, NoPrefetch{});
+    process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, CL>(J, tile_in_job, gtile, 0u, s, counts, staging, ccounts, sm,
+                                                        NoPrefetch{});
 }
 
 // Persistent decide for one view: workgroup b takes tiles b, b + G, b + 2G, ... (no workgroup waits on another, so
@@ -451,9 +447,8 @@ template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CACHE = f
 __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* counts, uint2* staging, FrameCacheDev fc,
                                                        InstHistDev ih)
 {
-    __shared__ TileSmem<BLOCK, ITEMS> sm;
+    __shared__ TileSmem<BLOCK, ITEMS, LDS_TAB> sm;
     __shared__ uint32_t s_hist[INST ? kInstLdsBins : 1];
-    constexpr bool lds_tab = LDS_TAB;
     constexpr bool NT = (MODE == MODE_EARLY && CACHE) || (MODE == MODE_OTHER && !HIZ);
     uint32_t t, t_end, step;
     if constexpr (INST) {
@@ -467,7 +462,7 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
     }
     Streams<ITEMS> A, B;
     issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, t, A);
-    stage_tables<BLOCK, ITEMS>(J, sm, lds_tab);
+    stage_tables<BLOCK, ITEMS>(J, sm);
     __syncthreads();
     while (true) {
         {
@@ -476,8 +471,8 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
             // object, so each stream costs one cache line (discarded). A branch around the loads instead was 2.7 us
             // slower per pass, re-issuing the current tile 2.2 us slower (with non-temporal loads its lines are
             // fetched again).
-            process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, A, counts, staging, nullptr, sm,
-                                                                                [&]() {
+            process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, t, 0u, A, counts, staging, nullptr,
+                                                                                sm, [&]() {
                 issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, B);
             }, fc, s_hist);
             t = tn;
@@ -485,8 +480,8 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
         }
         {
             const uint32_t tn = t + step;
-            process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, B, counts, staging, nullptr, sm,
-                                                                                [&]() {
+            process_tile<BLOCK, ITEMS, MODE, HIZ, LDS_TAB, false, CACHE, INST>(J, t, t, 1u, B, counts, staging, nullptr,
+                                                                                sm, [&]() {
                 issue_tile<BLOCK, ITEMS, MODE, CACHE, NT>(J, tn < t_end ? tn : J.n_tiles, A);
             }, fc, s_hist);
             t = tn;
@@ -527,7 +522,7 @@ __global__ __launch_bounds__(BLOCK) void decide_batch_kernel(const CullJob* __re
                                                              const uint32_t* __restrict__ starts, uint32_t n_jobs,
                                                              uint32_t* counts, uint2* staging, JobStartsArg sa)
 {
-    __shared__ TileSmem<BLOCK, ITEMS> sm;
+    __shared__ TileSmem<BLOCK, ITEMS, false> sm;
     __shared__ uint32_t s_start[kLdsJobs];
     const uint32_t t = blockIdx.x;
     uint32_t jb;
@@ -551,10 +546,10 @@ __global__ __launch_bounds__(BLOCK) void decide_batch_kernel(const CullJob* __re
 // every object, its LOD, and per tile the number of emitting objects (counts), their (objectId, LOD) list (staging)
 // and the sum of their LOD cluster counts (ccounts). One workgroup per tile.
 template <int BLOCK, int ITEMS, bool HIZ, bool LDS_TAB>
-__global__ __launch_bounds__(BLOCK) void decide_cluster_kernel(CullJob J, uint32_t* counts, uint2* staging,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 2 ? 8 : 4))) void decide_cluster_kernel(CullJob J, uint32_t* counts, uint2* staging,
                                                                uint32_t* ccounts)
 {
-    __shared__ TileSmem<BLOCK, ITEMS> sm;
+    __shared__ TileSmem<BLOCK, ITEMS, LDS_TAB> sm;
     decide_tile<BLOCK, ITEMS, MODE_OTHER, HIZ, LDS_TAB, true>(J, blockIdx.x, blockIdx.x, counts, staging, sm, ccounts);
 }
 

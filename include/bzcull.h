@@ -386,7 +386,7 @@ BZ_API bz_status bz_check(bz_ctx* ctx, void* stream);
 #define BZ_DEFAULT_WAIT_LIMIT 1048576u
 BZ_API bz_status bz_set_wait_limit(bz_ctx* ctx, uint32_t sleeps);
 /* Tuning used by bz_cull (kernel 0) and bz_cull_batch (kernel 1); defaults are built in, bz_autotune
- * replaces them. */
+ * replaces them. With the built-in one for kernel 0 (512, 2, 0), bz_cull chooses by the number of objects. */
 BZ_API bz_status bz_get_tuning(bz_ctx* ctx, uint32_t kernel /* 0 = single view, 1 = batched */, bz_tuning* out);
 BZ_API bz_status bz_set_tuning(bz_ctx* ctx, uint32_t kernel, const bz_tuning* t);
 /* Times every candidate tuning (block 256/512 x items 2/4, and for kernel 0 a persistent grid of 0, 1, 2
