@@ -72,7 +72,7 @@ struct PyrPlan {
     uint32_t base_w = 0, base_h = 0, mips = 0;
     uint32_t level_offset[kMaxMips] = {};
     uint64_t n_texels = 0;
-    uint32_t tile_w = 0, tile_h = 0, tiles_x = 0, tiles_y = 0, tile_levels = 0;
+    uint32_t tiles_x = 0, tiles_y = 0, tile_levels = 0;
     bool single_pass = false;
     PyramidDesc desc(const float* texels) const;
     PyrBuildJob build_job(const float* depth, uint32_t w, uint32_t h, float* texels, unsigned long long* tail) const;

@@ -70,13 +70,17 @@ constexpr uint32_t kScanTiles = 4096;
 // Exclusive prefix of counts[0, n) into prefix[0, n], prefix[n] = the total (one workgroup, linear in n).
 hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* prefix, hipStream_t st);
 
+constexpr uint32_t kPyrTile = 32;           // level-0 tile edge of the single-pass build
+constexpr uint32_t kPyrTileLevels = 6;      // its levels: 32 x 32 ... 1 x 1
+constexpr uint32_t kPyrTailTexels = 1024;   // the tile image's first reduction, held by the tail workgroup
+
 struct PyrBuildJob {
     const float* depth;
     uint32_t w, h;
     float* texels;
     uint32_t base_w, base_h, mips;
-    uint32_t tile_w, tile_h, tiles_x, tiles_y;  // single-pass tiling of level 0
-    uint32_t tile_levels;                        // levels reduced inside a tile (>= 1: includes level 0)
+    uint32_t tiles_x, tiles_y;                   // single-pass tiling of level 0 (kPyrTile x kPyrTile texels)
+    uint32_t tile_levels;                        // levels reduced inside a tile (includes level 0)
     uint32_t wg_start;                           // batched: first workgroup of this job
     uint32_t spin_limit;                         // sleeps before a wait for a tail word gives up
     unsigned long long* tail;                    // per job: one flagged word per tile, zero between builds

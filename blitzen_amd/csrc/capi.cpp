@@ -230,19 +230,12 @@ bool plan_pyramid(uint32_t base_w, uint32_t base_h, uint32_t mips, PyrPlan* p)
     if (off > 0xffffffffull) return false;
     p->n_texels = off;
     const bool pow2 = (base_w & (base_w - 1)) == 0 && (base_h & (base_h - 1)) == 0;
-    p->tile_w = std::min<uint32_t>(32u, base_w);
-    p->tile_h = std::min<uint32_t>(32u, base_h);
-    p->tiles_x = base_w / p->tile_w;
-    p->tiles_y = base_h / p->tile_h;
-    uint32_t tl = 1, m = std::max(p->tile_w, p->tile_h);
-    while (m > 1) {
-        m >>= 1;
-        ++tl;
-    }
-    p->tile_levels = std::min(tl, mips);
+    p->tiles_x = std::max(1u, base_w / kPyrTile);
+    p->tiles_y = std::max(1u, base_h / kPyrTile);
+    p->tile_levels = std::min(kPyrTileLevels, mips);
     // single pass: power-of-two extent, and the tile image's first reduction fits the tail workgroup's LDS tile
     const uint64_t tail_texels = (uint64_t)std::max(1u, p->tiles_x / 2u) * std::max(1u, p->tiles_y / 2u);
-    p->single_pass = pow2 && (p->tile_levels >= mips || tail_texels <= 1024u);
+    p->single_pass = pow2 && (p->tile_levels >= mips || tail_texels <= kPyrTailTexels);
     return true;
 }
 
@@ -816,8 +809,6 @@ PyrBuildJob PyrPlan::build_job(const float* depth, uint32_t w, uint32_t h, float
     j.base_w = base_w;
     j.base_h = base_h;
     j.mips = mips;
-    j.tile_w = tile_w;
-    j.tile_h = tile_h;
     j.tiles_x = tiles_x;
     j.tiles_y = tiles_y;
     j.tile_levels = tile_levels;

@@ -80,9 +80,9 @@ __device__ __forceinline__ uint32_t wave_compact(const bool (&pred)[ITEMS], uint
 }
 
 // Object streams of one tile held in registers. Indices are clamped into the job so every load is issued without
-// waiting on another; out-of-range lanes are discarded afterwards. Item k of a thread is object tile_object + 64 k of the
-// job: a wave's objects are consecutive, so that their order within the tile is (wave, item, lane) and a wave ranks its
-// own without its neighbours. The indices are recomputed from the tile's number where they are needed, not kept: two
+// waiting on another; out-of-range lanes are discarded afterwards. Item k of a thread is object tile_object + 64 k of
+// the job: a wave's objects are consecutive, so that their order within the tile is (wave, item, lane) and a wave ranks
+// its own without its neighbours. The indices are recomputed from the tile's number where they are needed, not kept: two
 // tiles' streams are live at once, and 64 registers a thread is what a fourth workgroup per CU fits in.
 template <int ITEMS>
 struct Streams {
@@ -222,7 +222,8 @@ struct NoPrefetch {
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false, bool CACHE = false, bool INST = false,
           class Prefetch>
 __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t parity,
-                                             const Streams<ITEMS>& s, uint32_t* counts, uint2* staging, uint32_t* ccounts,
+                                             const Streams<ITEMS>& s, uint32_t* counts, uint2* staging,
+                                             uint32_t* ccounts,
                                              TileSmem<BLOCK, ITEMS, LDS_TAB>& sm, Prefetch&& prefetch,
                                              FrameCacheDev fc = FrameCacheDev{}, uint32_t* lds_hist = nullptr)
 {
@@ -375,8 +376,8 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
         for (int k = 0; k < ITEMS; ++k)
             if (i0 + 64u * k < J.n) J.vis_out[J.begin + i0 + 64u * k] = vis_new[k] ? 1u : 0u;
     }
-    // A wave's ranks come from its own ballots (without a frame cache those of the LOD compaction); the waves' totals go
-    // through LDS, and each wave adds up the totals before its own. One barrier per tile: the totals alternate between
+    // A wave's ranks come from its own ballots (without a frame cache those of the LOD compaction); the waves' totals
+    // go through LDS, and each wave adds up the totals before its own. One barrier per tile: the totals alternate between
     // two sets by the tile's parity, so a wave that is a tile ahead does not overwrite what a slower one still reads.
     uint32_t erank[ITEMS], etot = ne;
     if constexpr (CACHE) etot = wave_compact<ITEMS>(emit, erank, lane);
@@ -425,7 +426,8 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
 // One tile, loads and decision (non-persistent form, used by the batched kernel and the cluster object pass).
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false>
 __device__ __forceinline__ void decide_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t* counts,
-                                            uint2* staging, TileSmem<BLOCK, ITEMS, LDS_TAB>& sm, uint32_t* ccounts = nullptr)
+                                            uint2* staging, TileSmem<BLOCK, ITEMS, LDS_TAB>& sm,
+                                            uint32_t* ccounts = nullptr)
 {
     constexpr bool NT = MODE == MODE_OTHER && !HIZ;  // PLAIN / ONPC: streamed once, no Hi-Z
     Streams<ITEMS> s;
@@ -544,10 +546,12 @@ __global__ __launch_bounds__(BLOCK) void decide_batch_kernel(const CullJob* __re
 
 // Cluster object pass (PreClusterDrawCull.comp.glsl:13-47): the PLAIN (or, with a pyramid, TEMPORAL) decision of
 // every object, its LOD, and per tile the number of emitting objects (counts), their (objectId, LOD) list (staging)
-// and the sum of their LOD cluster counts (ccounts). One workgroup per tile.
+// and the sum of their LOD cluster counts (ccounts). One workgroup per tile. The register cap keeps two
+// items per thread at four 512-thread workgroups a CU (68 registers without it: 1 M objects took a second round, 11.8
+// against 10.1 us).
 template <int BLOCK, int ITEMS, bool HIZ, bool LDS_TAB>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 2 ? 8 : 4))) void decide_cluster_kernel(CullJob J, uint32_t* counts, uint2* staging,
-                                                               uint32_t* ccounts)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 2 ? 8 : 4)))
+void decide_cluster_kernel(CullJob J, uint32_t* counts, uint2* staging, uint32_t* ccounts)
 {
     __shared__ TileSmem<BLOCK, ITEMS, LDS_TAB> sm;
     decide_tile<BLOCK, ITEMS, MODE_OTHER, HIZ, LDS_TAB, true>(J, blockIdx.x, blockIdx.x, counts, staging, sm, ccounts);

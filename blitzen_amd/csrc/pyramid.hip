@@ -4,8 +4,8 @@
 // (vulkanDraw.cpp:554-622). Each level texel is the MIN over the non-zero-weight texels of the bilinear
 // footprint of its centre in the level above (level 0 samples the depth buffer), the rule in cull_math.h.
 //
-// Single pass for power-of-two bases: each workgroup owns a tile of level 0 (up to 32 x 32 texels), writes it,
-// and reduces it in LDS down to 1 x 1 (levels 1..5, exact 2:1 with edge clamp). The last workgroup
+// Single pass for power-of-two bases: each workgroup owns a tile of level 0 (32 x 32 texels), writes it,
+// and reduces it in registers down to 1 x 1 (levels 1..5, exact 2:1 with edge clamp). The last workgroup
 // (the highest-numbered one, waiting on flagged words) reduces the remaining levels from the
 // 1-texel-per-tile image. Non-power-of-two
 // bases fall back to one launch per level with the general footprint rule.
@@ -16,33 +16,43 @@ namespace bz {
 
 namespace {
 
-constexpr uint32_t kPyrBlock = 256;
-constexpr uint32_t kTile = 32;
+constexpr uint32_t kPyrBlock = 512;
+constexpr uint32_t kTile = kPyrTile;  // level-0 tile edge of a workgroup: eight waves of 32 x 4 texels
 constexpr unsigned long long kTailFlag = 1ull << 63;
 constexpr uint32_t kLdsJobs = 1024;  // batched: job start table staged in LDS up to this many jobs
 
-__device__ __forceinline__ float min4(float a, float b, float c, float d) { return glsl_min(glsl_min(a, b), glsl_min(c, d)); }
-
-// Reduce src (sw x sh, LDS) to dst (dw x dh = max(1, s/2)) exactly 2:1 with clamp, and write it to global.
-// All extents are powers of two (single-pass pyramids only).
-template <uint32_t NT>
-__device__ __forceinline__ void reduce_lds(const float* src, uint32_t sw, uint32_t sh, float* dst, uint32_t dw,
-                                           uint32_t dh, float* gdst, uint32_t gpitch, uint32_t gx, uint32_t gy)
+__device__ __forceinline__ float min4(float a, float b, float c, float d)
 {
-    const uint32_t dshift = (uint32_t)__builtin_ctz(dw);
-    for (uint32_t t = threadIdx.x; t < dw * dh; t += NT) {
-        const uint32_t lx = t & (dw - 1u), ly = t >> dshift;
-        const uint32_t x0 = 2u * lx, y0 = 2u * ly;
-        const uint32_t x1 = sw > 1u ? x0 + 1u : x0;
-        const uint32_t y1 = sh > 1u ? y0 + 1u : y0;
-        const float d = min4(src[y0 * sw + x0], src[y0 * sw + x1], src[y1 * sw + x0], src[y1 * sw + x1]);
-        dst[t] = d;
-        gdst[(size_t)(gy + ly) * gpitch + gx + lx] = d;
-    }
+    return glsl_min(glsl_min(a, b), glsl_min(c, d));
 }
 
-// Waits for one flagged per-tile word of the tail, already loaded once into w (the wait is bounded; giving up sets
-// *err), and clears it after reading, so the next build starts from zero.
+typedef float float4_unaligned __attribute__((ext_vector_type(4), aligned(4)));  // one 16-byte load at any dword
+
+// A quad_perm of the four lanes of each quad.
+template <int A, int B, int C, int D>
+__device__ __forceinline__ float quad_perm(float v)
+{
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), A | B << 2 | C << 4 | D << 6, 0xf, 0xf, true));
+}
+// min of the value in the lane whose bit `off` is clear and the one whose bit is set, in that order, for both lanes.
+__device__ __forceinline__ float min_across(float v, uint32_t lane, uint32_t off)
+{
+    const float o = __shfl_xor(v, (int)off, 64);
+    return (lane & off) ? glsl_min(o, v) : glsl_min(v, o);
+}
+
+// Orders a wave's LDS writes before its later LDS reads.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_wave_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// One flagged word of the tail: waits until it is there (bounded; giving up sets *err) and clears it, so the next build
+// starts from zero.
 __device__ __forceinline__ float tail_finish(const PyrBuildJob& J, uint32_t idx, unsigned long long w, uint32_t* err)
 {
     uint32_t spins = 0;
@@ -58,193 +68,165 @@ __device__ __forceinline__ float tail_finish(const PyrBuildJob& J, uint32_t idx,
     return __uint_as_float((uint32_t)w);
 }
 
-// Reads one per-tile word for the tail: the owner's own value, or the flagged word another workgroup stored
-// (cleared after reading, so the next build starts from zero). The wait is bounded; giving up sets *err.
-__device__ __forceinline__ float tail_word(const PyrBuildJob& J, uint32_t idx, uint32_t own_tile, float own,
-                                           uint32_t* err)
-{
-    if (idx == own_tile) return own;
-    unsigned long long w = __hip_atomic_load(&J.tail[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t spins = 0;
-    while (!(w & kTailFlag)) {
-        if (++spins > J.spin_limit) {
-            atomicExch(err, 1u);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-        w = __hip_atomic_load(&J.tail[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __hip_atomic_store(&J.tail[idx], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __uint_as_float((uint32_t)w);
-}
+struct PyrSmem {
+    float l2[64];                                              // level 2 of the tile: a row of 8 per wave
+    float a[kPyrTailTexels * 4u], b[kPyrTailTexels];          // the tile image, then the tail's levels in turn
+};
 
-constexpr uint32_t kTileTexels = kTile * kTile;
-constexpr uint32_t kPyrBlockWide = 512;  // single-view builds whose level 0 uses the general footprint rule
-
-// One workgroup's tile of a single-pass (power-of-two) pyramid. bufA holds kTileTexels floats, bufB half that.
-// NT threads per workgroup: 256 for exact 2:1 level 0 (and batches), 512 for the general footprint rule of a single
-// build (more gathers in flight per tile: measured 5% faster there, slower for 2:1).
-template <uint32_t NT>
-__device__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile, float* bufA, float* bufB, uint32_t* err)
+// One workgroup's tile of a single-pass (power-of-two) pyramid, levels 0 to 5: a lane owns two level-0 texels side by side
+// and a wave 32 x 4 (16 lanes across, so every store of level 0 covers whole 128-byte lines), so that levels 1 and 2 come
+// from exchanges between its lanes; levels 3 to 5 from exchanges within the first wave, which reads the eight waves'
+// rows from LDS behind the only barrier. Texels outside the base are +infinity, which no minimum takes over a texel, so
+// every power-of-two extent down to 1 x 1 goes the same way.
+// What bounded a build before was the levels as much as the depth image: a barrier and an LDS round trip per level held
+// each workgroup's slots for half as long again as its loads (2560 x 1440 depth onto 2048 x 1024: level 0 alone 7.2 us,
+// with its levels 10.8, the whole build 14.5; now 12.4. 1920 x 1080 onto 1024 x 1024: 8.9 -> 8.2; 64 pyramids of the batch
+// with exact 2:1: 85 -> 78 us). Lanes in Morton order, which need no LDS up to level 4, store level 0 in 64-byte pieces:
+// level 0 alone 10.5 us. Four texels a lane and 256 threads: 11.5, but 8.2 instead of 6.6 us for 1024 x 512.
+__device__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile, PyrSmem& sm, uint32_t* err)
 {
-    constexpr uint32_t kPerThread = kTileTexels / NT;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t tx = tile % J.tiles_x, ty = tile / J.tiles_x;
-    const uint32_t tw = J.tile_w, th = J.tile_h, n0 = tw * th;
-    const uint32_t tshift = (uint32_t)__builtin_ctz(tw);
-    float* lvl0 = J.texels + J.level_offset[0];
-    // ---- level 0 from the depth buffer; every load of a thread is issued before the first min
-    if (J.w == 2u * J.base_w && J.h == 2u * J.base_h && ((uintptr_t)J.depth & 7u) == 0) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t tx = tile % J.tiles_x, ty = tile / J.tiles_x, bw = J.base_w, bh = J.base_h;
+    const uint32_t x1 = tx * (kTile / 2u) + (lane & 15u);                // the lane's level-1 column
+    const uint32_t x0 = 2u * x1, y0 = ty * kTile + wave * 4u + (lane >> 4);  // and its first level-0 texel
+    const float inf = __builtin_inff();
+    float ta = inf, tb = inf;  // level-0 texels
+    // ---- level 0 from the depth image; every load of a lane is issued before the first minimum
+    if (J.w == 2u * bw && J.h == 2u * bh && bw >= 2u && ((uintptr_t)J.depth & 15u) == 0) {
         // exactly 2:1: the footprint of texel (x, y) is depth {2x, 2x+1} x {2y, 2y+1} (frac(tx) = 0.5 on both axes)
-        float2 r0[kPerThread], r1[kPerThread];
-#pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k) {
-            const uint32_t t0 = tid + k * NT, t = t0 < n0 ? t0 : 0u;
-            const uint32_t x = tx * tw + (t & (tw - 1u)), y = ty * th + (t >> tshift);
-            const float2* row = reinterpret_cast<const float2*>(J.depth + (size_t)(2u * y) * J.w) + x;
-            r0[k] = row[0];
-            r1[k] = row[J.w / 2u];
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k) {
-            const uint32_t t = tid + k * NT;
-            if (t < n0) {
-                const uint32_t x = tx * tw + (t & (tw - 1u)), y = ty * th + (t >> tshift);
-                const float d = min4(r0[k].x, r0[k].y, r1[k].x, r1[k].y);
-                bufA[t] = d;
-                lvl0[(size_t)y * J.base_w + x] = d;
-            }
+        if (x0 < bw && y0 < bh) {
+            const float4* p = reinterpret_cast<const float4*>(J.depth + (size_t)(2u * y0) * J.w) + x1;
+            const float4 r0 = p[0], r1 = p[J.w / 4u];
+            ta = min4(r0.x, r0.y, r1.x, r1.y);
+            tb = min4(r0.z, r0.w, r1.z, r1.w);
         }
     } else {
         // general ratio: the footprint rule; the base extent is a power of two, so (x + 0.5) / W equals
         // (x + 0.5) * (1 / W) exactly
-        const float rbw = 1.0f / (float)J.base_w, rbh = 1.0f / (float)J.base_h;
-        float d00[kPerThread], d01[kPerThread], d10[kPerThread], d11[kPerThread];
-#pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k) {
-            const uint32_t t0 = tid + k * NT, t = t0 < n0 ? t0 : 0u;
-            const uint32_t x = tx * tw + (t & (tw - 1u)), y = ty * th + (t >> tshift);
-            const Footprint f = footprint(((float)x + 0.5f) * rbw, ((float)y + 0.5f) * rbh, J.w, J.h);
-            d00[k] = J.depth[(size_t)f.y0 * J.w + f.x0];
-            d01[k] = J.depth[(size_t)f.y0 * J.w + f.x1];
-            d10[k] = J.depth[(size_t)f.y1 * J.w + f.x0];
-            d11[k] = J.depth[(size_t)f.y1 * J.w + f.x1];
+        const float rbw = 1.0f / (float)bw, rbh = 1.0f / (float)bh;
+        const uint32_t xa = x0 < bw ? x0 : bw - 1u, xb = x0 + 1u < bw ? x0 + 1u : bw - 1u, y = y0 < bh ? y0 : bh - 1u;
+        const Footprint f = footprint(((float)xa + 0.5f) * rbw, ((float)y + 0.5f) * rbh, J.w, J.h);
+        const Footprint e = footprint(((float)xb + 0.5f) * rbw, ((float)y + 0.5f) * rbh, J.w, J.h);
+        const float *r0 = J.depth + (size_t)f.y0 * J.w, *r1 = J.depth + (size_t)f.y1 * J.w;
+        float a0, a1, a2, a3, b0, b1, b2, b3;
+        if (J.w <= 2u * bw && J.w >= 4u) {
+            // At most two depth texels per base texel: the two footprints lie within four texels of a row (their
+            // positions differ by at most 2, so floor of the second is at most 2 further, and one more for its right
+            // neighbour), read as one 16-byte load that starts early enough to end inside the row. Eight 4-byte
+            // loads touched each line four times (1366 x 768 onto 1024 x 512: 7.2 us).
+            const uint32_t xs = f.x0 < J.w - 4u ? f.x0 : J.w - 4u;
+            const float4_unaligned p = *reinterpret_cast<const float4_unaligned*>(r0 + xs);
+            const float4_unaligned q = *reinterpret_cast<const float4_unaligned*>(r1 + xs);
+            auto pick = [](float4_unaligned r, uint32_t i) {
+                const float lo = i & 1u ? r.y : r.x, hi = i & 1u ? r.w : r.z;
+                return i & 2u ? hi : lo;
+            };
+            a0 = pick(p, f.x0 - xs);
+            a1 = pick(p, f.x1 - xs);
+            a2 = pick(q, f.x0 - xs);
+            a3 = pick(q, f.x1 - xs);
+            b0 = pick(p, e.x0 - xs);
+            b1 = pick(p, e.x1 - xs);
+            b2 = pick(q, e.x0 - xs);
+            b3 = pick(q, e.x1 - xs);
+        } else {
+            a0 = r0[f.x0], a1 = r0[f.x1], a2 = r1[f.x0], a3 = r1[f.x1];
+            b0 = r0[e.x0], b1 = r0[e.x1], b2 = r1[e.x0], b3 = r1[e.x1];
         }
-#pragma unroll
-        for (uint32_t k = 0; k < kPerThread; ++k) {
-            const uint32_t t = tid + k * NT;
-            if (t < n0) {
-                const uint32_t x = tx * tw + (t & (tw - 1u)), y = ty * th + (t >> tshift);
-                const float d = min4(d00[k], d01[k], d10[k], d11[k]);
-                bufA[t] = d;
-                lvl0[(size_t)y * J.base_w + x] = d;
-            }
-        }
+        if (x0 < bw && y0 < bh) ta = min4(a0, a1, a2, a3);
+        if (x0 + 1u < bw && y0 < bh) tb = min4(b0, b1, b2, b3);
+    }
+    if (y0 < bh) {  // (8-byte aligned: even pitch, and the levels start at the allocation's start)
+        if (x0 + 1u < bw) *reinterpret_cast<float2*>(J.texels + (size_t)y0 * bw + x0) = make_float2(ta, tb);
+        else if (x0 < bw) J.texels[(size_t)y0 * bw + x0] = ta;  // a base one texel wide
+    }
+    // ---- levels 1 and 2: (x1, y0 / 2) >> (L - 1) is the lane's texel of level L, stored by the first lane of its group
+    const uint32_t levels = J.tile_levels;
+    auto store = [&](uint32_t L, uint32_t x, uint32_t y, float t) {
+        const uint32_t w = level_dim(bw, L);
+        if (L < levels && x < w && y < level_dim(bh, L)) J.texels[J.level_offset[L] + (size_t)y * w + x] = t;
+    };
+    float v = min_across(glsl_min(ta, tb), lane, 16u);
+    if ((lane & 16u) == 0u) store(1u, x1, y0 >> 1, v);
+    v = min_across(glsl_min(quad_perm<0, 0, 2, 2>(v), quad_perm<1, 1, 3, 3>(v)), lane, 32u);
+    if ((lane & 49u) == 0u) {
+        store(2u, x1 >> 1, y0 >> 2, v);
+        sm.l2[wave * 8u + (lane >> 1)] = v;
     }
     __syncthreads();
-    // ---- levels inside the tile, in LDS
-    uint32_t cw = tw, ch = th;
-    float* src = bufA;
-    float* dst = bufB;
-    for (uint32_t L = 1; L < J.tile_levels; ++L) {
-        const uint32_t nw = cw > 1u ? cw >> 1 : 1u, nh = ch > 1u ? ch >> 1 : 1u;
-        reduce_lds<NT>(src, cw, ch, dst, nw, nh, J.texels + J.level_offset[L], level_dim(J.base_w, L), tx * nw, ty * nh);
-        __syncthreads();
-        float* tmp = src;
-        src = dst;
-        dst = tmp;
-        cw = nw;
-        ch = nh;
+    // ---- levels 3 to 5: lane = level-2 texel (lane & 7, lane >> 3) of the tile
+    const uint32_t n_tiles = J.tiles_x * J.tiles_y;
+    const bool tail = levels < J.mips && tile + 1u == n_tiles;
+    if (wave && !tail) return;
+    {
+        const uint32_t lx = lane & 7u, ly = lane >> 3;
+        v = sm.l2[lane];
+        v = min_across(glsl_min(quad_perm<0, 0, 2, 2>(v), quad_perm<1, 1, 3, 3>(v)), lane, 8u);
+        if (wave == 0u && ((lx | ly) & 1u) == 0u) store(3u, tx * 4u + (lx >> 1), ty * 4u + (ly >> 1), v);
+        v = min_across(glsl_min(quad_perm<0, 0, 0, 0>(v), quad_perm<2, 2, 2, 2>(v)), lane, 16u);
+        if (wave == 0u && ((lx | ly) & 3u) == 0u) store(4u, tx * 2u + (lx >> 2), ty * 2u + (ly >> 2), v);
+        v = min_across(min_across(v, lane, 4u), lane, 32u);
+        if (tid == 0u) store(5u, tx, ty, v);
     }
-    if (J.tile_levels >= J.mips) return;
+    if (levels >= J.mips) return;
     // ---- hand each tile's 1x1 value to the highest-numbered workgroup, which reduces the tail levels. The value
     // travels in a 64-bit agent-scope atomic word with a presence flag; the receiving workgroup clears each word
     // after reading it, so every build starts with all words zero. Neither a release fence (an L2 write-back per
     // workgroup) nor a shared completion counter (a serialised atomic per workgroup) is needed.
-    const uint32_t n_tiles = J.tiles_x * J.tiles_y;
-    if (tile + 1u < n_tiles) {
+    if (!tail) {
         if (tid == 0)
-            __hip_atomic_store(&J.tail[tile], kTailFlag | __float_as_uint(src[0]), __ATOMIC_RELAXED,
+            __hip_atomic_store(&J.tail[tile], kTailFlag | __float_as_uint(v), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    const float own = src[0];
-    __syncthreads();  // every thread has read `own` before bufA is rewritten
-    const uint32_t L0 = J.tile_levels - 1u;
-    cw = level_dim(J.base_w, L0);
-    ch = level_dim(J.base_h, L0);
-    if (n_tiles <= kTileTexels) {
-        // the whole tile image (one texel per tile, level L0) fits the LDS tile: every word of a thread is loaded
-        // before the first wait (one round trip), then the remaining levels are reduced in LDS
-        constexpr uint32_t KW = kTileTexels / NT;
-        unsigned long long w[KW];
+    // the tile image (one texel per tile, level 5): the words of a thread are loaded together, before the first wait
+    constexpr uint32_t KW = kPyrTailTexels * 4u / kPyrBlock;
+    unsigned long long w[KW];
 #pragma unroll
-        for (uint32_t k = 0; k < KW; ++k) {
-            const uint32_t i = tid + k * NT;
-            w[k] = (i < n_tiles && i != tile)
-                       ? __hip_atomic_load(&J.tail[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                       : 0ull;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < KW; ++k) {
-            const uint32_t i = tid + k * NT;
-            if (i < n_tiles) bufA[i] = i == tile ? own : tail_finish(J, i, w[k], err);
-        }
-        __syncthreads();
-        src = bufA;
-        dst = bufB;
-        for (uint32_t L = L0 + 1u; L < J.mips; ++L) {
-            const uint32_t nw = cw > 1u ? cw >> 1 : 1u, nh = ch > 1u ? ch >> 1 : 1u;
-            reduce_lds<NT>(src, cw, ch, dst, nw, nh, J.texels + J.level_offset[L], nw, 0u, 0u);
-            __syncthreads();
-            float* tmp = src;
-            src = dst;
-            dst = tmp;
-            cw = nw;
-            ch = nh;
-        }
-        return;
+    for (uint32_t k = 0; k < KW; ++k) {
+        const uint32_t i = tid + k * kPyrBlock;
+        w[k] = i < n_tiles ? __hip_atomic_load(&J.tail[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
     }
-    // larger tile images: reduced to the next level while they are collected
-    {
-        const uint32_t nw = cw > 1u ? cw >> 1 : 1u, nh = ch > 1u ? ch >> 1 : 1u;
-        const uint32_t nshift = (uint32_t)__builtin_ctz(nw);
-        float* g = J.texels + J.level_offset[L0 + 1u];
-        for (uint32_t t = tid; t < nw * nh; t += NT) {
-            const uint32_t x0 = 2u * (t & (nw - 1u)), y0 = 2u * (t >> nshift);
-            const bool hx = cw > 1u, hy = ch > 1u;  // a second column / row exists (else the clamp repeats the first)
-            const float v00 = tail_word(J, y0 * cw + x0, tile, own, err);
-            const float v01 = hx ? tail_word(J, y0 * cw + x0 + 1u, tile, own, err) : v00;
-            const float v10 = hy ? tail_word(J, (y0 + 1u) * cw + x0, tile, own, err) : v00;
-            const float v11 = (hx && hy) ? tail_word(J, (y0 + 1u) * cw + x0 + 1u, tile, own, err) : (hx ? v01 : v10);
-            const float d = min4(v00, v01, v10, v11);
-            bufA[t] = d;
-            g[t] = d;
-        }
+#pragma unroll
+    for (uint32_t k = 0; k < KW; ++k) {
+        const uint32_t i = tid + k * kPyrBlock;
+        if (i < n_tiles) sm.a[i] = i == tile ? v : tail_finish(J, i, w[k], err);
+    }
+    uint32_t nw = J.tiles_x, nh = J.tiles_y, cw, ch;
+    float* g;
+    float* src = sm.a;
+    float* dst = sm.b;
+    bool one_wave = false;
+    // the remaining levels in LDS; from the first of at most 64 texels on, by one wave
+    for (uint32_t L = levels; L < J.mips; ++L) {
+        if (one_wave) wave_lds_sync();
+        else __syncthreads();
         cw = nw;
         ch = nh;
-    }
-    __syncthreads();
-    src = bufA;
-    dst = bufB;
-    for (uint32_t L = L0 + 2u; L < J.mips; ++L) {
-        const uint32_t nw = cw > 1u ? cw >> 1 : 1u, nh = ch > 1u ? ch >> 1 : 1u;
-        reduce_lds<NT>(src, cw, ch, dst, nw, nh, J.texels + J.level_offset[L], nw, 0u, 0u);
-        __syncthreads();
+        nw = cw > 1u ? cw >> 1 : 1u;
+        nh = ch > 1u ? ch >> 1 : 1u;
+        if (!one_wave && nw * nh <= 64u) {
+            if (wave) return;
+            one_wave = true;
+        }
+        const uint32_t nshift = (uint32_t)__builtin_ctz(nw), dx = cw > 1u ? 1u : 0u, dy = ch > 1u ? cw : 0u;
+        g = J.texels + J.level_offset[L];
+        for (uint32_t t = tid; t < nw * nh; t += kPyrBlock) {
+            const float* p = src + (t >> nshift) * (dy ? 2u * cw : cw) + (t & (nw - 1u)) * (1u + dx);
+            const float m = min4(p[0], p[dx], p[dy], p[dx + dy]);
+            dst[t] = m;
+            g[t] = m;
+        }
         float* tmp = src;
         src = dst;
         dst = tmp;
-        cw = nw;
-        ch = nh;
     }
 }
 
-template <uint32_t NT>
-__global__ __launch_bounds__(NT) void pyramid_kernel(PyrBuildJob J, uint32_t* err)
+__global__ __launch_bounds__(kPyrBlock) void pyramid_kernel(PyrBuildJob J, uint32_t* err)
 {
-    __shared__ float bufA[kTileTexels];
-    __shared__ float bufB[kTileTexels / 2];
-    pyramid_tile<NT>(J, blockIdx.x, bufA, bufB, err);
+    __shared__ PyrSmem sm;
+    pyramid_tile(J, blockIdx.x, sm, err);
 }
 
 // Last entry of the ascending table `starts` that is <= x (searched in LDS when staged there).
@@ -261,20 +243,15 @@ __device__ __forceinline__ uint32_t last_le(const uint32_t* starts, uint32_t n, 
 
 // Many pyramids in one launch: workgroup (x, y) builds level-0 tile x of job y; workgroups past the job's tiles return
 // at once. The job index is the workgroup's y, so no table of first workgroups is searched (the search's load cost
-// each workgroup a round trip: the 256-view batch 336.6 us against 314.6 us); the descriptor is copied to LDS. Within
-// a job, workgroups are dispatched in tile order, so the job's last tile (which waits on the others' hand-off words)
-// starts after every tile it waits for.
+// each workgroup a round trip: the 256-view batch 336.6 us against 314.6 us), and the descriptor is read in place with
+// scalar loads. Within a job, workgroups are dispatched in tile order, so the job's last tile (which waits on the others'
+// hand-off words) starts after every tile it waits for.
 __global__ __launch_bounds__(kPyrBlock) void pyramid_batch_kernel(const PyrBuildJob* __restrict__ jobs, uint32_t* err)
 {
-    __shared__ float bufA[kTileTexels];
-    __shared__ float bufB[kTileTexels / 2];
-    __shared__ PyrBuildJob sJ;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&jobs[blockIdx.y]);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&sJ);
-    for (uint32_t w = threadIdx.x; w < sizeof(PyrBuildJob) / 4; w += kPyrBlock) dst[w] = src[w];
-    __syncthreads();
-    if (blockIdx.x >= sJ.tiles_x * sJ.tiles_y) return;
-    pyramid_tile<kPyrBlock>(sJ, blockIdx.x, bufA, bufB, err);
+    __shared__ PyrSmem sm;
+    const PyrBuildJob& J = jobs[blockIdx.y];
+    if (blockIdx.x >= J.tiles_x * J.tiles_y) return;
+    pyramid_tile(J, blockIdx.x, sm, err);
 }
 
 // General per-level footprint reduction (any sizes).
@@ -383,11 +360,7 @@ __global__ __launch_bounds__(256) void synth_depth_batch_kernel(const SynthJob* 
 
 hipError_t launch_pyramid(const PyrBuildJob& job, uint32_t* err, hipStream_t st)
 {
-    if (job.w == 2u * job.base_w && job.h == 2u * job.base_h)
-        hipLaunchKernelGGL(pyramid_kernel<kPyrBlock>, dim3(job.tiles_x * job.tiles_y), dim3(kPyrBlock), 0, st, job, err);
-    else
-        hipLaunchKernelGGL(pyramid_kernel<kPyrBlockWide>, dim3(job.tiles_x * job.tiles_y), dim3(kPyrBlockWide), 0, st,
-                           job, err);
+    hipLaunchKernelGGL(pyramid_kernel, dim3(job.tiles_x * job.tiles_y), dim3(kPyrBlock), 0, st, job, err);
     return hipGetLastError();
 }
 
