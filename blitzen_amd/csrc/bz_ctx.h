@@ -73,7 +73,9 @@ struct PyrPlan {
     uint32_t level_offset[kMaxMips] = {};
     uint64_t n_texels = 0;
     uint32_t tiles_x = 0, tiles_y = 0, tile_levels = 0;
-    bool single_pass = false;
+    bool single_pass = false;   // power-of-two extent, one launch (also in batches)
+    bool region = false;        // any other extent that one launch can take (tiles_x, tiles_y, tile_levels are its own)
+    uint64_t tail_words() const;
     PyramidDesc desc(const float* texels) const;
     PyrBuildJob build_job(const float* depth, uint32_t w, uint32_t h, float* texels, unsigned long long* tail) const;
 };
@@ -82,7 +84,11 @@ bool plan_pyramid(uint32_t base_w, uint32_t base_h, uint32_t mips, PyrPlan* out)
 
 struct Pyramid : PyrPlan {
     float* texels = nullptr;
-    unsigned long long* tail = nullptr;  // [tiles_x * tiles_y] flagged per-tile words of the single-pass build
+    unsigned long long* tail = nullptr;  // [tail_words()] flagged words of the single-launch builds
+    // a build that is not single_pass: by regions in one launch, or one launch per level
+    hipError_t launch_other(const float* depth, uint32_t w, uint32_t h, uint32_t wait_limit, uint32_t* err,
+                            hipStream_t st) const;
+    PyrRegion* plan_dev = nullptr;       // region builds: (tiles_x + tiles_y) * kRegionLevels
     PyramidDesc desc() const { return PyrPlan::desc(texels); }
     PyrBuildJob build_job(const float* depth, uint32_t w, uint32_t h) const
     {

@@ -74,6 +74,18 @@ constexpr uint32_t kPyrTile = 32;           // level-0 tile edge of the single-p
 constexpr uint32_t kPyrTileLevels = 6;      // its levels: 32 x 32 ... 1 x 1
 constexpr uint32_t kPyrTailTexels = 1024;   // the tile image's first reduction, held by the tail workgroup
 
+// Other extents in one launch: a workgroup's region of each level along one axis. It stores texels [begin, end) and
+// computes [begin, need).
+constexpr uint32_t kRegionTile = 2;         // texels of the last level per workgroup and axis
+constexpr uint32_t kRegionLevels = 5;       // at most this many levels in the regions
+constexpr uint32_t kRegionMax = 48;         // a region's widest levels 0, 2, 4 (half of it: levels 1, 3)
+constexpr uint32_t kRegionTail = 8192;      // texels of the last level, held by the tail workgroup
+struct PyrRegion {
+    uint32_t begin, end, need;
+};
+// Fills the regions of one axis of `base` texels, kRegionLevels per tile, for levels 0 .. K; false if one is too wide.
+bool plan_region_axis(uint32_t base, uint32_t K, PyrRegion* out);
+
 struct PyrBuildJob {
     const float* depth;
     uint32_t w, h;
@@ -84,6 +96,7 @@ struct PyrBuildJob {
     uint32_t wg_start;                           // batched: first workgroup of this job
     uint32_t spin_limit;                         // sleeps before a wait for a tail word gives up
     unsigned long long* tail;                    // per job: one flagged word per tile, zero between builds
+    const PyrRegion* plan;                       // region builds: the tiles' regions along x, then along y
     uint32_t level_offset[16];
 };
 
@@ -188,6 +201,7 @@ hipError_t launch_pyramid(const PyrBuildJob& job, uint32_t* err, hipStream_t st)
 // Many pyramid builds in one launch, one workgroup per (level-0 tile, job); max_tiles = the largest job's tiles.
 hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_dev, uint32_t n_jobs, uint32_t max_tiles, uint32_t* err,
                                 hipStream_t st);
+hipError_t launch_pyramid_region(const PyrBuildJob& job, uint32_t* err, hipStream_t st);
 hipError_t launch_pyramid_level(const float* src, uint32_t sw, uint32_t sh, float* dst, uint32_t dw, uint32_t dh,
                                 hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t st);

@@ -86,6 +86,13 @@ Pyramid::~Pyramid()
 {
     if (texels) (void)hipFree(texels);
     if (tail) (void)hipFree(tail);
+    if (plan_dev) (void)hipFree(plan_dev);
+}
+
+uint64_t PyrPlan::tail_words() const
+{
+    if (region) return (uint64_t)level_dim(base_w, tile_levels - 1u) * level_dim(base_h, tile_levels - 1u);
+    return (uint64_t)tiles_x * tiles_y;
 }
 
 StreamScratch::~StreamScratch()
@@ -236,6 +243,16 @@ bool plan_pyramid(uint32_t base_w, uint32_t base_h, uint32_t mips, PyrPlan* p)
     // single pass: power-of-two extent, and the tile image's first reduction fits the tail workgroup's LDS tile
     const uint64_t tail_texels = (uint64_t)std::max(1u, p->tiles_x / 2u) * std::max(1u, p->tiles_y / 2u);
     p->single_pass = pow2 && (p->tile_levels >= mips || tail_texels <= kPyrTailTexels);
+    if (!p->single_pass) {  // the regions of the last level must all reach one workgroup's LDS
+        const uint32_t K = std::min(kRegionLevels, mips) - 1u;
+        const uint32_t w = level_dim(base_w, K), h = level_dim(base_h, K);
+        if ((uint64_t)w * h <= kRegionTail) {
+            p->region = true;
+            p->tile_levels = K + 1u;
+            p->tiles_x = (w + kRegionTile - 1u) / kRegionTile;
+            p->tiles_y = (h + kRegionTile - 1u) / kRegionTile;
+        }
+    }
     return true;
 }
 
@@ -764,9 +781,18 @@ bz_status bz_pyramid_create(bz_ctx* ctx, uint32_t base_w, uint32_t base_h, uint3
     // one spare texel past the last level: the Hi-Z lookup reads texels in pairs (footprint_texels)
     hipError_t e = hipMalloc((void**)&p->texels, (off + 1) * 4);
     if (e == hipSuccess) e = hipMemset(p->texels, 0, (off + 1) * 4);
-    const size_t n_tiles = (size_t)p->tiles_x * p->tiles_y;
-    if (e == hipSuccess) e = hipMalloc((void**)&p->tail, n_tiles * 8);
-    if (e == hipSuccess) e = hipMemset(p->tail, 0, n_tiles * 8);
+    if (p->region) {
+        std::vector<PyrRegion> plan((size_t)(p->tiles_x + p->tiles_y) * kRegionLevels);
+        const uint32_t K = p->tile_levels - 1u;
+        p->region = plan_region_axis(base_w, K, plan.data()) &&
+                    plan_region_axis(base_h, K, plan.data() + (size_t)p->tiles_x * kRegionLevels);
+        if (p->region && e == hipSuccess) e = hipMalloc((void**)&p->plan_dev, plan.size() * sizeof(PyrRegion));
+        if (p->region && e == hipSuccess)
+            e = hipMemcpy(p->plan_dev, plan.data(), plan.size() * sizeof(PyrRegion), hipMemcpyHostToDevice);
+    }
+    const size_t tail_bytes = (size_t)p->tail_words() * 8;
+    if (e == hipSuccess) e = hipMalloc((void**)&p->tail, tail_bytes);
+    if (e == hipSuccess) e = hipMemset(p->tail, 0, tail_bytes);
     if (e != hipSuccess) return ctx->hip_fail(e, "pyramid allocation");
     const bz_pyramid h = ++ctx->next_handle;
     ctx->pyramids[h] = std::move(p);
@@ -829,14 +855,26 @@ bz_status Ctx::build_pyramid(Pyramid* p, const float* depth, uint32_t w, uint32_
         j.spin_limit = wait_limit;
         e = launch_pyramid(j, sc->err + 1, st);
     } else {
-        e = launch_pyramid_level(depth, w, h, p->texels, p->base_w, p->base_h, st);
-        for (uint32_t L = 1; L < p->mips && e == hipSuccess; ++L)
-            e = launch_pyramid_level(p->texels + p->level_offset[L - 1], level_dim(p->base_w, L - 1),
-                                     level_dim(p->base_h, L - 1), p->texels + p->level_offset[L],
-                                     level_dim(p->base_w, L), level_dim(p->base_h, L), st);
+        e = p->launch_other(depth, w, h, wait_limit, sc->err + 1, st);
     }
     if (e != hipSuccess) return hip_fail(e, "pyramid launch");
     return BZ_OK;
+}
+
+hipError_t Pyramid::launch_other(const float* depth, uint32_t w, uint32_t h, uint32_t wait_limit, uint32_t* err,
+                                 hipStream_t st) const
+{
+    if (region) {
+        PyrBuildJob j = build_job(depth, w, h);
+        j.spin_limit = wait_limit;
+        j.plan = plan_dev;
+        return launch_pyramid_region(j, err, st);
+    }
+    hipError_t e = launch_pyramid_level(depth, w, h, texels, base_w, base_h, st);
+    for (uint32_t L = 1; L < mips && e == hipSuccess; ++L)
+        e = launch_pyramid_level(texels + level_offset[L - 1], level_dim(base_w, L - 1), level_dim(base_h, L - 1),
+                                 texels + level_offset[L], level_dim(base_w, L), level_dim(base_h, L), st);
+    return e;
 }
 }  // namespace bz
 
@@ -1303,7 +1341,7 @@ bz_status bz_check(bz_ctx* ctx, void* stream)
         e = hipDeviceSynchronize();
         for (auto& p : ctx->pyramids)
             if (e == hipSuccess && p.second->tail)
-                e = hipMemset(p.second->tail, 0, (size_t)p.second->tiles_x * p.second->tiles_y * 8u);
+                e = hipMemset(p.second->tail, 0, (size_t)p.second->tail_words() * 8u);
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e != hipSuccess) return ctx->hip_fail(e, "pyramid hand-off reset");
     }
@@ -1399,12 +1437,7 @@ bz_status bz_batch_graph_create(bz_ctx* ctx, const bz_pyramid_job* pyr_jobs, uin
     }
     for (auto& m : multi) {
         if (e != hipSuccess) break;
-        Pyramid* p = m.first;
-        e = launch_pyramid_level(m.second.depth_dev, m.second.w, m.second.h, p->texels, p->base_w, p->base_h, cs);
-        for (uint32_t L = 1; L < p->mips && e == hipSuccess; ++L)
-            e = launch_pyramid_level(p->texels + p->level_offset[L - 1], level_dim(p->base_w, L - 1),
-                                     level_dim(p->base_h, L - 1), p->texels + p->level_offset[L],
-                                     level_dim(p->base_w, L), level_dim(p->base_h, L), cs);
+        e = m.first->launch_other(m.second.depth_dev, m.second.w, m.second.h, ctx->wait_limit, g->err + 1, cs);
     }
     if (e == hipSuccess) e = zero_counts(empty, cs);
     if (e == hipSuccess && !cj.empty())

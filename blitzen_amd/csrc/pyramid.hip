@@ -7,8 +7,8 @@
 // Single pass for power-of-two bases: each workgroup owns a tile of level 0 (32 x 32 texels), writes it,
 // and reduces it in registers down to 1 x 1 (levels 1..5, exact 2:1 with edge clamp). The last workgroup
 // (the highest-numbered one, waiting on flagged words) reduces the remaining levels from the
-// 1-texel-per-tile image. Non-power-of-two
-// bases fall back to one launch per level with the general footprint rule.
+// 1-texel-per-tile image. Other bases go by regions, also in one launch (pyramid_region_kernel), and those too large for
+// either take one launch per level with the general footprint rule.
 #include "bz_internal.h"
 #include "synth_rng.h"
 
@@ -254,6 +254,151 @@ __global__ __launch_bounds__(kPyrBlock) void pyramid_batch_kernel(const PyrBuild
     pyramid_tile(J, blockIdx.x, sm, err);
 }
 
+// The coordinates of a footprint along one axis: texels i0 and i1 (equal when the second has no weight) of `src` texels
+// below texel x of `dst` (footprint() of cull_math.h, axis by axis).
+__device__ __forceinline__ void footprint_axis(uint32_t x, uint32_t dst, uint32_t src, uint32_t& i0, uint32_t& i1)
+{
+    const float u = ((float)x + 0.5f) / (float)dst;
+    const float t = u * (float)src - 0.5f, f = floorf(t);
+    i0 = clamp_texel(f, src);
+    i1 = (t - f) > 0.0f ? clamp_texel(f + 1.0f, src) : i0;
+}
+
+// Extents that are not powers of two, in one launch. A workgroup owns kRegionTile x kRegionTile texels of level K (the
+// last of `tile_levels`) and, of every level below, the texels from the first one under its own first texel to the first
+// one under the next tile's; it computes those and the few of its neighbours' that its own footprints reach into (the
+// plan's `need`), level by level in LDS, and stores what it owns. Level K then goes to the highest-numbered workgroup as
+// flagged words, like the tile image of the power-of-two build, which reduces the levels that remain. One launch per
+// level, as larger bases still take, costs a launch and a round trip per level for ever fewer texels (800 x 450 with 10
+// mips: 10.2 us against 21.5 us of kernels, 30 us a build where the host is the bound). Two texels of level 4 and axis per
+// workgroup: 350 workgroups for 800 x 450, each computing at most 47 x 47 texels of level 0 for 32 x 32 of its own.
+constexpr uint32_t kRegionBlock = 512;
+struct RegionSmem {
+    uint32_t c0[2][kRegionLevels][kRegionMax], c1[2][kRegionLevels][kRegionMax];  // per axis and level: footprint
+    float a[kRegionTail];                       // level 0, 2, 4 of the region; then the tail's image ...
+    float b[kRegionTail / 2u];                  // levels 1, 3; then its levels in turn (half: an image one texel wide)
+};
+static_assert(kRegionMax * kRegionMax <= kRegionTail, "the region's level 0 fits the tail's image");
+
+__global__ __launch_bounds__(kRegionBlock) void pyramid_region_kernel(PyrBuildJob J, uint32_t* err)
+{
+    __shared__ RegionSmem sm;
+    const uint32_t tid = threadIdx.x, lx = tid & 31u, ly = tid >> 5;
+    const uint32_t K = J.tile_levels - 1u;
+    const PyrRegion* px = J.plan + (size_t)(blockIdx.x % J.tiles_x) * kRegionLevels;
+    const PyrRegion* py = J.plan + (size_t)(J.tiles_x + blockIdx.x / J.tiles_x) * kRegionLevels;
+    for (uint32_t q = tid; q < 2u * kRegionLevels * kRegionMax; q += kRegionBlock) {
+        const uint32_t axis = q / (kRegionLevels * kRegionMax), L = q / kRegionMax % kRegionLevels, i = q % kRegionMax;
+        const PyrRegion* p = axis ? py : px;
+        if (L <= K && p[L].begin + i < p[L].need) {
+            const uint32_t base = axis ? J.base_h : J.base_w;
+            const uint32_t src = L ? level_dim(base, L - 1u) : (axis ? J.h : J.w), off = L ? p[L - 1u].begin : 0u;
+            uint32_t i0, i1;
+            footprint_axis(p[L].begin + i, level_dim(base, L), src, i0, i1);
+            sm.c0[axis][L][i] = i0 - off;
+            sm.c1[axis][L][i] = i1 - off;
+        }
+    }
+    __syncthreads();
+    // ---- level 0 from the depth image: the loads of three texels of a thread before the first minimum
+    {
+        const PyrRegion rx = px[0], ry = py[0];
+        const uint32_t nw = rx.need - rx.begin, nh = ry.need - ry.begin;
+        for (uint32_t x = lx; x < nw; x += 32u) {
+            const uint32_t x0 = sm.c0[0][0][x], x1 = sm.c1[0][0][x];
+            for (uint32_t yb = ly; yb < nh; yb += 48u) {
+                float d[3][4];
+#pragma unroll
+                for (uint32_t k = 0; k < 3u; ++k) {
+                    const uint32_t y = yb + 16u * k < nh ? yb + 16u * k : yb;
+                    const float* r0 = J.depth + (size_t)sm.c0[1][0][y] * J.w;
+                    const float* r1 = J.depth + (size_t)sm.c1[1][0][y] * J.w;
+                    d[k][0] = r0[x0];
+                    d[k][1] = r0[x1];
+                    d[k][2] = r1[x0];
+                    d[k][3] = r1[x1];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 3u; ++k) {
+                    const uint32_t y = yb + 16u * k;
+                    if (y >= nh) continue;
+                    const float m = min4(d[k][0], d[k][1], d[k][2], d[k][3]);
+                    sm.a[y * kRegionMax + x] = m;
+                    if (rx.begin + x < rx.end && ry.begin + y < ry.end)
+                        J.texels[(size_t)(ry.begin + y) * J.base_w + rx.begin + x] = m;
+                }
+            }
+        }
+    }
+    const bool handoff = J.tile_levels < J.mips;
+    for (uint32_t L = 1; L <= K; ++L) {
+        __syncthreads();
+        const float* src = (L & 1u) ? sm.a : sm.b;
+        float* dst = (L & 1u) ? sm.b : sm.a;
+        const uint32_t ps = (L & 1u) ? kRegionMax : kRegionMax / 2u, pd = (L & 1u) ? kRegionMax / 2u : kRegionMax;
+        const PyrRegion rx = px[L], ry = py[L];
+        const uint32_t nw = rx.need - rx.begin, nh = ry.need - ry.begin, W = level_dim(J.base_w, L);
+        float* g = J.texels + J.level_offset[L];
+        for (uint32_t y = ly; y < nh; y += 16u) {
+            const float* r0 = src + sm.c0[1][L][y] * ps;
+            const float* r1 = src + sm.c1[1][L][y] * ps;
+            for (uint32_t x = lx; x < nw; x += 32u) {
+                const uint32_t x0 = sm.c0[0][L][x], x1 = sm.c1[0][L][x];
+                const float m = min4(r0[x0], r0[x1], r1[x0], r1[x1]);
+                dst[y * pd + x] = m;
+                if (rx.begin + x < rx.end && ry.begin + y < ry.end) {
+                    const size_t at = (size_t)(ry.begin + y) * W + rx.begin + x;
+                    g[at] = m;
+                    if (L == K && handoff)
+                        __hip_atomic_store(&J.tail[at], kTailFlag | __float_as_uint(m), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+    }
+    if (!handoff || blockIdx.x + 1u < gridDim.x) return;
+    // ---- the tail: level K from all workgroups (this one's too), then the levels that remain, in LDS
+    __syncthreads();
+    uint32_t nw = level_dim(J.base_w, K), nh = level_dim(J.base_h, K);
+    constexpr uint32_t KW = 8;  // words of a thread in flight
+    for (uint32_t i0 = 0; i0 < nw * nh; i0 += KW * kRegionBlock) {
+        unsigned long long w[KW];
+#pragma unroll
+        for (uint32_t k = 0; k < KW; ++k) {
+            const uint32_t i = i0 + k * kRegionBlock + tid;
+            w[k] = i < nw * nh ? __hip_atomic_load(&J.tail[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < KW; ++k) {
+            const uint32_t i = i0 + k * kRegionBlock + tid;
+            if (i < nw * nh) sm.a[i] = tail_finish(J, i, w[k], err);
+        }
+    }
+    const float* src = sm.a;
+    float* dst = sm.b;
+    for (uint32_t L = J.tile_levels; L < J.mips; ++L) {
+        __syncthreads();
+        const uint32_t cw = nw, ch = nh;
+        nw = level_dim(J.base_w, L);
+        nh = level_dim(J.base_h, L);
+        float* g = J.texels + J.level_offset[L];
+        for (uint32_t y = ly; y < nh; y += 16u) {
+            uint32_t y0, y1;
+            footprint_axis(y, nh, ch, y0, y1);
+            for (uint32_t x = lx; x < nw; x += 32u) {
+                uint32_t x0, x1;
+                footprint_axis(x, nw, cw, x0, x1);
+                const float m = min4(src[y0 * cw + x0], src[y0 * cw + x1], src[y1 * cw + x0], src[y1 * cw + x1]);
+                dst[y * nw + x] = m;
+                g[y * nw + x] = m;
+            }
+        }
+        const float* done = dst;
+        dst = dst == sm.b ? sm.a : sm.b;
+        src = done;
+    }
+}
+
 // General per-level footprint reduction (any sizes).
 __global__ void pyramid_level_kernel(const float* __restrict__ src, uint32_t sw, uint32_t sh, float* __restrict__ dst,
                                      uint32_t dw, uint32_t dh)
@@ -375,6 +520,43 @@ hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_dev, uint32_t n_jobs, ui
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
+    return hipGetLastError();
+}
+
+// The regions of one axis (kRegionLevels per tile): the same float arithmetic as the kernel's footprints.
+bool plan_region_axis(uint32_t base, uint32_t K, PyrRegion* out)
+{
+    const uint32_t n = level_dim(base, K), tiles = (n + kRegionTile - 1u) / kRegionTile;
+    auto at = [&](uint32_t L, uint32_t x, uint32_t& i0, uint32_t& i1) {  // footprint of level L's texel x in level L - 1
+        const uint32_t src = level_dim(base, L - 1u);
+        const Footprint f = footprint(((float)x + 0.5f) / (float)level_dim(base, L), 0.0f, src, 1u);
+        i0 = f.x0;
+        i1 = f.x1;
+    };
+    for (uint32_t t = 0; t < tiles; ++t) {
+        PyrRegion* r = out + (size_t)t * kRegionLevels;
+        for (uint32_t L = 0; L < kRegionLevels; ++L) r[L] = PyrRegion{ 0u, 0u, 0u };
+        r[K].begin = t * kRegionTile;
+        r[K].end = t + 1u < tiles ? (t + 1u) * kRegionTile : n;
+        r[K].need = r[K].end;
+        for (uint32_t L = K; L >= 1u; --L) {
+            uint32_t i0, i1;
+            at(L, r[L].begin, i0, i1);
+            r[L - 1u].begin = t ? i0 : 0u;
+            if (t + 1u < tiles) at(L, r[L].end, r[L - 1u].end, i1);
+            else r[L - 1u].end = level_dim(base, L - 1u);
+            at(L, r[L].need - 1u, i0, i1);
+            r[L - 1u].need = i1 + 1u > r[L - 1u].end ? i1 + 1u : r[L - 1u].end;
+            const uint32_t room = ((L - 1u) & 1u) ? kRegionMax / 2u : kRegionMax;
+            if (r[L - 1u].need - r[L - 1u].begin > room) return false;
+        }
+    }
+    return true;
+}
+
+hipError_t launch_pyramid_region(const PyrBuildJob& job, uint32_t* err, hipStream_t st)
+{
+    hipLaunchKernelGGL(pyramid_region_kernel, dim3(job.tiles_x * job.tiles_y), dim3(kRegionBlock), 0, st, job, err);
     return hipGetLastError();
 }
 

@@ -21,6 +21,11 @@ SHAPES = [(1, 1, 1, 1, 1), (2, 2, 1, 1, 3), (5, 3, 2, 1, 4), (3, 130, 1, 64, 9),
           (64, 64, 32, 32, 6), (64, 64, 32, 32, 9), (70, 50, 64, 32, 7), (128, 64, 64, 32, 5), (100, 200, 32, 128, 8),
           (512, 4, 256, 2, 9), (700, 1, 512, 1, 10), (256, 256, 128, 128, 3), (1366, 768, 1024, 512, 11),
           (4096, 4096, 2048, 2048, 12), (3001, 1500, 2048, 1024, 12)]
+# not powers of two: regions of one tile and of many, odd halves, one texel wide or high, fewer and more levels than the
+# regions hold, the largest image of the last level (120 x 67) and one that takes a launch per level (128 x 68)
+SHAPES += [(5, 5, 3, 5, 3), (37, 23, 18, 11, 5), (101, 7, 99, 1, 7), (7, 3000, 1, 1500, 11), (1000, 777, 500, 388, 9),
+           (640, 360, 321, 179, 1), (640, 360, 320, 181, 4), (1600, 900, 800, 450, 10), (1366, 768, 683, 384, 12),
+           (3840, 2160, 1920, 1080, 11), (4100, 2200, 2050, 1100, 12)]
 
 
 def image(w, h, seed, odd_values):
