@@ -106,7 +106,7 @@ struct StreamScratch {
     PyrBuildJob* pjobs_dev = nullptr;
     PyrBuildJob* pjobs_host = nullptr;
     uint32_t pjobs_cap = 0;
-    hipEvent_t upload_done = nullptr; // last job-table upload from the pinned buffers
+    hipEvent_t jobs_copied = nullptr, pjobs_copied = nullptr;  // the tables' last copies from the pinned buffers
     ClusterScratch xs{};              // cluster pass
     uint32_t* inst_hist = nullptr;    // LOD-instanced output: chunk x LOD histogram, then each chunk's first slots
     uint64_t inst_hist_cap = 0;
@@ -195,14 +195,15 @@ ViewConsts make_view_consts(const bz_CameraViewData& v);
 // Device address of the fixed scratch array on `device` (the current device), looked up once per device.
 hipError_t noalloc_scratch_address(int device, void** out);
 
-// Job tables live in one allocation: cap descriptors, then cap uint32 first-tile (or first-workgroup) indices, which
-// the batched kernels stage in LDS for their job lookup. The host copy is pinned and reused once the previous
-// upload from it has completed.
+// Job tables live in one allocation: n descriptors, then their n uint32 first-tile (or first-workgroup) indices, sent in
+// one copy. The host copy is pinned and reused once the previous copy from it has completed: `wait` is an event not
+// earlier than that copy, and `record` (may be nullptr) is recorded behind this one, so that a caller's next batch is
+// prepared while the kernels of this one run.
 template <class T>
-inline bz_status upload_table(Ctx* ctx, T*& dev, T*& host, uint32_t& cap, hipEvent_t done, const T* jobs,
-                              const uint32_t* starts, uint32_t n, hipStream_t st, const char* what)
+inline bz_status upload_table(Ctx* ctx, T*& dev, T*& host, uint32_t& cap, hipEvent_t wait, hipEvent_t record,
+                              const T* jobs, const uint32_t* starts, uint32_t n, hipStream_t st, const char* what)
 {
-    (void)hipEventSynchronize(done);
+    (void)hipEventSynchronize(wait);
     if (cap < n) {
         if (dev) (void)hipFree(dev);
         if (host) (void)hipHostFree(host);
@@ -216,20 +217,18 @@ inline bz_status upload_table(Ctx* ctx, T*& dev, T*& host, uint32_t& cap, hipEve
         if (e != hipSuccess) return ctx->hip_fail(e, what);
         cap = c;
     }
-    char* hs = reinterpret_cast<char*>(host) + (size_t)cap * sizeof(T);
-    char* ds = reinterpret_cast<char*>(dev) + (size_t)cap * sizeof(T);
     std::memcpy(host, jobs, (size_t)n * sizeof(T));
-    std::memcpy(hs, starts, (size_t)n * 4);
-    hipError_t e = hipMemcpyAsync(dev, host, (size_t)n * sizeof(T), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(ds, hs, (size_t)n * 4, hipMemcpyHostToDevice, st);
+    std::memcpy(reinterpret_cast<char*>(host) + (size_t)n * sizeof(T), starts, (size_t)n * 4);
+    hipError_t e = hipMemcpyAsync(dev, host, (size_t)n * (sizeof(T) + 4), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && record) e = hipEventRecord(record, st);
     if (e != hipSuccess) return ctx->hip_fail(e, what);
     return BZ_OK;
 }
 
 template <class T>
-inline const uint32_t* table_starts(const T* dev, uint32_t cap)
+inline const uint32_t* table_starts(const T* dev, uint32_t n)
 {
-    return reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(dev) + (size_t)cap * sizeof(T));
+    return dev ? reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(dev) + (size_t)n * sizeof(T)) : nullptr;
 }
 
 uint32_t tiles_for(uint32_t n, uint32_t block, uint32_t items);

@@ -52,16 +52,23 @@ struct CullJob {
 
 // Scratch of the two-kernel compaction: per-tile command counts and per-tile staging slots (objectId, LOD) of
 // tile_size entries each, and room for the counts' exclusive prefix. Fully rewritten by every decide launch; nothing
-// needs clearing between launches. `counts` and `prefix` share one allocation of counts_words(capacity_tiles).
+// needs clearing between launches. `counts` and `prefix` share one allocation of counts_words(capacity_tiles), with
+// `tile_job` behind them batch_words(capacity_tiles).
 struct CompactScratch {
     uint32_t* counts;            // [capacity_tiles]
     uint2* staging;              // [capacity_entries]
     uint32_t capacity_tiles;
     uint64_t capacity_entries;
     uint32_t* prefix;            // [capacity_tiles + 1] exclusive prefix of counts (written by the scan, when used)
+    uint32_t* tile_job;          // [capacity_tiles] batches: the job of each tile (nullptr in the fixed scratch)
 };
 constexpr uint64_t counts_words(uint32_t capacity_tiles) { return 2ull * capacity_tiles + 1u; }
-inline void set_prefix(CompactScratch& s) { s.prefix = s.counts ? s.counts + s.capacity_tiles : nullptr; }
+constexpr uint64_t batch_words(uint64_t capacity_tiles) { return 3ull * capacity_tiles + 1u; }  // with tile_job
+inline void set_prefix(CompactScratch& s, bool batches)
+{
+    s.prefix = s.counts ? s.counts + s.capacity_tiles : nullptr;
+    s.tile_job = s.counts && batches ? s.prefix + s.capacity_tiles + 1u : nullptr;
+}
 
 // An emit workgroup adds the counts of its job's earlier tiles itself when there are at most kScanTiles of them (one
 // round of loads). A job with more tiles gets their exclusive prefix from one scan launch between the decide and the
@@ -184,8 +191,19 @@ constexpr uint32_t kArgJobs = 512;
 struct JobStartsArg {
     uint32_t v[kArgJobs];
 };
-// jobs_host: the same n_jobs jobs in host memory (their tile_start values fill the kernel-argument table)
-// starts_dev: the jobs' tile_start values as a compact ascending array (the batched kernels stage it in LDS)
+// A batch of up to kArgFullJobs jobs travels whole in the kernel arguments: no table in device memory, no copy.
+constexpr uint32_t kArgFullJobs = 12;
+struct JobArgs {
+    CullJob j[kArgFullJobs];
+};
+constexpr uint32_t kArgPyrJobs = 16;
+struct PyrArgs {
+    PyrBuildJob j[kArgPyrJobs];
+};
+static_assert(sizeof(JobArgs) <= 3840 && sizeof(PyrArgs) <= 3840, "kernel arguments are at most 4 KiB");
+// jobs_host: the same n_jobs jobs in host memory (they, or their tile_start values, fill the kernel arguments)
+// jobs_dev, starts_dev: the jobs, and their tile_start values as a compact ascending array; not read (nullptr) up to
+// kArgFullJobs jobs
 // max_job_tiles: the largest job's tile count (above kScanTiles the emit reads a scanned prefix of the batch)
 hipError_t launch_cull_batch(const CullJob* jobs_host, const CullJob* jobs_dev, const uint32_t* starts_dev,
                              uint32_t n_jobs, uint32_t total_tiles, uint32_t max_job_tiles, const CompactScratch& s,
@@ -197,10 +215,10 @@ inline uint32_t max_job_tiles(const CullJob* jobs, size_t n)
     return m;
 }
 hipError_t launch_pyramid(const PyrBuildJob& job, uint32_t* err, hipStream_t st);
-// starts_dev: the jobs' wg_start values as a compact ascending array (the batched kernels stage it in LDS)
-// Many pyramid builds in one launch, one workgroup per (level-0 tile, job); max_tiles = the largest job's tiles.
-hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_dev, uint32_t n_jobs, uint32_t max_tiles, uint32_t* err,
-                                hipStream_t st);
+// Many pyramid builds in one launch, one workgroup per (level-0 tile, job). jobs_dev is not read (nullptr) up to
+// kArgPyrJobs jobs.
+hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_host, const PyrBuildJob* jobs_dev, uint32_t n_jobs,
+                                uint32_t* err, hipStream_t st);
 hipError_t launch_pyramid_region(const PyrBuildJob& job, uint32_t* err, hipStream_t st);
 hipError_t launch_pyramid_level(const float* src, uint32_t sw, uint32_t sh, float* dst, uint32_t dw, uint32_t dh,
                                 hipStream_t st);

@@ -103,7 +103,8 @@ StreamScratch::~StreamScratch()
         if (p) (void)hipFree(p);
     if (jobs_host) (void)hipHostFree(jobs_host);
     if (pjobs_host) (void)hipHostFree(pjobs_host);
-    if (upload_done) (void)hipEventDestroy(upload_done);
+    if (jobs_copied) (void)hipEventDestroy(jobs_copied);
+    if (pjobs_copied) (void)hipEventDestroy(pjobs_copied);
 }
 
 // Compaction scratch for `stream`, sized for at least `tiles` tiles and `entries` staging entries. Growth
@@ -118,7 +119,8 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(error flags)");
         e = hipMemset(s.err, 0, 16);
         if (e != hipSuccess) return hip_fail(e, "hipMemset(error flags)");
-        e = hipEventCreateWithFlags(&s.upload_done, hipEventDisableTiming);
+        e = hipEventCreateWithFlags(&s.jobs_copied, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&s.pjobs_copied, hipEventDisableTiming);
         if (e != hipSuccess) return hip_fail(e, "hipEventCreate");
     }
     if (s.cs.capacity_tiles < tiles || s.cs.capacity_entries < entries) {
@@ -133,12 +135,12 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
         if (s.cs.counts) (void)hipFree(s.cs.counts);
         if (s.cs.staging) (void)hipFree(s.cs.staging);
         s.cs = CompactScratch{};
-        e = hipMalloc((void**)&s.cs.counts, (size_t)counts_words(cap_t) * 4);
+        e = hipMalloc((void**)&s.cs.counts, (size_t)batch_words(cap_t) * 4);
         if (e == hipSuccess) e = hipMalloc((void**)&s.cs.staging, (size_t)cap_e * sizeof(uint2));
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(compaction scratch)");
         s.cs.capacity_tiles = cap_t;
         s.cs.capacity_entries = cap_e;
-        set_prefix(s.cs);
+        set_prefix(s.cs, true);
     }
     *out = &s;
     return BZ_OK;
@@ -219,7 +221,6 @@ PyramidDesc PyrPlan::desc(const float* texels) const
     p.base_w = base_w;
     p.base_h = base_h;
     p.mips = mips;
-    for (uint32_t i = 0; i < mips && i < (uint32_t)kMaxMips; ++i) p.level_offset[i] = level_offset[i];
     return p;
 }
 
@@ -919,12 +920,9 @@ bz_status bz_pyramid_build_batch(bz_ctx* ctx, const bz_pyramid_job* jobs, uint32
     StreamScratch* sc = nullptr;
     bz_status s = ctx->scratch_for(st, 0, 0, &sc);
     if (s) return s;
-    s = ctx->upload_pjobs(sc, sp.data(), (uint32_t)sp.size(), st);
+    if (sp.size() > kArgPyrJobs) s = ctx->upload_pjobs(sc, sp.data(), (uint32_t)sp.size(), st);
     if (s) return s;
-    uint32_t mt = 0;
-    for (auto& q : sp) mt = std::max<uint32_t>(mt, q.tiles_x * q.tiles_y);
-    hipError_t e = launch_pyramid_batch(sc->pjobs_dev, (uint32_t)sp.size(), mt, sc->err + 1, st);
-    if (e == hipSuccess) e = hipEventRecord(sc->upload_done, st);
+    hipError_t e = launch_pyramid_batch(sp.data(), sc->pjobs_dev, (uint32_t)sp.size(), sc->err + 1, st);
     if (e != hipSuccess) return ctx->hip_fail(e, "pyramid batch launch");
     return BZ_OK;
 }
@@ -1208,7 +1206,8 @@ bz_status Ctx::upload_jobs(StreamScratch* sc, const CullJob* jobs, uint32_t n, h
 {
     std::vector<uint32_t> starts(n);
     for (uint32_t k = 0; k < n; ++k) starts[k] = jobs[k].tile_start;
-    return upload_table(this, sc->jobs_dev, sc->jobs_host, sc->jobs_cap, sc->upload_done, jobs, starts.data(), n, st,
+    return upload_table(this, sc->jobs_dev, sc->jobs_host, sc->jobs_cap, sc->jobs_copied, sc->jobs_copied, jobs,
+                        starts.data(), n, st,
                         "job table upload");
 }
 
@@ -1216,7 +1215,8 @@ bz_status Ctx::upload_pjobs(StreamScratch* sc, const PyrBuildJob* jobs, uint32_t
 {
     std::vector<uint32_t> starts(n);
     for (uint32_t k = 0; k < n; ++k) starts[k] = jobs[k].wg_start;
-    return upload_table(this, sc->pjobs_dev, sc->pjobs_host, sc->pjobs_cap, sc->upload_done, jobs, starts.data(), n,
+    return upload_table(this, sc->pjobs_dev, sc->pjobs_host, sc->pjobs_cap, sc->pjobs_copied, sc->pjobs_copied, jobs,
+                        starts.data(), n,
                         st, "pyramid job table upload");
 }
 
@@ -1288,11 +1288,11 @@ bz_status bz_cull_batch(bz_ctx* ctx, const bz_view_job* jobs, uint32_t n_jobs, v
     StreamScratch* sc = nullptr;
     s = ctx->scratch_for(st, tiles, (uint64_t)tiles * t.block * t.items, &sc);
     if (s) return s;
-    s = ctx->upload_jobs(sc, cj.data(), (uint32_t)cj.size(), st);
+    if (cj.size() > kArgFullJobs) s = ctx->upload_jobs(sc, cj.data(), (uint32_t)cj.size(), st);
     if (s) return s;
-    e = launch_cull_batch(cj.data(), sc->jobs_dev, table_starts(sc->jobs_dev, sc->jobs_cap), (uint32_t)cj.size(),
-                          tiles, max_job_tiles(cj.data(), cj.size()), sc->cs, t.block, t.items, st);
-    if (e == hipSuccess) e = hipEventRecord(sc->upload_done, st);
+    e = launch_cull_batch(cj.data(), sc->jobs_dev, table_starts(sc->jobs_dev, (uint32_t)cj.size()),
+                          (uint32_t)cj.size(), tiles, max_job_tiles(cj.data(), cj.size()), sc->cs, t.block, t.items,
+                          st);
     if (e != hipSuccess) return ctx->hip_fail(e, "batched cull launch");
     return BZ_OK;
 }
@@ -1396,14 +1396,14 @@ bz_status bz_batch_graph_create(bz_ctx* ctx, const bz_pyramid_job* pyr_jobs, uin
     // graph-owned device state
     hipError_t e = hipSuccess;
     const uint32_t cap = std::max<uint32_t>(tiles, 1u);
-    e = hipMalloc((void**)&g->cs.counts, (size_t)counts_words(cap) * 4);
+    e = hipMalloc((void**)&g->cs.counts, (size_t)batch_words(cap) * 4);
     if (e == hipSuccess) e = hipMalloc((void**)&g->cs.staging, (size_t)cap * t.block * t.items * sizeof(uint2));
     if (e == hipSuccess) e = hipMalloc((void**)&g->err, 16);
     if (e == hipSuccess) e = hipMemset(g->err, 0, 16);
     if (e != hipSuccess) return ctx->hip_fail(e, "graph scratch");
     g->cs.capacity_tiles = cap;
     g->cs.capacity_entries = (uint64_t)cap * t.block * t.items;
-    set_prefix(g->cs);
+    set_prefix(g->cs, true);
     // job tables (descriptors, then the compact start indices), owned by the graph
     if (!cj.empty()) {
         std::vector<uint32_t> starts(cj.size());
@@ -1429,12 +1429,7 @@ bz_status bz_batch_graph_create(bz_ctx* ctx, const bz_pyramid_job* pyr_jobs, uin
     e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
     if (e != hipSuccess) return ctx->hip_fail(e, "capture stream");
     e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess && !pj.empty())
-    {
-        uint32_t mt = 0;
-        for (auto& q : pj) mt = std::max<uint32_t>(mt, q.tiles_x * q.tiles_y);
-        e = launch_pyramid_batch(g->pjobs_dev, (uint32_t)pj.size(), mt, g->err + 1, cs);
-    }
+    if (e == hipSuccess) e = launch_pyramid_batch(pj.data(), g->pjobs_dev, (uint32_t)pj.size(), g->err + 1, cs);
     for (auto& m : multi) {
         if (e != hipSuccess) break;
         e = m.first->launch_other(m.second.depth_dev, m.second.w, m.second.h, ctx->wait_limit, g->err + 1, cs);

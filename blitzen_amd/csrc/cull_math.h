@@ -40,8 +40,7 @@ struct ViewConsts {
 // Device view of one depth pyramid.
 struct PyramidDesc {
     const float* texels;
-    uint32_t base_w, base_h, mips, pad;
-    uint32_t level_offset[16];
+    uint32_t base_w, base_h, mips, pad;  // (the kernels compute the levels' offsets from the extent)
 };
 
 // a * b + c with one rounding

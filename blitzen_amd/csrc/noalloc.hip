@@ -68,6 +68,6 @@ extern "C" bz_status bz_cull_noalloc(bz_ctx* ctx, const bz_cull_args* a, void* s
     fixed.staging = reinterpret_cast<uint2*>(base + kNoAllocCountsBytes);
     fixed.capacity_tiles = kNoAllocTiles;
     fixed.capacity_entries = kNoAllocEntries;
-    set_prefix(fixed);
+    set_prefix(fixed, false);
     return ctx->cull(a, (hipStream_t)stream, &fixed);
 }

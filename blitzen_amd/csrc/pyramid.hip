@@ -83,7 +83,7 @@ struct PyrSmem {
 // with its levels 10.8, the whole build 14.5; now 12.4. 1920 x 1080 onto 1024 x 1024: 8.9 -> 8.2; 64 pyramids of the batch
 // with exact 2:1: 85 -> 78 us). Lanes in Morton order, which need no LDS up to level 4, store level 0 in 64-byte pieces:
 // level 0 alone 10.5 us. Four texels a lane and 256 threads: 11.5, but 8.2 instead of 6.6 us for 1024 x 512.
-__device__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile, PyrSmem& sm, uint32_t* err)
+__device__ __forceinline__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile, PyrSmem& sm, uint32_t* err)
 {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t tx = tile % J.tiles_x, ty = tile / J.tiles_x, bw = J.base_w, bh = J.base_h;
@@ -250,6 +250,15 @@ __global__ __launch_bounds__(kPyrBlock) void pyramid_batch_kernel(const PyrBuild
 {
     __shared__ PyrSmem sm;
     const PyrBuildJob& J = jobs[blockIdx.y];
+    if (blockIdx.x >= J.tiles_x * J.tiles_y) return;
+    pyramid_tile(J, blockIdx.x, sm, err);
+}
+
+// The same for a few jobs, which come in the kernel arguments.
+__global__ __launch_bounds__(kPyrBlock) void pyramid_few_kernel(PyrArgs jobs, uint32_t* err)
+{
+    __shared__ PyrSmem sm;
+    const PyrBuildJob& J = jobs.j[blockIdx.y];
     if (blockIdx.x >= J.tiles_x * J.tiles_y) return;
     pyramid_tile(J, blockIdx.x, sm, err);
 }
@@ -421,7 +430,7 @@ constexpr uint32_t kMaxRects = kSynthMaxRects;
 constexpr uint32_t kRectChunk = 512;
 constexpr uint32_t kRasterPix = kRasterTile * kRasterTile / 256;
 
-__device__ void synth_depth_tile(uint64_t seed, uint32_t W, uint32_t H, uint32_t n_rects, float p11, float znear,
+__device__ __forceinline__ void synth_depth_tile(uint64_t seed, uint32_t W, uint32_t H, uint32_t n_rects, float p11, float znear,
                                  float* __restrict__ depth, uint32_t bx, uint32_t by, int4* s_rect, float* s_depth,
                                  uint32_t* s_n)
 {
@@ -509,10 +518,21 @@ hipError_t launch_pyramid(const PyrBuildJob& job, uint32_t* err, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_dev, uint32_t n_jobs, uint32_t max_tiles, uint32_t* err,
-                                hipStream_t st)
+hipError_t launch_pyramid_batch(const PyrBuildJob* jobs_host, const PyrBuildJob* jobs_dev, uint32_t n_jobs,
+                                uint32_t* err, hipStream_t st)
 {
-    if (n_jobs == 0 || max_tiles == 0) return hipSuccess;
+    if (n_jobs == 0) return hipSuccess;
+    uint32_t max_tiles = 1;
+    for (uint32_t k = 0; k < n_jobs; ++k) {
+        const uint32_t t = jobs_host[k].tiles_x * jobs_host[k].tiles_y;
+        max_tiles = t > max_tiles ? t : max_tiles;
+    }
+    if (n_jobs <= kArgPyrJobs) {
+        PyrArgs a;
+        for (uint32_t k = 0; k < kArgPyrJobs; ++k) a.j[k] = jobs_host[k < n_jobs ? k : 0u];
+        hipLaunchKernelGGL(pyramid_few_kernel, dim3(max_tiles, n_jobs), dim3(kPyrBlock), 0, st, a, err);
+        return hipGetLastError();
+    }
     constexpr uint32_t kMaxGridY = 65535;  // jobs per launch (the grid's y extent); more go in further launches
     for (uint32_t j0 = 0; j0 < n_jobs; j0 += kMaxGridY) {
         const uint32_t n = n_jobs - j0 < kMaxGridY ? n_jobs - j0 : kMaxGridY;

@@ -99,11 +99,11 @@ bz_status HipDevice::init(const bz_server_cfg& cfg)
         s.err = s.counts_dev + cfg.max_batch_requests;
         const uint64_t tiles = kBatchObjects / 256 + cfg.max_batch_requests;  // smallest tile: 256 objects
         const uint64_t entries = kBatchObjects + (uint64_t)cfg.max_batch_requests * 2048;
-        if (e == hipSuccess) e = hipMalloc((void**)&s.cs.counts, (size_t)counts_words((uint32_t)tiles) * 4);
+        if (e == hipSuccess) e = hipMalloc((void**)&s.cs.counts, (size_t)batch_words(tiles) * 4);
         if (e == hipSuccess) e = hipMalloc((void**)&s.cs.staging, (size_t)entries * sizeof(uint2));
         s.cs.capacity_tiles = (uint32_t)tiles;
         s.cs.capacity_entries = entries;
-        set_prefix(s.cs);
+        set_prefix(s.cs, true);
         if (e != hipSuccess) return ctx->hip_fail(e, "server slot");
     }
     e = hipStreamCreateWithFlags(&fetch_st, hipStreamNonBlocking);
@@ -213,33 +213,28 @@ bz_status HipDevice::launch(uint32_t slot, const std::vector<ReqP>& batch)
         s.cs = CompactScratch{};
         const uint32_t ct = std::max<uint32_t>(tiles, 1u << 12);
         const uint64_t ce = std::max<uint64_t>((uint64_t)tiles * tile, 1ull << 20);
-        e = hipMalloc((void**)&s.cs.counts, (size_t)counts_words(ct) * 4);
+        e = hipMalloc((void**)&s.cs.counts, (size_t)batch_words(ct) * 4);
         if (e == hipSuccess) e = hipMalloc((void**)&s.cs.staging, (size_t)ce * sizeof(uint2));
         if (e != hipSuccess) return ctx->hip_fail(e, "server compaction scratch");
         s.cs.capacity_tiles = ct;
         s.cs.capacity_entries = ce;
-        set_prefix(s.cs);
+        set_prefix(s.cs, true);
     }
-    bz_status st = upload_table(ctx, s.sjobs_dev, s.sjobs_host, s.sjobs_cap, s.done, sj.data(), sstart.data(), B,
+    bz_status st = upload_table(ctx, s.sjobs_dev, s.sjobs_host, s.sjobs_cap, s.done, nullptr, sj.data(), sstart.data(), B,
                                 s.st, "server raster jobs");
-    if (!st && !pj.empty())
-        st = upload_table(ctx, s.pjobs_dev, s.pjobs_host, s.pjobs_cap, s.done, pj.data(), pstart.data(),
+    if (!st && pj.size() > kArgPyrJobs)
+        st = upload_table(ctx, s.pjobs_dev, s.pjobs_host, s.pjobs_cap, s.done, nullptr, pj.data(), pstart.data(),
                           (uint32_t)pj.size(), s.st, "server pyramid jobs");
-    if (!st && !cj.empty())
-        st = upload_table(ctx, s.jobs_dev, s.jobs_host, s.jobs_cap, s.done, cj.data(), cstart.data(),
+    if (!st && cj.size() > kArgFullJobs)
+        st = upload_table(ctx, s.jobs_dev, s.jobs_host, s.jobs_cap, s.done, nullptr, cj.data(), cstart.data(),
                           (uint32_t)cj.size(), s.st, "server cull jobs");
     if (st) return st;
     e = launch_fill_u32(s.counts_dev, 0u, B, s.st);
     if (e == hipSuccess)
-        e = launch_synth_depth_batch(s.sjobs_dev, table_starts(s.sjobs_dev, s.sjobs_cap), B, swg, s.st);
-    if (e == hipSuccess && !pj.empty())
-    {
-        uint32_t mt = 0;
-        for (auto& q : pj) mt = std::max<uint32_t>(mt, q.tiles_x * q.tiles_y);
-        e = launch_pyramid_batch(s.pjobs_dev, (uint32_t)pj.size(), mt, s.err + 1, s.st);
-    }
+        e = launch_synth_depth_batch(s.sjobs_dev, table_starts(s.sjobs_dev, B), B, swg, s.st);
+    if (e == hipSuccess) e = launch_pyramid_batch(pj.data(), s.pjobs_dev, (uint32_t)pj.size(), s.err + 1, s.st);
     if (e == hipSuccess && !cj.empty())
-        e = launch_cull_batch(cj.data(), s.jobs_dev, table_starts(s.jobs_dev, s.jobs_cap), (uint32_t)cj.size(),
+        e = launch_cull_batch(cj.data(), s.jobs_dev, table_starts(s.jobs_dev, (uint32_t)cj.size()), (uint32_t)cj.size(),
                               tiles, max_job_tiles(cj.data(), cj.size()), s.cs, t.block, t.items, s.st);
     if (e == hipSuccess)
         e = hipMemcpyAsync(s.counts_host, s.counts_dev, (size_t)B * 4, hipMemcpyDeviceToHost, s.st);

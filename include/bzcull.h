@@ -368,8 +368,8 @@ typedef struct bz_tuning {
 
 /* Culls every job in one launch pair (decide + emit over the jobs' concatenated tiles). Each job's output
  * equals what bz_cull gives for it alone. Jobs with no objects only get their count zeroed. The job table
- * is staged through a context-owned pinned buffer, so this call cannot be stream-captured: capture a fixed
- * batch with bz_batch_graph_create instead. Jobs that write one visibility buffer in overlapping ranges race. */
+ * of more than a dozen jobs is staged through a context-owned pinned buffer, so this call cannot be stream-captured:
+ * capture a fixed batch with bz_batch_graph_create instead. Jobs that write one visibility buffer in overlapping ranges race. */
 BZ_API bz_status bz_cull_batch(bz_ctx* ctx, const bz_view_job* jobs, uint32_t n_jobs, void* stream);
 /* Synchronizes `stream` and reports BZ_E_INTERNAL if a kernel launched on it gave up a bounded wait
  * since the last check (the flag is then cleared). A pyramid build whose tail workgroup gave up waiting for a
