@@ -602,7 +602,7 @@ def main():
                 "kernel": ("C1 frame: pyramid_kernel + decide_kernel (EARLY) + emit_kernel + decide_kernel (LATE) + "
                            "emit_kernel" if args.no_frame_cache else
                            "C1 frame: pyramid_kernel + decide_kernel (EARLY, frame cache) + emit_kernel + "
-                           "late_cached_kernel + emit_kernel"),
+                           "late_tile_kernel + emit_kernel"),
                 "algorithmic_bytes": frame_bytes, "avg_us": round(frame_ms * 1e3, 2)}
     if traffic and not traffic_ok and not args.no_frame_cache:  # measured on other kernels: reported, not used
         roofline["traffic_stale"] = {"bytes_per_launch": traffic.get("bytes_per_launch"),

@@ -99,7 +99,8 @@ struct Pyramid : PyrPlan {
 
 struct StreamScratch {
     CompactScratch cs{};
-    uint32_t* err = nullptr;          // [0] instanced scan wait gave up, [1] pyramid tail wait gave up, [2] staged transform id out of range
+    unsigned long long* fuse = nullptr;  // [kFuseWords] the one-launch passes' published counts
+    uint32_t* err = nullptr;          // [0] instanced scan or one-launch pass wait gave up, [1] pyramid tail wait gave up, [2] staged transform id out of range
     CullJob* jobs_dev = nullptr;
     CullJob* jobs_host = nullptr;     // pinned
     uint32_t jobs_cap = 0;
@@ -164,6 +165,8 @@ struct Ctx {
     bz_tuning tune[2] = {};
     // The tuning of one single-view pass over n objects: tune[0], or where that is the built-in one, the choice by n.
     bz_tuning pass_tuning(uint32_t n) const;
+    bool built_in_tuning() const;
+    bool one_launch(uint32_t n) const;  // such a pass goes in one launch (launch_fused)
     std::unique_ptr<Server> server;
     void* noalloc_scratch = nullptr;  // device address of this device's fixed scratch (bz_cull_noalloc)
 

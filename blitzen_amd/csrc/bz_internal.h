@@ -125,6 +125,18 @@ struct FrameCacheDev {
 // survivors there.
 hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t block, uint32_t items, uint32_t n_cu,
                        uint32_t per_cu, hipStream_t st, const FrameCacheDev* cache = nullptr);
+// One launch for the whole pass over at most kFuseObjects objects, tiles of kFuseBlock x kFuseItems: each workgroup adds
+// up the counts that the tiles before it publish, instead of an emit launch. That trades a launch (about 2 us, and as long
+// on the host) for a wait on the slowest earlier tile, which grows with the tiles: PLAIN of 131 072 objects 9.3 -> 6.9 us,
+// of 330 000 10.5 -> 8.7; EARLY + pyramid + LATE of 1000 objects 20 -> 15.7, of 262 144 27.5 -> 26.0, of 330 000 in region
+// order 28.4 -> 28.6, of 380 000 28.6 -> 29.5: the line is 640 tiles. `words` holds kFuseWords 64-bit words that are zero
+// before the first launch and kept between launches; launches on one array are ordered. err: set when a wait gives up.
+constexpr uint32_t kFuseBlock = 256, kFuseItems = 2;
+constexpr uint32_t kFuseObjects = 5u << 16;
+constexpr uint32_t kFuseFirst = 16;  // (a cache line for the launch number)
+constexpr uint32_t kFuseWords = kFuseFirst + kFuseObjects / (kFuseBlock * kFuseItems);
+hipError_t launch_fused(const CullJob& job, unsigned long long* words, uint32_t* err, hipStream_t st,
+                        const FrameCacheDev* cache = nullptr);
 // Chunks of consecutive tiles: chunk c of a job holds tiles [t0, t1), the first n_long chunks tpc + 1 tiles and the
 // others tpc (so that as many chunks as workgroups fit at once take the whole job evenly).
 __host__ __device__ inline void chunk_range(uint32_t c, uint32_t tpc, uint32_t n_long, uint32_t n_tiles, uint32_t& t0,
@@ -178,13 +190,12 @@ hipError_t launch_instanced(const InstancedJob& job, const CompactScratch& s, ui
 void decide_inst_chunks(const CullJob& job, uint32_t block, uint32_t items, uint32_t n_cu, uint32_t per_cu,
                         uint32_t* tiles_per_chunk, uint32_t* n_long, uint32_t* n_chunks);
 
-// LATE pass from a frame cache recorded with the same tile size (block x items) over the same range. It runs over
-// super-tiles of kSuperTile objects and needs late_cached_tiles(n) counts and late_cached_entries(n) staging slots.
-constexpr uint32_t kSuperTile = 4096;
-inline uint32_t late_cached_tiles(uint32_t n) { return (uint32_t)(((uint64_t)n + kSuperTile - 1) / kSuperTile); }
-inline uint64_t late_cached_entries(uint32_t n) { return (uint64_t)late_cached_tiles(n) * kSuperTile; }
-hipError_t launch_late_cached(const CullJob& job, const CompactScratch& s, const FrameCacheDev& cache, uint32_t block,
-                              uint32_t items, hipStream_t st);
+// LATE pass from a frame cache recorded over the same range in tiles of `rec` objects (512, 1024 or 2048; job.n_tiles of
+// them): with an emit launch, or in one launch (a cache recorded by launch_fused; words, err: as there).
+hipError_t launch_late_cached(const CullJob& job, const CompactScratch& s, const FrameCacheDev& cache, uint32_t rec,
+                              hipStream_t st);
+hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, unsigned long long* words, uint32_t* err,
+                             hipStream_t st);
 // The first tiles of up to kArgJobs jobs, passed to the batched decide as a kernel argument (2 KiB of the 4 KiB
 // kernarg segment).
 constexpr uint32_t kArgJobs = 512;

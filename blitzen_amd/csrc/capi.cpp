@@ -97,7 +97,7 @@ uint64_t PyrPlan::tail_words() const
 
 StreamScratch::~StreamScratch()
 {
-    void* ps[] = { cs.counts, cs.staging, jobs_dev, pjobs_dev, err, xs.ccounts, xs.rbase, xs.scount, xs.sprefix,
+    void* ps[] = { cs.counts, cs.staging, jobs_dev, pjobs_dev, err, fuse, xs.ccounts, xs.rbase, xs.scount, xs.sprefix,
                    xs.survivors, inst_hist, inst_seg };
     for (void* p : ps)
         if (p) (void)hipFree(p);
@@ -115,10 +115,18 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
     if (!slot) slot.reset(new StreamScratch());
     StreamScratch& s = *slot;
     if (!s.err) {
-        hipError_t e = hipMalloc((void**)&s.err, 16);
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc(error flags)");
-        e = hipMemset(s.err, 0, 16);
-        if (e != hipSuccess) return hip_fail(e, "hipMemset(error flags)");
+        hipError_t e = hipMalloc((void**)&s.fuse, kFuseWords * 8u);
+        if (e == hipSuccess) e = hipMemset(s.fuse, 0, kFuseWords * 8u);
+        if (e == hipSuccess) e = hipMalloc((void**)&s.err, 16);
+        if (e == hipSuccess) e = hipMemset(s.err, 0, 16);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // cleared before a launch on any stream
+        if (e != hipSuccess) {
+            for (void* p : { (void*)s.fuse, (void*)s.err })
+                if (p) (void)hipFree(p);
+            s.fuse = nullptr;
+            s.err = nullptr;
+            return hip_fail(e, "stream words");
+        }
         e = hipEventCreateWithFlags(&s.jobs_copied, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&s.pjobs_copied, hipEventDisableTiming);
         if (e != hipSuccess) return hip_fail(e, "hipEventCreate");
@@ -266,17 +274,25 @@ uint32_t tiles_for(uint32_t n, uint32_t block, uint32_t items)
 
 constexpr bz_tuning kBuiltInTuning{ 512, 2, 0, 0 };
 
-// Up to 2^19 objects a pass is a few rounds of dependent latencies: tiles of 512 objects give every CU two workgroups or
-// more (65 536 objects, EARLY + pyramid + LATE: 27.8 us against 29.4 us with 1024-object tiles of 512 threads; 262 161:
-// 28.2 against 28.8; 500 009 TEMPORAL: 34.3 against 34.3-38). Above it the streams bound it and four objects a thread
-// are better: a wave's compacted LOD selection then runs on twice the lanes (1 048 576: 40.1 against 41.9 us; 4 194 304
-// with the frame cache: 59.2 against 62.1; PLAIN of 16 777 216: 83.1 against 84.3).
+// Two objects a thread up to 2^21 objects, four above. Four are better where the streams bound the pass and the objects
+// in view are spread over all tiles: a wave's compacted LOD selection then runs on twice the lanes (4 194 304 objects at
+// random with the frame cache 59.2 against 62.8 us, PLAIN of 16 777 216 83.1 against 92.5; 2 000 000 only 41.8 against 42.8).
+// Where neighbouring ids are neighbours in space, a tile is all in view or not at all, and a wave works through its
+// survivors 64 at a time: half as many per wave spread them better (2 000 000 in region order 41.7 against 49.9 us, 1 048 576
+// 34.0 against 38.7, 600 000 30.7 against 34.3).
+bool Ctx::built_in_tuning() const
+{
+    const bz_tuning &t = tune[0], &d = kBuiltInTuning;
+    return t.block == d.block && t.items == d.items && t.grid_per_cu == d.grid_per_cu;
+}
+
+bool Ctx::one_launch(uint32_t n) const { return n <= kFuseObjects && built_in_tuning(); }
+
 bz_tuning Ctx::pass_tuning(uint32_t n) const
 {
-    const bz_tuning& t = tune[0];
-    const bz_tuning& d = kBuiltInTuning;
-    if (t.block != d.block || t.items != d.items || t.grid_per_cu != d.grid_per_cu) return t;
-    return n <= (1u << 19) ? bz_tuning{ 256, 2, 0, 0 } : bz_tuning{ 256, 4, 0, 0 };
+    if (!built_in_tuning()) return tune[0];
+    if (one_launch(n)) return bz_tuning{ kFuseBlock, kFuseItems, 0, 0 };
+    return n <= (1u << 21) ? bz_tuning{ 256, 2, 0, 0 } : bz_tuning{ 256, 4, 0, 0 };
 }
 
 // Validates one view's cull and fills a CullJob (without tile_start).
@@ -977,18 +993,34 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
         // the EARLY pass of this view recorded the frustum survivors: read those (and the current visibility)
         // instead of every transform
         job.n_tiles = tiles_for(job.n, fc.block, fc.items);
-        s = compact(late_cached_tiles(job.n), late_cached_entries(job.n), &cs);
-        if (s) return s;
         const FrameCacheDev d{ fc.sph, fc.meta, fc.counts };
-        hipError_t e = launch_late_cached(job, cs, d, fc.block, fc.items, st);
+        hipError_t e = hipSuccess;
+        if (!fixed && one_launch(job.n) && fc.block * fc.items == kFuseBlock * kFuseItems) {
+            StreamScratch* sc = nullptr;
+            s = scratch_for(st, 0, 0, &sc);
+            if (s) return s;
+            e = launch_late_fused(job, d, sc->fuse, sc->err, st);
+        } else {
+            s = compact(job.n_tiles, (uint64_t)job.n_tiles * fc.block * fc.items, &cs);
+            if (s) return s;
+            e = launch_late_cached(job, cs, d, fc.block * fc.items, st);
+        }
         if (e != hipSuccess) return hip_fail(e, "cached late-pass launch");
         ++fc.reused;
         return BZ_OK;
     }
-    s = compact(job.n_tiles, (uint64_t)job.n_tiles * t.block * t.items, &cs);
+    // few objects under the built-in tuning: the whole pass in one launch, with no compaction scratch
+    StreamScratch* fuse = nullptr;
+    if (!fixed && one_launch(job.n)) s = scratch_for(st, 0, 0, &fuse);
+    else s = compact(job.n_tiles, (uint64_t)job.n_tiles * t.block * t.items, &cs);
     if (s) return s;
+    auto launch = [&](const FrameCacheDev* d) {
+        return fuse ? launch_fused(job, fuse->fuse, fuse->err, st, d)
+                    : launch_cull(job, cs, t.block, t.items, n_cu, t.grid_per_cu, st, d);
+    };
     if (cache && job.pass == PASS_EARLY) {
         const uint64_t entries = (uint64_t)job.n_tiles * t.block * t.items;
+        const uint32_t cap_tiles = (uint32_t)(entries / 512u);  // in the smallest tiles: a part of the range may use them
         if (fc.cap_entries < entries || fc.cap_tiles < job.n_tiles) {
             if (fixed)
                 return fail(BZ_E_STATE, "the scene's frame cache is not allocated for this range: run one bz_cull "
@@ -1003,13 +1035,13 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
             fc.cap_tiles = 0;
             if (e == hipSuccess) e = hipMalloc((void**)&fc.sph, (size_t)entries * sizeof(float4));
             if (e == hipSuccess) e = hipMalloc((void**)&fc.meta, (size_t)entries * sizeof(uint2));
-            if (e == hipSuccess) e = hipMalloc((void**)&fc.counts, (size_t)job.n_tiles * 4);
+            if (e == hipSuccess) e = hipMalloc((void**)&fc.counts, (size_t)cap_tiles * 4);
             if (e != hipSuccess) {
                 fc.valid = false;
                 return hip_fail(e, "frame cache allocation");
             }
             fc.cap_entries = entries;
-            fc.cap_tiles = job.n_tiles;
+            fc.cap_tiles = cap_tiles;
         }
         fc.valid = true;
         std::memcpy(fc.view_key, key, sizeof key);
@@ -1019,7 +1051,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
         fc.items = t.items;
         fc.xf_version = scn->xf_version;
         const FrameCacheDev d{ fc.sph, fc.meta, fc.counts };
-        hipError_t e = launch_cull(job, cs, t.block, t.items, n_cu, t.grid_per_cu, st, &d);
+        hipError_t e = launch(&d);
         if (e != hipSuccess) {
             fc.valid = false;
             return hip_fail(e, "cull launch");
@@ -1027,7 +1059,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
         ++fc.recorded;
         return BZ_OK;
     }
-    hipError_t e = launch_cull(job, cs, t.block, t.items, n_cu, t.grid_per_cu, st);
+    hipError_t e = launch(nullptr);
     if (e != hipSuccess) return hip_fail(e, "cull launch");
     return BZ_OK;
 }
@@ -1335,6 +1367,14 @@ bz_status bz_check(bz_ctx* ctx, void* stream)
     for (auto& g : ctx->graphs)
         if (e == hipSuccess && g.second->launched && g.second->last_stream == st) e = read_flags(g.second->err);
     if (e != hipSuccess) return ctx->hip_fail(e, "error flag read");
+    if (flags[0]) {
+        // A workgroup of a one-launch pass that gave up may have published its count under a later launch's number
+        e = hipDeviceSynchronize();
+        for (auto& x : ctx->scratch)
+            if (e == hipSuccess && x.second->fuse) e = hipMemset(x.second->fuse, 0, kFuseWords * 8u);
+        if (e == hipSuccess) e = hipDeviceSynchronize();
+        if (e != hipSuccess) return ctx->hip_fail(e, "one-launch words reset");
+    }
     if (flags[1]) {
         // A tail workgroup that gave up may have missed hand-off words that tiles stored after it looked: clear every
         // pyramid's words (with the device idle, so no build is in flight) for the next builds to start from zero.

@@ -209,6 +209,76 @@ __device__ __forceinline__ void stage_tables(const CullJob& J, TileSmem<BLOCK, I
     }
 }
 
+__device__ __forceinline__ void write_command(uint32_t* cmds, uint32_t pos, uint32_t object, uint2 draw)
+{
+    uint2* cmd = reinterpret_cast<uint2*>(cmds + (size_t)pos * 6u);
+    cmd[0] = make_uint2(object, draw.x);  // objectId, indexCount
+    cmd[1] = make_uint2(1u, draw.y);       // instanceCount, firstIndex
+    cmd[2] = make_uint2(0u, 0u);           // vertexOffset, firstInstance
+}
+
+// The word another workgroup publishes for a tile in one launch: the tile's command count with the launch's number above
+// it. A word of another launch is not taken, so nothing is cleared between launches.
+struct FuseDev {
+    unsigned long long* words;  // [0] number of the last launch, [kFuseFirst + tile] the tiles' words
+    uint32_t* err;              // set when a wait gives up
+};
+
+// Commands of the tiles before `tile`, by the whole workgroup (red: BLOCK / 64 LDS words; one barrier). Every word of a
+// thread is loaded before its first wait; a tile only waits on workgroups dispatched before it.
+template <uint32_t BLOCK>
+__device__ __forceinline__ uint32_t fuse_prefix(const FuseDev& fuse, uint32_t launch, uint32_t tile, uint32_t* red)
+{
+    constexpr uint32_t KW = 4;
+    const uint32_t tid = threadIdx.x;
+    uint32_t part = 0;
+    for (uint32_t u0 = 0; u0 < tile; u0 += KW * BLOCK) {
+        unsigned long long w[KW];
+#pragma unroll
+        for (uint32_t k = 0; k < KW; ++k) {
+            const uint32_t u = u0 + k * BLOCK + tid;
+            w[k] = u < tile ? __hip_atomic_load(&fuse.words[kFuseFirst + u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                            : (unsigned long long)launch << 32;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < KW; ++k) {
+            uint32_t spins = 0;
+            while ((uint32_t)(w[k] >> 32) != launch) {
+                if (++spins > BZ_DEFAULT_WAIT_LIMIT) {
+                    atomicExch(fuse.err, 1u);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+                w[k] = __hip_atomic_load(&fuse.words[kFuseFirst + u0 + k * BLOCK + tid], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+            }
+            part += (uint32_t)w[k];
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+    if ((tid & 63u) == 0) red[tid >> 6] = part;
+    __syncthreads();
+    uint32_t prefix = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < BLOCK / 64u; ++w) prefix += red[w];
+    return prefix;
+}
+__device__ __forceinline__ uint32_t fuse_launch(const FuseDev& fuse)  // this launch's number
+{
+    return (uint32_t)__hip_atomic_load(&fuse.words[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+}
+__device__ __forceinline__ void fuse_publish(const FuseDev& fuse, uint32_t launch, uint32_t tile, uint32_t count)
+{
+    __hip_atomic_store(&fuse.words[kFuseFirst + tile], (unsigned long long)launch << 32 | count, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+// By the last tile, which has had every word: each workgroup has read the launch's number, so it can move on.
+__device__ __forceinline__ void fuse_finish(const FuseDev& fuse, uint32_t launch)
+{
+    __hip_atomic_store(&fuse.words[0], (unsigned long long)launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 struct NoPrefetch {
     __device__ __forceinline__ void operator()() const {}
 };
@@ -219,13 +289,15 @@ struct NoPrefetch {
 // CL (cluster object pass): ccounts[gtile] also receives the sum of the emitting objects' LOD cluster counts.
 // CACHE (EARLY with all streams loaded): every frustum survivor of the tile is recorded in the frame cache `fc`.
 // INST (LOD-instanced output): each emitting object also adds 1 to its LOD's bin of the workgroup's LDS histogram.
+// FUSED (one tile per workgroup): the tile's commands are written here (fuse_emit) and not staged for an emit launch.
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false, bool CACHE = false, bool INST = false,
-          class Prefetch>
+          bool FUSED = false, class Prefetch>
 __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t parity,
                                              const Streams<ITEMS>& s, uint32_t* counts, uint2* staging,
                                              uint32_t* ccounts,
                                              TileSmem<BLOCK, ITEMS, LDS_TAB>& sm, Prefetch&& prefetch,
-                                             FrameCacheDev fc = FrameCacheDev{}, uint32_t* lds_hist = nullptr)
+                                             FrameCacheDev fc = FrameCacheDev{}, uint32_t* lds_hist = nullptr,
+                                             FuseDev fuse = FuseDev{}, uint32_t launch = 0u)
 {
     constexpr bool lds_tab = LDS_TAB;
     constexpr int NW = BLOCK / 64;
@@ -399,7 +471,8 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
         }
     }
     if (tid == 0) {
-        counts[gtile] = total;
+        if constexpr (FUSED) fuse_publish(fuse, launch, gtile, total);
+        else counts[gtile] = total;
         if constexpr (CACHE) fc.counts[gtile] = ctotal;
         if constexpr (CL) {
             uint32_t tot = 0;
@@ -408,10 +481,12 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
             ccounts[gtile] = tot;
         }
     }
-    uint2* stage = staging + (size_t)gtile * TILE + before;
+    if constexpr (!FUSED) {
+        uint2* stage = staging + (size_t)gtile * TILE + before;
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k)
-        if (emit[k]) stage[CACHE ? erank[k] : eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
+        for (int k = 0; k < ITEMS; ++k)
+            if (emit[k]) stage[CACHE ? erank[k] : eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
+    }
     if constexpr (CACHE) {
         const size_t cb = (size_t)gtile * TILE + cbefore;
 #pragma unroll
@@ -420,6 +495,22 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
                 fc.sph[cb + eslot[k]] = make_float4(cx[k], cy[k], cz[k], rad[k]);
                 fc.meta[cb + eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
             }
+    }
+    if constexpr (FUSED) {
+        // the draw data is gathered while the earlier tiles' words arrive
+        uint2 d[ITEMS];
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) d[k] = emit[k] ? S.lod_draw[lod_abs[k]] : make_uint2(0u, 0u);
+        const uint32_t prefix = fuse_prefix<BLOCK>(fuse, launch, gtile, sm.wtot[parity ^ 1u]);
+        if (tid == 0 && gtile + 1u == J.n_tiles) {
+            *J.count = prefix + total;
+            fuse_finish(fuse, launch);
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t pos = prefix + before + (CACHE ? erank[k] : eslot[k]);
+            if (emit[k] && pos < J.capacity) write_command(J.cmds, pos, J.begin + i0 + 64u * k, d[k]);
+        }
     }
 }
 
@@ -495,6 +586,23 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
         uint32_t* row = ih.hist + (size_t)blockIdx.x * ih.n_lods;
         for (uint32_t i = threadIdx.x; i < ih.n_lods; i += BLOCK) row[i] = s_hist[i];
     }
+}
+
+// A pass over few objects in one launch: one tile per workgroup, which also writes the tile's commands. A workgroup's first
+// command follows from the counts that the workgroups before it publish. Every object's streams are loaded at once, in
+// EARLY too (the visibility's round trip costs more than the other objects' bytes here); the tables are read from global
+// memory, as for the batches.
+template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool CACHE>
+__global__ __launch_bounds__(BLOCK) void fused_kernel(CullJob J, FrameCacheDev fc, FuseDev fuse)
+{
+    __shared__ TileSmem<BLOCK, ITEMS, false> sm;
+    const uint32_t launch = fuse_launch(fuse);
+    Streams<ITEMS> s;
+    issue_tile<BLOCK, ITEMS, MODE, true, false>(J, blockIdx.x, s);
+    stage_tables<BLOCK, ITEMS>(J, sm);
+    __syncthreads();
+    process_tile<BLOCK, ITEMS, MODE, HIZ, false, false, CACHE, false, true>(
+        J, blockIdx.x, blockIdx.x, 0u, s, nullptr, nullptr, nullptr, sm, NoPrefetch{}, fc, nullptr, fuse, launch);
 }
 
 // Last entry of the ascending table `starts` that is <= t.
@@ -623,14 +731,6 @@ __device__ __forceinline__ void block_lds_sync()
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-__device__ __forceinline__ void write_command(uint32_t* cmds, uint32_t pos, uint32_t object, uint2 draw)
-{
-    uint2* cmd = reinterpret_cast<uint2*>(cmds + (size_t)pos * 6u);
-    cmd[0] = make_uint2(object, draw.x);  // objectId, indexCount
-    cmd[1] = make_uint2(1u, draw.y);       // instanceCount, firstIndex
-    cmd[2] = make_uint2(0u, 0u);           // vertexOffset, firstInstance
 }
 
 // Writes the commands of tiles [t0, t1) of one job (t1 - t0 <= kEmitTiles; tile_size >= 64 * kEmitUnroll). One round
@@ -818,161 +918,112 @@ hipError_t launch_emit(const CullJob& job, uint32_t tile_size, const CompactScra
 // visible ones read their current visibility (as LateDrawCull.comp.glsl:51 does, so any write to it since the EARLY
 // pass is seen) and, when newly visible, are emitted with their recorded LOD -- the same arithmetic on the same values
 // as the full LATE pass, so the commands, count and visibility are identical.
-constexpr uint32_t kLcBlock = 512;  // threads per workgroup of the cached late pass (kSuperTile objects each)
-
-// A workgroup takes a super-tile of kSuperTile objects (kSuperTile / TILE recorded tiles): the survivors of its
-// tiles with their LOD and the Hi-Z test; the current visibility of the survivors that pass it (gathered after the
-// test: a survivor occluded now is not emitted whatever it was, and a tenth of them pass, so the pass reads a tenth
-// of the words: 17.6 us against 18.4 us when every survivor's word was gathered with its texels); then the
-// visibility of the whole super-tile (coalesced; 0 outside the frustum) and the newly visible survivors' commands in
-// survivor order. No transform, surface or LOD table is read. (A coalesced load of the whole super-tile's visibility
-// instead took 8 more registers per thread, which cost a quarter of the resident workgroups: 25.9 us against 14.6 us
-// per C1 pass.)
-template <int TILE>
-__global__ __launch_bounds__(kLcBlock) void late_cached_kernel(CullJob J, FrameCacheDev fc, uint32_t n_rec_tiles,
-                                                               uint32_t* counts, uint2* staging)
+//
+// One 256-thread workgroup per recorded tile: its survivors in rounds of 256, the first loaded together with the tile's
+// count, each with the Hi-Z test; then the current visibility of the survivors that pass it (gathered after the test: a
+// survivor occluded now is not emitted whatever it was, and a tenth of them pass); then the visibility of the whole tile
+// (coalesced 16-byte stores; 0 outside the frustum) and the newly visible survivors' commands in survivor order. No
+// transform, surface or LOD table is read. Workgroups of 512 threads per 4096 objects, which this replaced, were all
+// resident at once, so that their loads, tests and stores ran in step across the GPU, and a region that is all in view
+// (neighbouring ids, neighbouring objects) was one workgroup's, in four rounds of 1024 (4 194 304 objects at random: frame
+// 58.0 -> 56.9 us; 1 048 576 in region order: 50.2 -> 43.3; 131 072 in region order, one launch: 35.7 -> 24.4).
+constexpr uint32_t kLtBlock = 256;
+template <int TILE, bool FUSED>
+__global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCacheDev fc, uint32_t* counts,
+                                                             uint2* staging, FuseDev fuse)
 {
-    constexpr uint32_t BLOCK = kLcBlock, NW = BLOCK / 64;
-    constexpr uint32_t S = kSuperTile / TILE;            // recorded tiles per super-tile
-    constexpr uint32_t OPT = kSuperTile / BLOCK;         // objects per thread
-    constexpr uint32_t U = 2;                            // survivors per thread in the first round
-    __shared__ uint32_t s_new[kSuperTile / 32];
-    __shared__ uint32_t s_lvl[kMaxMips], s_cnt[S + 1], s_woff[U][NW], s_base;
-    const uint32_t st = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t base = st * kSuperTile;  // first object of the super-tile, relative to the job's range
-    const uint32_t nt = J.n - base < kSuperTile ? J.n - base : kSuperTile;
-    const uint32_t obj0 = J.begin + base;
-    // speculative first round, issued before the counts are known: entries [0, WIN) of every recorded tile, survivor
-    // slot g = k * BLOCK + tid -> (tile g / WIN, entry g % WIN), i.e. ascending objectId
-    constexpr uint32_t WIN = BLOCK * U / S;
-    float4 sp[U];
-    uint2 mt[U];
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-        const uint32_t g = k * BLOCK + tid, rt = st * S + g / WIN;
-        const size_t slot = (size_t)(rt < n_rec_tiles ? rt : 0u) * TILE + g % WIN;
-        sp[k] = fc.sph[slot];
-        mt[k] = fc.meta[slot];
-    }
-    uint32_t cnt = 0;
-    if (tid < S) {
-        const uint32_t t = st * S + tid;
-        cnt = t < n_rec_tiles ? fc.counts[t] : 0u;
-    }
-    if (wave == 0) {  // prefix of the recorded tiles' counts (S <= 8 lanes)
-        uint32_t x = lane < S ? cnt : 0u;
-#pragma unroll
-        for (int off = 1; off < 8; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off, 64);
-            if (lane >= (uint32_t)off) x += y;
-        }
-        if (lane < S) s_cnt[lane + 1] = x;
-        if (lane == 0) s_cnt[0] = 0;
-    }
+    constexpr uint32_t NW = kLtBlock / 64, ROUNDS = TILE / kLtBlock;
+    __shared__ uint32_t s_new[TILE / 32], s_lvl[kMaxMips], s_tot[ROUNDS][NW], s_red[NW];
+    const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t base = t * TILE, nt = J.n - base < TILE ? J.n - base : TILE, obj0 = J.begin + base;
+    const uint32_t launch = FUSED ? fuse_launch(fuse) : 0u;
+    const size_t slot0 = (size_t)t * TILE + tid;
+    float4 sp = fc.sph[slot0];
+    uint2 mt = fc.meta[slot0];
+    const uint32_t n = __builtin_amdgcn_readfirstlane(fc.counts[t]);
     if (tid < (uint32_t)kMaxMips) {
         uint32_t off = 0;
         for (uint32_t L = 0; L < tid; ++L) off += level_dim(J.pyr.base_w, L) * level_dim(J.pyr.base_h, L);
         s_lvl[tid] = off;
     }
-    for (uint32_t x = tid; x < kSuperTile / 32; x += BLOCK) s_new[x] = 0u;
-    if (tid == 0) s_base = 0;
+    if (tid < TILE / 32) s_new[tid] = 0u;
     __syncthreads();
-    const uint32_t total = s_cnt[S];
-    uint2* stage = staging + (size_t)st * kSuperTile;
-    // one round of up to BLOCK x U survivors: Hi-Z test, visibility bits, commands in (k, wave, lane) order after the
-    // earlier rounds
-    auto round = [&](const float4 (&sp)[U], const uint2 (&mt)[U], const bool (&have)[U]) {
-        bool emit[U];
-        uint32_t lod_abs[U];
+    uint32_t before = 0;      // the tile's commands of the rounds so far
+    bool emit[ROUNDS];        // FUSED: a round's commands wait for the tile's first slot
+    uint32_t rank[ROUNDS], obj[ROUNDS];
+    uint2 d[ROUNDS];
 #pragma unroll
-        for (uint32_t k = 0; k < U; ++k) {
-            emit[k] = false;
-            lod_abs[k] = 0u;
-            const uint32_t local = mt[k].x - obj0;
-            if (have[k] && local < nt) {  // (an entry outside the super-tile can only come from a mismatched cache)
+    for (uint32_t r = 0; r < ROUNDS; ++r) {
+        emit[r] = false;
+        rank[r] = obj[r] = 0u;
+        d[r] = make_uint2(0u, 0u);
+        if (r * kLtBlock < n) {  // uniform
+            const uint32_t e = r * kLtBlock + tid;
+            if (r) {
+                sp = fc.sph[slot0 + r * kLtBlock];
+                mt = fc.meta[slot0 + r * kLtBlock];
+            }
+            const uint32_t local = mt.x - obj0;
+            if (e < n && local < nt) {  // (an entry outside the tile can only come from a mismatched cache)
                 float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-                const bool test = project_sphere(sp[k].x, sp[k].y, sp[k].z, sp[k].w, J.view.znear, J.view.p00,
-                                                 J.view.p11, a0, a1, a2, a3);
+                const bool test =
+                    project_sphere(sp.x, sp.y, sp.z, sp.w, J.view.znear, J.view.p00, J.view.p11, a0, a1, a2, a3);
                 // a sphere crossing the near plane is not tested and stays visible
-                const bool vis =
-                    test ? occlusion_visible(J.view, J.pyr, s_lvl, a0, a1, a2, a3, sp[k].z, sp[k].w) : true;
+                const bool vis = test ? occlusion_visible(J.view, J.pyr, s_lvl, a0, a1, a2, a3, sp.z, sp.w) : true;
                 if (vis) atomicOr(&s_new[local >> 5], 1u << (local & 31u));
-                // the current visibility (LateDrawCull:51), read only where it decides: for the visible survivors
-                emit[k] = vis && J.vis_in[mt[k].x] == 0u;
-                lod_abs[k] = mt[k].y;
+                emit[r] = vis && J.vis_in[mt.x] == 0u;  // the current visibility (LateDrawCull:51), where it decides
             }
-        }
-        uint32_t rank[U];
+            const unsigned long long m = __ballot(emit[r]);
+            rank[r] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            obj[r] = mt.x;
+            d[r].x = mt.y;
+            if (lane == 0) s_tot[r][wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t total = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < U; ++k) {
-            const unsigned long long m = __ballot(emit[k]);
-            rank[k] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            if (lane == 0) s_woff[k][wave] = (uint32_t)__popcll(m);
+            for (uint32_t w = 0; w < NW; ++w) {
+                const uint32_t x = s_tot[r][w];
+                rank[r] += w < wave ? x : 0u;
+                total += x;
+            }
+            rank[r] += before;
+            before += total;
+            if constexpr (!FUSED)
+                if (emit[r]) staging[(size_t)t * TILE + rank[r]] = make_uint2(obj[r], d[r].x);
         }
-        __syncthreads();
-        if (wave == 0) {
-            constexpr uint32_t E = U * NW;
-            const uint32_t c = lane < E ? (&s_woff[0][0])[lane] : 0u;
-            const uint32_t incl = wave_incl_scan(c, lane);
-            if (lane < E) (&s_woff[0][0])[lane] = s_base + incl - c;
-            if (lane == 63) s_base += incl;
+    }
+    if (n == 0) __syncthreads();  // (s_new cleared; with survivors a round's barrier has followed its last bit)
+    if (tid == 0) {
+        if constexpr (FUSED) fuse_publish(fuse, launch, t, before);
+        else counts[t] = before;
+    }
+    // the visibility is next read by the following frame's EARLY pass: stored non-temporal
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    if (nt == TILE && ((uintptr_t)(J.vis_out + obj0) & 15u) == 0) {
+        for (uint32_t i = tid; i < TILE / 4u; i += kLtBlock) {
+            const uint32_t b = s_new[i >> 3] >> ((i & 7u) * 4u);
+            const u32x4 v = { b & 1u, (b >> 1) & 1u, (b >> 2) & 1u, (b >> 3) & 1u };
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(J.vis_out + obj0) + i);
         }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < U; ++k)
-            if (emit[k]) stage[s_woff[k][wave] + rank[k]] = make_uint2(mt[k].x, lod_abs[k]);
-        __syncthreads();  // s_woff is rewritten by the next round
-    };
-    bool fast = true;  // every recorded tile's survivors fit its window: the speculative round is the whole pass
-#pragma unroll
-    for (uint32_t q = 0; q < S; ++q) fast = fast && s_cnt[q + 1] - s_cnt[q] <= WIN;
-    if (fast) {
-        bool have[U];
-#pragma unroll
-        for (uint32_t k = 0; k < U; ++k) {
-            const uint32_t g = k * BLOCK + tid, j = g / WIN;
-            have[k] = g % WIN < s_cnt[j + 1] - s_cnt[j];
-        }
-        round(sp, mt, have);
     } else {
-        // survivors in rounds of BLOCK x U; g = k * BLOCK + tid is the survivor's rank in the super-tile
-        for (uint32_t g0 = 0; g0 < total; g0 += BLOCK * U) {
-            float4 sp2[U];
-            uint2 mt2[U];
-            bool have[U];
+        for (uint32_t i = tid; i < nt; i += kLtBlock)
+            __builtin_nontemporal_store((s_new[i >> 5] >> (i & 31u)) & 1u, J.vis_out + obj0 + i);
+    }
+    if constexpr (FUSED) {
 #pragma unroll
-            for (uint32_t k = 0; k < U; ++k) {
-                const uint32_t g = g0 + k * BLOCK + tid;
-                have[k] = g < total;
-                uint32_t j = 0;  // recorded tile holding survivor g
+        for (uint32_t r = 0; r < ROUNDS; ++r)
+            if (emit[r]) d[r] = J.scene.lod_draw[d[r].x];
+        const uint32_t prefix = fuse_prefix<kLtBlock>(fuse, launch, t, s_red);
+        if (tid == 0 && t + 1u == J.n_tiles) {
+            *J.count = prefix + before;
+            fuse_finish(fuse, launch);
+        }
 #pragma unroll
-                for (uint32_t q = 1; q < S; ++q) j += g >= s_cnt[q] ? 1u : 0u;
-                const uint32_t e = have[k] ? g - s_cnt[j] : 0u;
-                const size_t slot = (size_t)(st * S + (have[k] ? j : 0u)) * TILE + e;  // in the cache region
-                sp2[k] = fc.sph[slot];
-                mt2[k] = fc.meta[slot];
-            }
-            round(sp2, mt2, have);
+        for (uint32_t r = 0; r < ROUNDS; ++r) {
+            const uint32_t pos = prefix + rank[r];
+            if (emit[r] && pos < J.capacity) write_command(J.cmds, pos, obj[r], d[r]);
         }
     }
-    // the visibility is next read by the following frame's EARLY pass: stored non-temporal (1 us faster here)
-#pragma unroll
-    for (uint32_t k = 0; k < OPT; ++k) {
-        const uint32_t i = k * BLOCK + tid;
-        if (i < nt) __builtin_nontemporal_store((s_new[i >> 5] >> (i & 31u)) & 1u, J.vis_out + obj0 + i);
-    }
-    if (tid == 0) counts[st] = s_base;
-}
-
-template <int TILE>
-hipError_t launch_late_cached_t(const CullJob& job, const CompactScratch& s, const FrameCacheDev& fc,
-                                uint32_t n_rec_tiles, hipStream_t st)
-{
-    hipLaunchKernelGGL((late_cached_kernel<TILE>), dim3(job.n_tiles), dim3(kLcBlock), 0, st, job, fc, n_rec_tiles,
-                       s.counts, s.staging);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_emit(job, kSuperTile, s, st);
 }
 
 // Persistent grid: `per_cu` workgroups per CU, or (per_cu == 0) as many as are resident at once per CU.
@@ -1058,6 +1109,29 @@ hipError_t launch_cull_t(const CullJob& job, const CompactScratch& s, uint32_t n
     return launch_emit(job, (uint32_t)(BLOCK * ITEMS), s, st);
 }
 
+hipError_t launch_fused_t(const CullJob& job, const FrameCacheDev& fc, bool record, const FuseDev& f, hipStream_t st)
+{
+    const dim3 g(job.n_tiles), b(kFuseBlock);
+#define BZ_FUSED(M, HZ, CA) \
+    hipLaunchKernelGGL((fused_kernel<kFuseBlock, kFuseItems, M, HZ, CA>), g, b, 0, st, job, fc, f)
+    const bool h = job.hiz != 0;
+    if (job.pass == PASS_EARLY && record) {
+        if (h) BZ_FUSED(MODE_EARLY, true, true);
+        else BZ_FUSED(MODE_EARLY, false, true);
+    } else if (job.pass == PASS_EARLY) {
+        if (h) BZ_FUSED(MODE_EARLY, true, false);
+        else BZ_FUSED(MODE_EARLY, false, false);
+    } else if (job.pass == PASS_LATE) {
+        BZ_FUSED(MODE_LATE, true, false);
+    } else if (h) {
+        BZ_FUSED(MODE_OTHER, true, false);
+    } else {
+        BZ_FUSED(MODE_OTHER, false, false);
+    }
+#undef BZ_FUSED
+    return hipGetLastError();
+}
+
 template <int BLOCK, int ITEMS>
 hipError_t launch_cull_batch_t(const CullJob* jobs_host, const CullJob* jobs, const uint32_t* starts, uint32_t n_jobs,
                                uint32_t total_tiles, uint32_t max_job_tiles, const CompactScratch& s, hipStream_t st)
@@ -1111,6 +1185,13 @@ hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t blo
     return hipErrorInvalidValue;
 }
 
+hipError_t launch_fused(const CullJob& job, unsigned long long* words, uint32_t* err, hipStream_t st,
+                        const FrameCacheDev* cache)
+{
+    const FrameCacheDev fc = cache ? *cache : FrameCacheDev{};
+    return launch_fused_t(job, fc, cache != nullptr, FuseDev{ words, err }, st);
+}
+
 hipError_t launch_decide_only(const CullJob& job, const CompactScratch& s, uint32_t block, uint32_t items,
                               uint32_t n_cu, uint32_t per_cu, hipStream_t st, const InstHistDev* ih)
 {
@@ -1148,20 +1229,29 @@ void decide_inst_chunks(const CullJob& job, uint32_t block, uint32_t items, uint
     }
 }
 
-hipError_t launch_late_cached(const CullJob& job_in, const CompactScratch& s, const FrameCacheDev& cache, uint32_t block,
-                              uint32_t items, hipStream_t st)
+hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, unsigned long long* words, uint32_t* err,
+                             hipStream_t st)
 {
-    // the pass runs over super-tiles; the recorded tiles (block x items objects) are what the cache holds
-    CullJob job = job_in;
-    const uint32_t rec = block * items;
-    const uint32_t n_rec_tiles = (job.n + rec - 1) / rec;
-    job.n_tiles = late_cached_tiles(job.n);
+    hipLaunchKernelGGL((late_tile_kernel<kFuseBlock * kFuseItems, true>), dim3(job.n_tiles), dim3(kLtBlock), 0, st, job,
+                       cache, (uint32_t*)nullptr, (uint2*)nullptr, FuseDev{ words, err });
+    return hipGetLastError();
+}
+
+hipError_t launch_late_cached(const CullJob& job, const CompactScratch& s, const FrameCacheDev& cache, uint32_t rec,
+                              hipStream_t st)
+{
+    const dim3 g(job.n_tiles), b(kLtBlock);
+#define BZ_LATE(T) \
+    hipLaunchKernelGGL((late_tile_kernel<T, false>), g, b, 0, st, job, cache, s.counts, s.staging, FuseDev{})
     switch (rec) {
-    case 512: return launch_late_cached_t<512>(job, s, cache, n_rec_tiles, st);
-    case 1024: return launch_late_cached_t<1024>(job, s, cache, n_rec_tiles, st);
-    case 2048: return launch_late_cached_t<2048>(job, s, cache, n_rec_tiles, st);
+    case 512: BZ_LATE(512); break;
+    case 1024: BZ_LATE(1024); break;
+    case 2048: BZ_LATE(2048); break;
     default: return hipErrorInvalidValue;
     }
+#undef BZ_LATE
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? launch_emit(job, rec, s, st) : e;
 }
 
 hipError_t launch_cluster_objects(const CullJob& job, const CompactScratch& s, uint32_t* ccounts, uint32_t block,

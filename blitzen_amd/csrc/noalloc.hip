@@ -15,11 +15,10 @@
 namespace bz {
 
 // counts[kNoAllocTiles] and their prefix[kNoAllocTiles + 1] (u32), then staging[kNoAllocEntries] (objectId, LOD)
-// pairs. Every tile size the tunings allow (512, 1024, 2048 objects) and the cached LATE pass's 4096-object
-// super-tiles fit BZ_NOALLOC_MAX_OBJECTS objects: at most BZ_NOALLOC_MAX_OBJECTS / 512 tiles, and the range rounded
-// up to a whole tile or super-tile of staging slots.
+// pairs. Every tile size the tunings allow (512, 1024, 2048 objects) fits BZ_NOALLOC_MAX_OBJECTS objects: at most
+// BZ_NOALLOC_MAX_OBJECTS / 512 tiles, and the range rounded up to a whole tile of staging slots (with room to spare).
 constexpr uint32_t kNoAllocTiles = BZ_NOALLOC_MAX_OBJECTS / 512u;
-constexpr uint64_t kNoAllocEntries = (uint64_t)BZ_NOALLOC_MAX_OBJECTS + kSuperTile;
+constexpr uint64_t kNoAllocEntries = (uint64_t)BZ_NOALLOC_MAX_OBJECTS + 4096u;
 constexpr uint64_t kNoAllocCountsBytes = (counts_words(kNoAllocTiles) * 4u + 255u) / 256u * 256u;
 constexpr uint64_t kNoAllocBytes = kNoAllocCountsBytes + kNoAllocEntries * sizeof(uint2);
 static_assert(kNoAllocBytes == 33652992ull, "the size bz_cull_noalloc's declaration states");
