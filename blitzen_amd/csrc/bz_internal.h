@@ -134,7 +134,8 @@ hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t blo
 constexpr uint32_t kFuseBlock = 256, kFuseItems = 2;
 constexpr uint32_t kFuseObjects = 5u << 16;
 constexpr uint32_t kFuseFirst = 16;  // (a cache line for the launch number)
-constexpr uint32_t kFuseWords = kFuseFirst + kFuseObjects / (kFuseBlock * kFuseItems);
+constexpr uint32_t kFuseTiles = kFuseObjects / (kFuseBlock * kFuseItems);
+constexpr uint32_t kFuseWords = kFuseFirst + kFuseTiles;
 hipError_t launch_fused(const CullJob& job, unsigned long long* words, uint32_t* err, hipStream_t st,
                         const FrameCacheDev* cache = nullptr);
 // Chunks of consecutive tiles: chunk c of a job holds tiles [t0, t1), the first n_long chunks tpc + 1 tiles and the
@@ -246,7 +247,8 @@ struct XfTarget {
 // Staged updates: ids[i] and the 32-byte MeshTransform record i (pos.xyz, scale | quaternion) scattered into the SoA
 // streams, the last occurrence of an id winning, and the world-space spheres of the objects that use those transforms;
 // an id >= n_transforms is skipped and sets err[2]. dev_records (2 n) and dev_ids (n): the device copies of both.
-hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n,
+// distinct: the caller knows that every id is in range and named once, so one launch does (no device copies).
+hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n, bool distinct,
                                             const XfTarget& target, float4* dev_records, uint32_t* dev_ids,
                                             uint32_t* err, hipStream_t st);
 // World-space spheres of every object of the scene.
@@ -302,7 +304,8 @@ struct ClusterScratch {
 
 hipError_t launch_cluster_objects(const CullJob& job, const CompactScratch& s, uint32_t* ccounts, uint32_t block,
                                   uint32_t items, hipStream_t st);
+// words, err: as for launch_fused
 hipError_t launch_cluster_pass(const ClusterJob& job, const CompactScratch& cs, const ClusterScratch& xs,
-                               hipStream_t st);
+                               unsigned long long* words, uint32_t* err, hipStream_t st);
 
 }  // namespace bz

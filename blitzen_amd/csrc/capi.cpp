@@ -639,9 +639,9 @@ bz_status bz_scene_transform_staging(bz_ctx* ctx, bz_scene scene, uint32_t capac
     return BZ_OK;
 }
 
-bz_status bz_scene_commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, void* stream)
+// distinct: the slot's first n ids are in range and name no transform twice.
+static bz_status commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, bool distinct, void* stream)
 {
-    if (!ctx) return BZ_E_INVALID;
     Scene* s = ctx->scene(scene);
     if (!s) return ctx->fail(BZ_E_INVALID, "unknown scene handle");
     if (s->xf_open < 0) return ctx->fail(BZ_E_STATE, "no staging slot handed out (bz_scene_transform_staging)");
@@ -659,7 +659,8 @@ bz_status bz_scene_commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, vo
         const uint32_t stamp = (uint32_t)(s->xf_version % 0xffffffffull) + 1u;
         const XfTarget to{ s->dev(), s->xf_ps, s->xf_q, s->world, s->xf_winner, s->xf_stamp, stamp };
         e = launch_scatter_staged_transforms(reinterpret_cast<const uint32_t*>(x.host),
-                                             reinterpret_cast<const float4*>(x.host + x.xf_offset), n, to, x.dev,
+                                             reinterpret_cast<const float4*>(x.host + x.xf_offset), n, distinct, to,
+                                             x.dev,
                                              reinterpret_cast<uint32_t*>(x.dev + 2 * (size_t)x.cap), sc->err, st);
     }
     if (e == hipSuccess) e = hipEventRecord(x.done, st);
@@ -667,6 +668,12 @@ bz_status bz_scene_commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, vo
     s->xf_next = (uint32_t)s->xf_open ^ 1u;
     s->xf_open = -1;
     return BZ_OK;
+}
+
+bz_status bz_scene_commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, void* stream)
+{
+    if (!ctx) return BZ_E_INVALID;
+    return commit_transforms(ctx, scene, n, false, stream);
 }
 
 bz_status bz_scene_update_transforms(bz_ctx* ctx, bz_scene scene, const uint32_t* ids, const bz_MeshTransform* xf,
@@ -677,8 +684,11 @@ bz_status bz_scene_update_transforms(bz_ctx* ctx, bz_scene scene, const uint32_t
     if (!s) return ctx->fail(BZ_E_INVALID, "unknown scene handle");
     if (n == 0) return BZ_OK;
     if (!ids || !xf) return ctx->fail(BZ_E_INVALID, "NULL ids / transforms");
-    for (uint32_t k = 0; k < n; ++k)
+    bool ascending = true;  // strictly: no id twice
+    for (uint32_t k = 0; k < n; ++k) {
         if (ids[k] >= s->n_transforms) return ctx->fail(BZ_E_INVALID, "transform id out of range");
+        ascending = ascending && (k == 0 || ids[k] > ids[k - 1]);
+    }
     if (s->xf_open >= 0) return ctx->fail(BZ_E_STATE, "a transform staging slot is open: commit it first");
     // through the staging slots: the host arrays are copied as they are (32-byte records), the kernel splits them
     uint32_t* sid = nullptr;
@@ -687,7 +697,7 @@ bz_status bz_scene_update_transforms(bz_ctx* ctx, bz_scene scene, const uint32_t
     if (st) return st;
     std::memcpy(sid, ids, (size_t)n * 4);
     std::memcpy(sxf, xf, (size_t)n * sizeof(bz_MeshTransform));
-    return bz_scene_commit_transforms(ctx, scene, n, stream);
+    return commit_transforms(ctx, scene, n, ascending, stream);
 }
 
 bz_status bz_scene_set_visibility(bz_ctx* ctx, bz_scene scene, const uint32_t* vis, uint32_t n, void* stream)
@@ -1228,7 +1238,7 @@ bz_status bz_cull_clusters(bz_ctx* ctx, const bz_cluster_cull_args* a, void* str
     cj.n_tiles = oj.n_tiles;
     cj.tile_size = t.block * t.items;
     hipError_t e = launch_cluster_objects(oj, sc->cs, sc->xs.ccounts, t.block, t.items, st);
-    if (e == hipSuccess) e = launch_cluster_pass(cj, sc->cs, sc->xs, st);
+    if (e == hipSuccess) e = launch_cluster_pass(cj, sc->cs, sc->xs, sc->fuse, sc->err, st);
     if (e != hipSuccess) return ctx->hip_fail(e, "cluster cull launch");
     return BZ_OK;
 }
