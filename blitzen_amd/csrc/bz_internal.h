@@ -71,8 +71,9 @@ inline void set_prefix(CompactScratch& s, bool batches)
 }
 
 // An emit workgroup adds the counts of its job's earlier tiles itself when there are at most kScanTiles of them (one
-// round of loads). A job with more tiles gets their exclusive prefix from one scan launch between the decide and the
-// emit instead, so the emit's work per workgroup stays constant and the pass stays linear in the object count.
+// round of loads), and in a launch of its own shape also beyond (kEmitSumTiles). Batches and cluster passes with more
+// tiles get their exclusive prefix from one scan launch between the decide and the emit instead, so that the work per
+// workgroup stays constant and the pass stays linear in the object count.
 constexpr uint32_t kScanTiles = 4096;
 // Exclusive prefix of counts[0, n) into prefix[0, n], prefix[n] = the total (one workgroup, linear in n).
 hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* prefix, hipStream_t st);

@@ -647,11 +647,15 @@ hipError_t launch_cluster_objects_t(const CullJob& job, const CompactScratch& s,
 // ------------------------------------------------------------------------------------------------ emit
 constexpr uint32_t kEmitBlock = 256;
 constexpr uint32_t kEmitTiles = kEmitBlock / 64;  // one tile per wave
+constexpr uint32_t kEmitWideBlock = 1024;         // jobs of more than kScanTiles tiles: 16 tiles per workgroup
+constexpr uint32_t kEmitSumTiles = 32768;         // up to these the workgroup adds up the earlier tiles' counts
 constexpr uint32_t kEmitUnroll = 2;               // entries per lane in flight (a tile emits ~70 on average)
 
+template <uint32_t BLOCK, bool WIDE>
 struct EmitSmem {
-    uint32_t red[kEmitBlock / 64];
-    uint32_t cnt[kEmitTiles + 1];     // exclusive prefix of the workgroup's tile counts
+    uint32_t red[BLOCK / 64];
+    uint32_t cnt[BLOCK / 64 + 1];                            // exclusive prefix of the workgroup's tile counts
+    alignas(16) uint2 buf[WIDE ? BLOCK / 64 : 1][64u * 3u];  // the waves' commands
 };
 
 // A workgroup barrier for LDS only: waits for this wave's LDS operations (lgkmcnt(0)) but not for its global loads in
@@ -664,16 +668,44 @@ __device__ __forceinline__ void block_lds_sync()
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// Writes the commands of tiles [t0, t1) of one job (t1 - t0 <= kEmitTiles; tile_size >= 64 * kEmitUnroll). One round
-// of loads gets the counts of the job's earlier tiles (reduced to the output base; at most kScanTiles of them), or
+// The commands of up to 64 staged entries (lane l holds entry l; the first cnt count), at cmds[pos0 ...), put together in
+// the wave's LDS and stored as 16-byte words (a command is 24 bytes: the words are 8-byte aligned, the last may be half a
+// one). For the large jobs, whose emit is bound by its stores: three 8-byte words per lane, 24 bytes apart, touch every
+// line of the output three times (16 777 216 objects, 1.6 M commands: 82.9 -> 81.7 us). A small job waits longer for the
+// LDS than it saves (4 194 304-object frame 57.7 -> 57.9 us) and keeps the plain stores.
+__device__ __forceinline__ void write_wave_commands(uint2* buf, uint32_t* cmds, uint32_t pos0, uint32_t cnt,
+                                                    uint32_t object, uint2 draw)
+{
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x4_at8 __attribute__((ext_vector_type(4), aligned(8)));
+    const uint32_t lane = threadIdx.x & 63u;
+    write_command(reinterpret_cast<uint32_t*>(buf), lane, object, draw);
+    wave_lds_sync();
+    uint32_t* out = cmds + (size_t)pos0 * 6u;
+    const uint32_t words = cnt * 6u;
+#pragma unroll
+    for (uint32_t k = 0; k < 2u; ++k) {
+        const uint32_t i = (k * 64u + lane) * 4u;
+        if (i >= words) break;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint32_t*>(buf) + i);
+        if (i + 4u <= words) *reinterpret_cast<u32x4_at8*>(out + i) = v;
+        else *reinterpret_cast<uint2*>(out + i) = make_uint2(v.x, v.y);
+    }
+    wave_lds_sync();
+}
+
+// Writes the commands of tiles [t0, t1) of one job (t1 - t0 <= BLOCK / 64; tile_size >= 64 * kEmitUnroll). One round
+// of loads gets the counts of the job's earlier tiles (reduced to the output base; 16 per thread and round), or
 // with `scanned` (the exclusive prefix of all counts) two entries of it, the workgroup's own counts and,
 // before any count is known, the first 64 * kEmitUnroll staging entries of each wave's tile (in bounds: every tile
 // owns tile_size slots); each wave gathers its entries' LOD draw data while the block scan of the counts runs, then
 // writes tile t0 + w's commands in order. Longer tiles continue in rounds of kEmitUnroll entries per lane.
+template <uint32_t BLOCK, bool WIDE>
 __device__ __forceinline__ void emit_tiles(const CullJob& J, uint32_t t0, uint32_t t1, uint32_t tile_size,
                                            const uint32_t* counts, const uint2* staging, const uint32_t* scanned,
-                                           EmitSmem& sm)
+                                           EmitSmem<BLOCK, WIDE>& sm)
 {
+    constexpr uint32_t NW = BLOCK / 64u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t nt = t1 - t0;
     const uint32_t tw = t0 + (wave < nt ? wave : 0u);  // this wave's tile (clamped for waves without one)
@@ -688,11 +720,11 @@ __device__ __forceinline__ void emit_tiles(const CullJob& J, uint32_t t0, uint32
     const uint32_t own = tid < nt ? counts[t0 + tid] : 0u;
     if (scanned) {  // one lane takes the difference of the scanned prefixes; the reduction below adds it
         if (tid == 0) part = scanned[t0] - scanned[J.tile_start];
-    } else for (uint32_t u0 = J.tile_start; u0 < t0; u0 += 16u * kEmitBlock) {
+    } else for (uint32_t u0 = J.tile_start; u0 < t0; u0 += 16u * BLOCK) {
         uint32_t v[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const uint32_t u = u0 + (uint32_t)j * kEmitBlock + tid;
+            const uint32_t u = u0 + (uint32_t)j * BLOCK + tid;
             v[j] = u < t0 ? counts[u] : 0u;
         }
 #pragma unroll
@@ -707,17 +739,17 @@ __device__ __forceinline__ void emit_tiles(const CullJob& J, uint32_t t0, uint32
     if (wave == 0) {
         uint32_t v = own;
 #pragma unroll
-        for (int off = 1; off < (int)kEmitTiles; off <<= 1) {
+        for (int off = 1; off < (int)NW; off <<= 1) {
             const uint32_t t = __shfl_up(v, off, 64);
             if (lane >= (uint32_t)off) v += t;
         }
-        if (lane < kEmitTiles) sm.cnt[lane + 1] = v;
+        if (lane < NW) sm.cnt[lane + 1] = v;
         if (lane == 0) sm.cnt[0] = 0;
     }
     block_lds_sync();
     uint32_t prefix = 0;
 #pragma unroll
-    for (uint32_t w = 0; w < kEmitBlock / 64u; ++w) prefix += sm.red[w];
+    for (uint32_t w = 0; w < NW; ++w) prefix += sm.red[w];
     if (tid == 0 && t1 == J.tile_start + J.n_tiles) *J.count = prefix + sm.cnt[nt];
     if (wave >= nt) return;
     const uint32_t base = prefix + sm.cnt[wave];
@@ -733,20 +765,29 @@ __device__ __forceinline__ void emit_tiles(const CullJob& J, uint32_t t0, uint32
         }
 #pragma unroll
         for (uint32_t u = 0; u < kEmitUnroll; ++u) {
-            const uint32_t e = e0 + u * 64u + lane;
-            const uint32_t pos = base + e;
-            if (e < c && pos < J.capacity) write_command(J.cmds, pos, ent[u].x, d[u]);
+            if constexpr (WIDE) {
+                const uint32_t e = e0 + u * 64u, pos = base + e;
+                if (e < c && pos < J.capacity) {  // uniform
+                    const uint32_t room = J.capacity - pos, left = c - e < 64u ? c - e : 64u;
+                    write_wave_commands(sm.buf[wave], J.cmds, pos, left < room ? left : room, ent[u].x, d[u]);
+                }
+            } else {
+                const uint32_t e = e0 + u * 64u + lane;
+                const uint32_t pos = base + e;
+                if (e < c && pos < J.capacity) write_command(J.cmds, pos, ent[u].x, d[u]);
+            }
         }
     }
 }
 
-__global__ __launch_bounds__(kEmitBlock) void emit_kernel(CullJob J, uint32_t tile_size, const uint32_t* counts,
-                                                          const uint2* staging, const uint32_t* prefix)
+template <uint32_t BLOCK, bool WIDE>
+__global__ __launch_bounds__(BLOCK) void emit_kernel(CullJob J, uint32_t tile_size, const uint32_t* counts,
+                                                     const uint2* staging, const uint32_t* prefix)
 {
-    __shared__ EmitSmem sm;
-    const uint32_t t0 = blockIdx.x * kEmitTiles;
-    const uint32_t t1 = t0 + kEmitTiles < J.n_tiles ? t0 + kEmitTiles : J.n_tiles;
-    emit_tiles(J, t0, t1, tile_size, counts, staging, prefix, sm);
+    __shared__ EmitSmem<BLOCK, WIDE> sm;
+    const uint32_t t0 = blockIdx.x * (BLOCK / 64u);
+    const uint32_t t1 = t0 + BLOCK / 64u < J.n_tiles ? t0 + BLOCK / 64u : J.n_tiles;
+    emit_tiles<BLOCK, WIDE>(J, t0, t1, tile_size, counts, staging, prefix, sm);
 }
 
 // Batched emit of one tile by one wave: its count, its first 64 * kEmitUnroll entries and its job's number are loaded
@@ -828,18 +869,27 @@ __global__ __launch_bounds__(kEmitBlock) void emit_few_kernel(JobArgs jobs, uint
     emit_batch_tile(jobs.j[few_job(jobs, t)], t, counts[t], ent, stage, counts, prefix);
 }
 
-// The emit launch of one job whose decide launch wrote s.counts / s.staging; a job of more than kScanTiles tiles
-// first gets its counts' prefix from the scan.
+// The emit launch of one job whose decide launch wrote s.counts / s.staging. Up to kScanTiles tiles, 4 per workgroup. Above,
+// 16 per workgroup of 1024 threads: each workgroup still adds up all the counts before its own, one round of loads per
+// 16 384 tiles, but there are a quarter as many workgroups to do so, and that costs less than a scan launch between the
+// two kernels, which one workgroup runs while the others wait (with the scan / without: 4199 tiles 29.3 / 26.5 us, 11 719
+// tiles 62.8 / 57.8, 16 384 tiles 82.9 / 78.1, 23 438 tiles 114.1 / 108.5; 512 threads at 16 384 tiles 78.3). The sums
+// grow with the square of the tiles: from three rounds on (46 875 tiles: 137.1 / 139.2 us) the scan is the better one.
 hipError_t launch_emit(const CullJob& job, uint32_t tile_size, const CompactScratch& s, hipStream_t st)
 {
     const uint32_t* prefix = nullptr;
-    if (job.n_tiles > kScanTiles) {
+    if (job.n_tiles > kEmitSumTiles) {
         const hipError_t e = launch_scan_counts(s.counts, job.n_tiles, s.prefix, st);
         if (e != hipSuccess) return e;
         prefix = s.prefix;
     }
-    hipLaunchKernelGGL(emit_kernel, dim3((job.n_tiles + kEmitTiles - 1) / kEmitTiles), dim3(kEmitBlock), 0, st, job,
-                       tile_size, (const uint32_t*)s.counts, (const uint2*)s.staging, prefix);
+#define BZ_EMIT(B, W) \
+    hipLaunchKernelGGL((emit_kernel<B, W>), dim3((job.n_tiles + B / 64u - 1u) / (B / 64u)), dim3(B), 0, st, job, \
+                       tile_size, (const uint32_t*)s.counts, (const uint2*)s.staging, prefix)
+    if (job.n_tiles <= kScanTiles) BZ_EMIT(kEmitBlock, false);
+    else if (!prefix) BZ_EMIT(kEmitWideBlock, true);
+    else BZ_EMIT(kEmitBlock, true);
+#undef BZ_EMIT
     return hipGetLastError();
 }
 
