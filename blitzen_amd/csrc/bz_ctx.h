@@ -56,7 +56,7 @@ struct Scene {
     // [ids | 32-byte MeshTransforms], used in turn
     struct XfSlot {
         uint8_t* host = nullptr;       // pinned, read by a kernel: cap ids, then cap transforms at xf_offset
-        float4* dev = nullptr;         // device copy of the committed updates: 2 cap float4 of transforms, then cap ids
+        uint32_t* dev = nullptr;       // device copy of the committed ids [cap]
         uint32_t cap = 0;
         size_t xf_offset = 0;
         hipEvent_t done = nullptr;     // the last commit from this slot completed
@@ -100,7 +100,8 @@ struct Pyramid : PyrPlan {
 struct StreamScratch {
     CompactScratch cs{};
     unsigned long long* fuse = nullptr;  // [kFuseWords] the one-launch passes' published counts
-    uint32_t* err = nullptr;          // [0] instanced scan or one-launch pass wait gave up, [1] pyramid tail wait gave up, [2] staged transform id out of range
+    uint32_t* err = nullptr;          // [0] instanced scan or one-launch pass wait gave up, [1] pyramid tail wait gave up,
+                                      // [2] staged transform id out of range
     CullJob* jobs_dev = nullptr;
     CullJob* jobs_host = nullptr;     // pinned
     uint32_t jobs_cap = 0;

@@ -15,8 +15,9 @@ namespace bz {
 // the translation of the sphere's centre do not depend on the view, so they are done once per transform that is set
 // (bz_scene_create, the transform updates) and not once per object, view and pass. The decide kernels are bound by these
 // streams (PLAIN decide of 16 777 216 objects 112 -> 70 us, recording EARLY of 4 194 304 objects 33.3 -> 25.6 us, batched
-// decide of 64 views, 9 M pairs, 104.5 -> 81.9 us; with transform indices, 262 161 objects, 14.0 -> 7.4 us). The values are the ones the passes computed, rounding for rounding (sphere_to_world). Transforms stay
-// resident beside them, split into two 16-byte streams (cluster tests, updates, read-back).
+// decide of 64 views, 9 M pairs, 104.5 -> 81.9 us; with transform indices, 262 161 objects, 14.0 -> 7.4 us). The
+// values are the ones the passes computed, rounding for rounding (sphere_to_world). Transforms stay resident beside them,
+// split into two 16-byte streams (cluster tests, updates, read-back).
 struct SceneDev {
     const uint32_t* obj_surf;   // [n_objects] RenderObject.surfaceId (nullptr when stored as 16-bit)
     const uint16_t* obj_surf16; // [n_objects] RenderObject.surfaceId when every id < 65536 (else nullptr)
@@ -247,11 +248,11 @@ struct XfTarget {
 };
 // Staged updates: ids[i] and the 32-byte MeshTransform record i (pos.xyz, scale | quaternion) scattered into the SoA
 // streams, the last occurrence of an id winning, and the world-space spheres of the objects that use those transforms;
-// an id >= n_transforms is skipped and sets err[2]. dev_records (2 n) and dev_ids (n): the device copies of both.
-// distinct: the caller knows that every id is in range and named once, so one launch does (no device copies).
+// an id >= n_transforms is skipped and sets err[2]. dev_ids (n): a device copy of the ids.
+// distinct: the caller knows that every id is in range and named once, so one launch does for up to kDistinctUpdates.
+constexpr uint32_t kDistinctUpdates = 16384;
 hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n, bool distinct,
-                                            const XfTarget& target, float4* dev_records, uint32_t* dev_ids,
-                                            uint32_t* err, hipStream_t st);
+                                            const XfTarget& target, uint32_t* dev_ids, uint32_t* err, hipStream_t st);
 // World-space spheres of every object of the scene.
 hipError_t launch_world_spheres(const SceneDev& scene, float4* world, hipStream_t st);
 hipError_t launch_synth_depth(uint64_t seed, uint32_t w, uint32_t h, uint32_t occluders, float p11, float znear,

@@ -276,7 +276,7 @@ constexpr bz_tuning kBuiltInTuning{ 512, 2, 0, 0 };
 
 // Two objects a thread up to 2^21 objects, four above. Four are better where the streams bound the pass and the objects
 // in view are spread over all tiles: a wave's compacted LOD selection then runs on twice the lanes (4 194 304 objects at
-// random with the frame cache 59.2 against 62.8 us, PLAIN of 16 777 216 83.1 against 92.5; 2 000 000 only 41.8 against 42.8).
+// random with the frame cache 59.2 against 62.8 us, PLAIN of 12 000 000 57.9 against 73.3; 2 000 000 only 41.8 against 42.8).
 // Where neighbouring ids are neighbours in space, a tile is all in view or not at all, and a wave works through its
 // survivors 64 at a time: half as many per wave spread them better (2 000 000 in region order 41.7 against 49.9 us, 1 048 576
 // 34.0 against 38.7, 600 000 30.7 against 34.3).
@@ -610,7 +610,7 @@ bz_status bz_scene_transform_staging(bz_ctx* ctx, bz_scene scene, uint32_t capac
         const size_t off = ((size_t)capacity * 4 + 255) / 256 * 256;
         const size_t bytes = off + (size_t)capacity * sizeof(bz_MeshTransform);
         hipError_t e = hipHostMalloc((void**)&x.host, bytes, hipHostMallocDefault);  // pinned, device-readable
-        if (e == hipSuccess) e = hipMalloc((void**)&x.dev, (size_t)capacity * (sizeof(bz_MeshTransform) + 4));
+        if (e == hipSuccess) e = hipMalloc((void**)&x.dev, (size_t)capacity * 4);
         if (e == hipSuccess && !s->xf_winner) {
             e = hipMalloc((void**)&s->xf_winner, (size_t)s->n_transforms * 4);
             if (e == hipSuccess) e = hipMemset(s->xf_winner, 0, (size_t)s->n_transforms * 4);
@@ -654,14 +654,13 @@ static bz_status commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, bool
     ++s->xf_version;  // frame-cache survivors recorded before this update no longer apply
     hipError_t e = hipSuccess;
     if (n) {
-        // a kernel reads the pinned slot over the host link, ids and records once
+        // the kernels read the pinned slot over the host link, ids and records once
         // (a stamp repeats after 2^32 - 1 updates, and then only has spheres recomputed that need not be)
         const uint32_t stamp = (uint32_t)(s->xf_version % 0xffffffffull) + 1u;
         const XfTarget to{ s->dev(), s->xf_ps, s->xf_q, s->world, s->xf_winner, s->xf_stamp, stamp };
         e = launch_scatter_staged_transforms(reinterpret_cast<const uint32_t*>(x.host),
                                              reinterpret_cast<const float4*>(x.host + x.xf_offset), n, distinct, to,
-                                             x.dev,
-                                             reinterpret_cast<uint32_t*>(x.dev + 2 * (size_t)x.cap), sc->err, st);
+                                             x.dev, sc->err, st);
     }
     if (e == hipSuccess) e = hipEventRecord(x.done, st);
     if (e != hipSuccess) return ctx->hip_fail(e, "staged transform update");
@@ -684,11 +683,13 @@ bz_status bz_scene_update_transforms(bz_ctx* ctx, bz_scene scene, const uint32_t
     if (!s) return ctx->fail(BZ_E_INVALID, "unknown scene handle");
     if (n == 0) return BZ_OK;
     if (!ids || !xf) return ctx->fail(BZ_E_INVALID, "NULL ids / transforms");
-    bool ascending = true;  // strictly: no id twice
-    for (uint32_t k = 0; k < n; ++k) {
-        if (ids[k] >= s->n_transforms) return ctx->fail(BZ_E_INVALID, "transform id out of range");
-        ascending = ascending && (k == 0 || ids[k] > ids[k - 1]);
+    uint32_t outside = ids[0] >= s->n_transforms ? 1u : 0u, unordered = 0;  // (no early exit: the loop is vectorised)
+    for (uint32_t k = 1; k < n; ++k) {
+        outside |= ids[k] >= s->n_transforms ? 1u : 0u;
+        unordered |= ids[k] <= ids[k - 1] ? 1u : 0u;
     }
+    if (outside) return ctx->fail(BZ_E_INVALID, "transform id out of range");
+    const bool ascending = !unordered;  // strictly: no id twice
     if (s->xf_open >= 0) return ctx->fail(BZ_E_STATE, "a transform staging slot is open: commit it first");
     // through the staging slots: the host arrays are copied as they are (32-byte records), the kernel splits them
     uint32_t* sid = nullptr;

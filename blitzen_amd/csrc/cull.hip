@@ -4,18 +4,19 @@
 // OnpcDrawCull.comp.glsl:11-52 and drawOccTemporal.hlsl:13-64. The per-object arithmetic is in cull_math.h.
 //
 // Two kernels per pass, both HBM-streaming, with no wait between workgroups:
-//   decide: one workgroup per tile of BLOCK x ITEMS objects (object tile*TILE + k*BLOCK + tid). Every object stream
+//   decide: tiles of BLOCK x ITEMS objects, each wave a run of 64 x ITEMS neighbouring ones. Every object stream
 //           of the tile is loaded at once (coalesced SoA float4 / uint32 loads); sphere -> view space and frustum
 //           test for every object; the frustum survivors of each wave are compacted into LDS so the Hi-Z test
 //           (two square roots, five divisions, a 2x2 gather) runs on dense lanes, and likewise the emitting objects
-//           for LOD selection. Emitting objects are ranked with a wave64 ballot and an LDS scan in (item, wave)
+//           for LOD selection. Emitting objects are ranked with wave64 ballots and the waves' totals in (wave, item)
 //           order, i.e. ascending object order, and written as (objectId, LOD) to the tile's staging slot; the
 //           tile's count goes to counts[tile]. The LATE pass also writes visibility here.
 //   emit:   each workgroup takes a run of tiles, adds the counts of the job's earlier tiles (a block reduction) to
 //           get its output base, and writes DrawIndexedIndirect commands in order, plus the draw count.
 // The output order is ascending objectId, independent of scheduling (the reference appends in atomicAdd order).
-// A single-pass decoupled look-back was measured slower here: cross-XCD status visibility costs ~1 us per round
-// trip and the first generation of workgroups walked back tens of round trips.
+// A pass over few objects is one kernel (fused_kernel, late_tile_kernel): each tile adds up the counts that the tiles
+// before it publish. For many tiles, and as a decoupled look-back, that was measured slower: cross-XCD status visibility
+// costs ~1 us per round trip and the first generation of workgroups waits for the slowest of them.
 #include "bz_internal.h"
 #include "fuse.h"
 
@@ -1346,32 +1347,28 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t 
 
 // Transform updates, in two launches so that an id named more than once in one commit takes its last occurrence
 // (UpdateObjectTransform copies updates into the staging buffer in call order, vulkanDraw.cpp:816-820):
-//   stage:   copies ids and records from the pinned slot into device memory, one coalesced 16-byte word per thread, and
-//            update i raises winner[id] to i + 1;
-//   scatter: update i writes its 32-byte record into the position/scale and quaternion streams only if it is the
-//            winner, which then clears winner[id] (the array is all zero between commits; a non-winner compares its
-//            own i + 1 and never matches, whether it reads before or after that clear).
+//   mark:    copies ids from the pinned slot into device memory; update i raises winner[id] to i + 1;
+//   scatter: update i reads its 32-byte record over the host link and writes it into the position/scale and quaternion
+//            streams, and its object's world-space sphere, only if it is the winner, which then clears winner[id] (the
+//            array is all zero between commits; a non-winner compares its own i + 1 and never matches, whether it reads
+//            before or after that clear).
 // Ids >= n_xf are skipped and set err[2].
-// The host link bounds the first launch, and everything that has to cross it does so there, in one round trip: reading
-// the records in the scatter, 32 bytes apart per lane and after its ids and winners had come back, cost a second one
-// (10 485 updates: 11.2 + 5.2 us with the objects' world-space spheres written too, against 4.1 + 9.6 us without them).
-__global__ __launch_bounds__(256) void stage_transforms_kernel(const uint32_t* __restrict__ ids,
-                                                               const float4* __restrict__ records, uint32_t n,
-                                                               uint32_t n_xf, float4* __restrict__ dev_records,
-                                                               uint32_t* __restrict__ dev_ids, uint32_t* winner,
-                                                               uint32_t* err)
+// The host link bounds both. One thread reads a whole record, and everything else that it needs before (id, winner,
+// surface): 41 943 updates 38.0 us, 200 000 152 us; with the records' loads issued first 38.5 and 161, with a thread per
+// 16-byte half 44.3 and 175. Writing the spheres costs 0.8 us of the 38.0.
+__global__ __launch_bounds__(256) void mark_staged_transforms_kernel(const uint32_t* __restrict__ ids, uint32_t n,
+                                                                     uint32_t n_xf, uint32_t* __restrict__ dev_ids,
+                                                                     uint32_t* winner, uint32_t* err)
 {
-    const uint32_t j = blockIdx.x * 256u + threadIdx.x;  // grid: 2n threads (n < 2^31 transforms fit the host's memory)
-    const bool own = j < n;
-    const uint32_t id = own ? ids[j] : 0u;
-    if (j < 2ull * n) dev_records[j] = records[j];
-    if (!own) return;
-    dev_ids[j] = id;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t id = ids[i];
+    dev_ids[i] = id;
     if (id >= n_xf) {
         atomicOr(&err[2], 1u);
         return;
     }
-    atomicMax(&winner[id], j + 1u);
+    atomicMax(&winner[id], i + 1u);
 }
 
 // World-space bounding sphere of an object, and its transform's scale.
@@ -1395,39 +1392,34 @@ __global__ __launch_bounds__(256) void scatter_staged_transforms_kernel(const ui
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
     const uint32_t id = dev_ids[i];
-    const float4 ps = records[2u * i], q = records[2u * i + 1u];
     if (id >= to.scene.n_transforms || to.winner[id] != i + 1u) return;
+    const bool sphere = !to.scene.obj_xf && id < to.scene.n_objects;
+    const float4 sph = sphere ? object_surface(to.scene, id) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 ps = records[2u * i], q = records[2u * i + 1u];
     to.xf_ps[id] = ps;
     to.xf_q[id] = q;
     to.winner[id] = 0u;
-    if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
-    else if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), ps, q);
+    if (sphere) to.world[id] = world_sphere(sph, ps, q);
+    else if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
 }
 
-// Updates that name every id once (and in range): straight from the pinned slot to the streams in one launch, two threads
-// an update (one 16-byte half each, so that the host link is read in whole lines), which exchange their halves for the
-// world-space sphere (10 485 updates: 11.5 us against 11.2 + 5.2 us).
+// Updates that name every id once (and in range), up to kDistinctUpdates of them: straight from the pinned slot to the
+// streams in one launch. Calls with 4096 updates 11.5 us against 14.3 in two launches, 10 485 16.2 against 18.6, 16 384 21.1
+// against 22.8, 24 576 27.7 against 28.7, but 41 943 51.5 against 39.1: ids and records read over the link at once slow each
+// other down when there are many.
 __global__ __launch_bounds__(256) void scatter_distinct_transforms_kernel(const uint32_t* __restrict__ ids,
                                                                           const float4* __restrict__ records,
                                                                           uint32_t n, XfTarget to)
 {
-    const uint64_t j = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    const bool in = j < 2ull * n;  // (2 n is even: both threads of an update are in, or neither)
-    const uint32_t id = in ? ids[j >> 1] : 0u;
-    const float4 h = in ? records[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 q;  // the odd thread's half
-    q.x = __shfl_xor(h.x, 1, 64);
-    q.y = __shfl_xor(h.y, 1, 64);
-    q.z = __shfl_xor(h.z, 1, 64);
-    q.w = __shfl_xor(h.w, 1, 64);
-    if (!in) return;
-    if (j & 1u) {
-        to.xf_q[id] = h;
-        return;
-    }
-    to.xf_ps[id] = h;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t id = ids[i];
+    const float4 ps = records[2u * i], q = records[2u * i + 1u];
+    if (id >= to.scene.n_transforms) return;  // (the caller has looked: only a caller's race on its ids gets here)
+    to.xf_ps[id] = ps;
+    to.xf_q[id] = q;
     if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
-    else if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), h, q);
+    else if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), ps, q);
 }
 
 // World-space spheres of the scene's objects: all of them (stamp == nullptr), or those whose transform carries the
@@ -1452,20 +1444,18 @@ hipError_t launch_world_spheres(const SceneDev& scene, float4* world, hipStream_
 }
 
 hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* records, uint32_t n, bool distinct,
-                                            const XfTarget& to, float4* dev_records, uint32_t* dev_ids, uint32_t* err,
-                                            hipStream_t st)
+                                            const XfTarget& to, uint32_t* dev_ids, uint32_t* err, hipStream_t st)
 {
     if (n == 0) return hipSuccess;
-    const dim3 g((n + 255u) / 256u), g2((uint32_t)((2ull * n + 255u) / 256u)), b(256);
-    if (distinct) {
-        hipLaunchKernelGGL(scatter_distinct_transforms_kernel, g2, b, 0, st, ids, records, n, to);
+    const dim3 g((n + 255u) / 256u), b(256);
+    if (distinct && n <= kDistinctUpdates) {
+        hipLaunchKernelGGL(scatter_distinct_transforms_kernel, g, b, 0, st, ids, records, n, to);
     } else {
-        hipLaunchKernelGGL(stage_transforms_kernel, g2, b, 0, st, ids, records, n, to.scene.n_transforms, dev_records,
-                           dev_ids, to.winner, err);
+        hipLaunchKernelGGL(mark_staged_transforms_kernel, g, b, 0, st, ids, n, to.scene.n_transforms, dev_ids, to.winner,
+                           err);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(scatter_staged_transforms_kernel, g, b, 0, st, (const uint32_t*)dev_ids,
-                           (const float4*)dev_records, n, to);
+        hipLaunchKernelGGL(scatter_staged_transforms_kernel, g, b, 0, st, (const uint32_t*)dev_ids, records, n, to);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !to.scene.obj_xf || to.scene.n_objects == 0) return e;

@@ -49,3 +49,31 @@ def test_update_reaches_every_object(n, mapping, surfaces):
             want, kw = orc.cull((objects, xfs, sc.surfaces, sc.lods), H.view_bytes(v), A.PASS_PLAIN)
             assert k == kw
             assert np.array_equal(H.cmds_u32(got), want)
+
+
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 40000])
+@pytest.mark.parametrize("order", ["ascending", "descending", "last twice"])
+def test_update_sizes(n, order):
+    """One launch for up to 16 384 ascending updates, two for more and for any other order."""
+    total = 50000
+    sc = bz.synth_scene(97, total, 16, 4)
+    rng = np.random.default_rng(n)
+    xfs, v = sc.transforms.copy(), H.view()
+    ids = np.sort(rng.permutation(total)[:n]).astype(np.uint32)
+    if order == "descending":
+        ids = np.ascontiguousarray(ids[::-1])
+    elif order == "last twice":
+        ids[-1] = ids[-2]
+    new = xfs[ids].copy()
+    new["pos"] = rng.uniform(-100, 100, (n, 3)).astype(np.float32)
+    for k, i in enumerate(ids):
+        xfs[i] = new[k]
+    with bz.Context(0) as ctx:
+        h = ctx.scene_create(sc.objects, sc.transforms, sc.surfaces, sc.lods)
+        cmds, cnt = ctx.alloc(total * 24), ctx.alloc(4)
+        ctx.update_transforms(h, ids, new)
+        ctx.cull(h, v, A.PASS_PLAIN, cmds, cnt)
+        got, k = ctx.read_commands(cmds, cnt)
+        ctx.check_kernels()
+        want, kw = orc.cull((sc.objects, xfs, sc.surfaces, sc.lods), H.view_bytes(v), A.PASS_PLAIN)
+        assert k == kw and np.array_equal(H.cmds_u32(got), want)
