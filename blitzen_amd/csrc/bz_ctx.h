@@ -180,6 +180,7 @@ struct Ctx {
     Scene* scene(bz_scene h);
     Pyramid* pyramid(bz_pyramid h);
     bz_status scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, StreamScratch** out);
+    bz_status words_for(hipStream_t st, StreamScratch** out);
     bz_status cluster_scratch_for(hipStream_t st, StreamScratch* sc, uint32_t tiles, uint64_t records);
     bz_status make_job(uint32_t pass, uint32_t flags, bz_scene sh, bz_pyramid ph, const bz_CameraViewData& view,
                        uint32_t begin, uint32_t count, const uint32_t* vis_in, uint32_t* vis_out, void* cmds,

@@ -154,6 +154,19 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
     return BZ_OK;
 }
 
+// The stream's words for a pass in one launch. A stream under capture whose first call this is has none yet.
+bz_status Ctx::words_for(hipStream_t st, StreamScratch** out)
+{
+    const auto it = scratch.find((uintptr_t)st);
+    if (it == scratch.end() || !it->second || !it->second->fuse) {
+        hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cst) == hipSuccess && cst != hipStreamCaptureStatusNone)
+            return fail(BZ_E_STATE, "the stream's words must be allocated, which is not allowed during stream capture; "
+                                    "run the call once before capturing");
+    }
+    return scratch_for(st, 0, 0, out);
+}
+
 // Cluster-pass scratch: per-tile arrays for `tiles` object tiles and a survivor buffer of `records` entries.
 bz_status Ctx::cluster_scratch_for(hipStream_t st, StreamScratch* sc, uint32_t tiles, uint64_t records)
 {
@@ -1008,7 +1021,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
         hipError_t e = hipSuccess;
         if (!fixed && one_launch(job.n) && fc.block * fc.items == kFuseBlock * kFuseItems) {
             StreamScratch* sc = nullptr;
-            s = scratch_for(st, 0, 0, &sc);
+            s = words_for(st, &sc);
             if (s) return s;
             e = launch_late_fused(job, d, sc->fuse, sc->err, st);
         } else {
@@ -1022,7 +1035,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
     }
     // few objects under the built-in tuning: the whole pass in one launch, with no compaction scratch
     StreamScratch* fuse = nullptr;
-    if (!fixed && one_launch(job.n)) s = scratch_for(st, 0, 0, &fuse);
+    if (!fixed && one_launch(job.n)) s = words_for(st, &fuse);
     else s = compact(job.n_tiles, (uint64_t)job.n_tiles * t.block * t.items, &cs);
     if (s) return s;
     auto launch = [&](const FrameCacheDev* d) {

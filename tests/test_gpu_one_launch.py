@@ -114,3 +114,25 @@ def test_graph_replays_between_eager_passes(world):
         g.launch(s)
         check(world, A.PASS_LATE, 9, 100000, stream=s)
     world["ctx"].check_kernels(s)
+
+
+def test_first_call_on_a_captured_stream(world):
+    """A stream's hand-off words are allocated by its first call, which is refused under capture; after one call outside,
+    the same call is captured and replayed."""
+    s = world["ctx"].stream()
+    got = []
+
+    def first():
+        with pytest.raises(A.BzError) as e:
+            run(world, A.PASS_PLAIN, 0, 3000, stream=s)
+        got.append(e.value.status)
+
+    StreamGraph(s, first)
+    assert got == [A.E_STATE]
+    run(world, A.PASS_PLAIN, 0, 3000, stream=s)
+    check(world, A.PASS_PLAIN, 0, 3000, stream=s)
+    g = StreamGraph(s, lambda: run(world, A.PASS_PLAIN, 5, 2000, stream=s))
+    for _ in range(3):
+        run(world, A.PASS_PLAIN, 0, 3000, stream=s)
+        g.launch(s)
+        check(world, A.PASS_PLAIN, 5, 2000, stream=s)
