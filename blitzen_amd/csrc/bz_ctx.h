@@ -25,7 +25,7 @@ struct Scene {
     float4* xf_ps = nullptr;
     float4* xf_q = nullptr;
     float4* world = nullptr;           // world-space bounding spheres' centres and the scale, per object
-    uint32_t* xf_stamp = nullptr;      // [n_transforms] xf_version of each transform's last update (shared transforms)
+    uint8_t* xf_stamp = nullptr;       // [n_transforms] xf_version (mod 255, + 1) of each one's last update (obj_xf)
     float4* surf_sphere = nullptr;
     uint2* surf_lod = nullptr;
     float* lod_error = nullptr;

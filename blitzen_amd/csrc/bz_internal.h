@@ -243,8 +243,8 @@ struct XfTarget {
     SceneDev scene;
     float4 *xf_ps, *xf_q, *world;
     uint32_t* winner;           // [n_transforms] zero before and after the launches
-    uint32_t* stamp;            // [n_transforms] the last update of each transform (scenes with obj_xf; else nullptr)
-    uint32_t version;           // this update's stamp (not 0)
+    uint8_t* stamp;             // [n_transforms] the last update of each transform (scenes with obj_xf; else nullptr)
+    uint8_t version;            // this update's stamp (not 0)
 };
 // Staged updates: ids[i] and the 32-byte MeshTransform record i (pos.xyz, scale | quaternion) scattered into the SoA
 // streams, the last occurrence of an id winning, and the world-space spheres of the objects that use those transforms;

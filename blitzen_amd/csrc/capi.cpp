@@ -633,8 +633,8 @@ bz_status bz_scene_transform_staging(bz_ctx* ctx, bz_scene scene, uint32_t capac
             }
         }
         if (e == hipSuccess && s->obj_xf && !s->xf_stamp) {  // zero is no update's stamp
-            e = hipMalloc((void**)&s->xf_stamp, (size_t)s->n_transforms * 4);
-            if (e == hipSuccess) e = hipMemset(s->xf_stamp, 0, (size_t)s->n_transforms * 4);
+            e = hipMalloc((void**)&s->xf_stamp, (size_t)s->n_transforms);
+            if (e == hipSuccess) e = hipMemset(s->xf_stamp, 0, (size_t)s->n_transforms);
             if (e != hipSuccess && s->xf_stamp) {
                 (void)hipFree(s->xf_stamp);
                 s->xf_stamp = nullptr;
@@ -668,8 +668,8 @@ static bz_status commit_transforms(bz_ctx* ctx, bz_scene scene, uint32_t n, bool
     hipError_t e = hipSuccess;
     if (n) {
         // the kernels read the pinned slot over the host link, ids and records once
-        // (a stamp repeats after 2^32 - 1 updates, and then only has spheres recomputed that need not be)
-        const uint32_t stamp = (uint32_t)(s->xf_version % 0xffffffffull) + 1u;
+        // (a stamp repeats after 255 updates, and then only has spheres recomputed that need not be)
+        const uint8_t stamp = (uint8_t)(s->xf_version % 255u + 1u);
         const XfTarget to{ s->dev(), s->xf_ps, s->xf_q, s->world, s->xf_winner, s->xf_stamp, stamp };
         e = launch_scatter_staged_transforms(reinterpret_cast<const uint32_t*>(x.host),
                                              reinterpret_cast<const float4*>(x.host + x.xf_offset), n, distinct, to,
