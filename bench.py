@@ -387,7 +387,7 @@ def bench_size_scaling(ctx, stream, view, steps: int, copies: int = 2):
         us = e0.elapsed_ms(e1) / steps * 1e3
         n_cmd = int(cnt.download(np.uint32, 1, stream)[0])
         alg = n * 40 + n_cmd * CMD_BYTES + 4
-        out["sizes"].append({"objects": n, "tiles": n // 1024, "scanned_prefix": n // 1024 > 4096,
+        out["sizes"].append({"objects": n, "tiles": n // 1024, "scanned_prefix": n // 1024 > 32768,
                              "us": round(us, 2), "us_per_mobject": round(us / (n / 1048576), 3), "commands": n_cmd,
                              "achieved_gbs": round(alg / (us * 1e-6) / 1e9, 1)})
     for h in scenes:

@@ -29,7 +29,7 @@ from pathlib import Path
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 # decide_kernel<BLOCK, ITEMS, MODE, ...> with MODE 1 = LATE, as a demangled or a mangled symbol
 LATE_DECIDE = re.compile(r"decide_kernel<\d+, \d+, 1,|decide_kernelILi\d+ELi\d+ELi1E")
-EMIT = re.compile(r"emit_kernel\(|11emit_kernelE")
+EMIT = re.compile(r"emit_kernel[<(]|11emit_kernel[EI]")
 
 
 def demangle_short(name: str) -> str:
