@@ -36,6 +36,7 @@ struct ExpandSmem {
     uint32_t coff[kXMaxTile];  // first cluster of the object's LOD
     uint32_t red[kXWaves];
     uint32_t lvl[kMaxMips];
+    uint32_t last;  // FUSED: the number of the launch before
 };
 
 __device__ __forceinline__ uint32_t incl_scan64(uint32_t v, uint32_t lane)
@@ -55,8 +56,10 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
     return v;
 }
 
-// Sum of a[u] for u in [0, end), by the whole workgroup (all loads of a thread issued before the first add).
-__device__ __forceinline__ uint32_t block_prefix(const uint32_t* a, uint32_t end, uint32_t* red)
+// Sum of a[u] for u in [0, end), by the whole workgroup (all loads of a thread issued before the first add). `share` runs
+// ahead of the first of its two barriers, once the loads have come back.
+template <class Share>
+__device__ __forceinline__ uint32_t block_prefix(const uint32_t* a, uint32_t end, uint32_t* red, Share&& share)
 {
     const uint32_t tid = threadIdx.x;
     uint32_t part = 0;
@@ -72,6 +75,7 @@ __device__ __forceinline__ uint32_t block_prefix(const uint32_t* a, uint32_t end
     }
     part = wave_sum(part);
     if ((tid & 63u) == 0) red[tid >> 6] = part;
+    share();
     __syncthreads();
     uint32_t s = 0;
 #pragma unroll
@@ -128,7 +132,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_expand_kernel(ClusterJob J, c
 {
     __shared__ ExpandSmem sm;
     const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t launch = FUSED ? fuse_launch(fuse) : 0u;
+    const uint32_t last = FUSED ? fuse_last(fuse) : 0u;
     const uint32_t ne = counts[t];
     // the tile's first kXBlock staging entries, loaded with its count (before it is known; every tile owns
     // tile_size >= 2 * kXBlock slots), so that they arrive in the same round trip as the counts and the prefix
@@ -138,7 +142,10 @@ __global__ __launch_bounds__(kXBlock) void cluster_expand_kernel(ClusterJob J, c
         for (uint32_t L = 0; L < tid; ++L) off += level_dim(J.pyr.base_w, L) * level_dim(J.pyr.base_h, L);
         sm.lvl[tid] = off;
     }
-    const uint32_t base = J.scanned ? rbase[t] : block_prefix(ccounts, t, sm.red);
+    const uint32_t base = J.scanned ? rbase[t] : block_prefix(ccounts, t, sm.red, [&] {
+        if (FUSED && tid == 0) sm.last = last;
+    });
+    const uint32_t launch = FUSED ? fuse_launch(sm.last) : 0u;
 
     // the tile's emitting objects -> LOD cluster ranges, inclusive scan of the cluster counts
     uint32_t carry = 0;
@@ -253,7 +260,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_emit_kernel(ClusterJob J, con
     const uint32_t t1 = t0 + kCEmitTiles < J.n_tiles ? t0 + kCEmitTiles : J.n_tiles;
     const uint32_t nt = t1 - t0;
     const uint32_t own = tid < nt ? scount[t0 + tid] : 0u;
-    const uint32_t prefix = J.scanned ? sprefix[t0] : block_prefix(scount, t0, red);
+    const uint32_t prefix = J.scanned ? sprefix[t0] : block_prefix(scount, t0, red, [] {});
     if (wave == 0) {
         uint32_t v = own;
 #pragma unroll

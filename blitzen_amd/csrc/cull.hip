@@ -50,6 +50,7 @@ struct TileSmem {
     uint32_t wtot[2][BLOCK / 64];     // per-wave totals of the emitting objects, by the tile's parity
     uint32_t ctot[2][BLOCK / 64];     // frame cache: per-wave totals of the survivors
     uint32_t csum[BLOCK / 64];        // cluster mode: per-wave sums of the emitting objects' cluster counts
+    uint32_t last;                    // one-launch passes: the number of the launch before
 };
 
 // Pass families compiled separately so the visibility stream is loaded unconditionally where it is used.
@@ -528,11 +529,13 @@ template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool CACHE>
 __global__ __launch_bounds__(BLOCK) void fused_kernel(CullJob J, FrameCacheDev fc, FuseDev fuse)
 {
     __shared__ TileSmem<BLOCK, ITEMS, false> sm;
-    const uint32_t launch = fuse_launch(fuse);
+    const uint32_t last = fuse_last(fuse);  // (no branch: its wait comes behind the streams' loads)
     Streams<ITEMS> s;
     issue_tile<BLOCK, ITEMS, MODE, true, false>(J, blockIdx.x, s);
     stage_tables<BLOCK, ITEMS>(J, sm);
+    if (threadIdx.x == 0) sm.last = last;
     __syncthreads();
+    const uint32_t launch = fuse_launch(sm.last);
     process_tile<BLOCK, ITEMS, MODE, HIZ, false, false, CACHE, false, true>(
         J, blockIdx.x, blockIdx.x, 0u, s, nullptr, nullptr, nullptr, sm, NoPrefetch{}, fc, nullptr, fuse, launch);
 }
@@ -915,10 +918,10 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
                                                              uint2* staging, FuseDev fuse)
 {
     constexpr uint32_t NW = kLtBlock / 64, ROUNDS = TILE / kLtBlock;
-    __shared__ uint32_t s_new[TILE / 32], s_lvl[kMaxMips], s_tot[ROUNDS][NW], s_red[NW];
+    __shared__ uint32_t s_new[TILE / 32], s_lvl[kMaxMips], s_tot[ROUNDS][NW], s_red[NW], s_last;
     const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t base = t * TILE, nt = J.n - base < TILE ? J.n - base : TILE, obj0 = J.begin + base;
-    const uint32_t launch = FUSED ? fuse_launch(fuse) : 0u;
+    const uint32_t last = FUSED ? fuse_last(fuse) : 0u;
     const size_t slot0 = (size_t)t * TILE + tid;
     float4 sp = fc.sph[slot0];
     uint2 mt = fc.meta[slot0];
@@ -929,7 +932,9 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
         s_lvl[tid] = off;
     }
     if (tid < TILE / 32) s_new[tid] = 0u;
+    if (FUSED && tid == 0) s_last = last;
     __syncthreads();
+    const uint32_t launch = FUSED ? fuse_launch(s_last) : 0u;
     uint32_t before = 0;      // the tile's commands of the rounds so far
     bool emit[ROUNDS];        // FUSED: a round's commands wait for the tile's first slot
     uint32_t rank[ROUNDS], obj[ROUNDS];

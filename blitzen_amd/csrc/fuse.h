@@ -16,7 +16,7 @@ __device__ __forceinline__ void write_command(uint32_t* cmds, uint32_t pos, uint
 // The word another workgroup publishes for a tile in one launch: the tile's command count with the launch's number above
 // it. A word of another launch is not taken, so nothing is cleared between launches.
 struct FuseDev {
-    unsigned long long* words;  // [0] number of the last launch, [kFuseFirst + tile] the tiles' words
+    unsigned long long* words;  // [0] number of the last launch (32 bits), [kFuseFirst + tile] the tiles' words
     uint32_t* err;              // set when a wait gives up
 };
 
@@ -60,9 +60,16 @@ __device__ __forceinline__ uint32_t fuse_prefix(const FuseDev& fuse, uint32_t la
     for (uint32_t w = 0; w < BLOCK / 64u; ++w) prefix += red[w];
     return prefix;
 }
-__device__ __forceinline__ uint32_t fuse_launch(const FuseDev& fuse)  // this launch's number
+// The number of the launch before. The value that thread 0 reads is the workgroup's: it hands it to the others through LDS,
+// ahead of a barrier that the workgroup's word is published behind, so that no read of words[0] that counts is outstanding
+// once the word has arrived (a wave that used a read of its own could still be waiting for it then, and get the next one).
+__device__ __forceinline__ uint32_t fuse_last(const FuseDev& fuse)
 {
-    return (uint32_t)__hip_atomic_load(&fuse.words[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    return __hip_atomic_load(reinterpret_cast<uint32_t*>(fuse.words), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t fuse_launch(uint32_t last)  // this launch's number
+{
+    return __builtin_amdgcn_readfirstlane(last) + 1u;
 }
 __device__ __forceinline__ void fuse_publish(const FuseDev& fuse, uint32_t launch, uint32_t tile, uint32_t count)
 {
@@ -72,7 +79,7 @@ __device__ __forceinline__ void fuse_publish(const FuseDev& fuse, uint32_t launc
 // By the last tile, which has had every word: each workgroup has read the launch's number, so it can move on.
 __device__ __forceinline__ void fuse_finish(const FuseDev& fuse, uint32_t launch)
 {
-    __hip_atomic_store(&fuse.words[0], (unsigned long long)launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(reinterpret_cast<uint32_t*>(fuse.words), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace bz
