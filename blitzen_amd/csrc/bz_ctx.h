@@ -99,7 +99,9 @@ struct Pyramid : PyrPlan {
 
 struct StreamScratch {
     CompactScratch cs{};
-    unsigned long long* fuse = nullptr;  // [kFuseWords] the one-launch passes' published counts
+    unsigned long long* fuse = nullptr;  // [kFuseWords] the one-launch passes' hand-over words
+    uint2* fuse_left = nullptr;          // [kFuseObjects] and the commands that their tiles left
+    FuseScratch fused() const { return FuseScratch{ fuse, fuse_left, err }; }
     uint32_t* err = nullptr;          // [0] instanced scan or one-launch pass wait gave up, [1] pyramid tail wait gave up,
                                       // [2] staged transform id out of range
     CullJob* jobs_dev = nullptr;

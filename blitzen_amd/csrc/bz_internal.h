@@ -131,14 +131,22 @@ hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t blo
 // up the counts that the tiles before it publish, instead of an emit launch. That trades a launch (about 2 us, and as long
 // on the host) for a wait on the slowest earlier tile, which grows with the tiles: PLAIN of 131 072 objects 9.3 -> 6.9 us,
 // of 330 000 10.5 -> 8.7; EARLY + pyramid + LATE of 1000 objects 20 -> 15.7, of 262 144 27.5 -> 26.0, of 330 000 in region
-// order 28.4 -> 28.6, of 380 000 28.6 -> 29.5: the line is 640 tiles. `words` holds kFuseWords 64-bit words that are zero
-// before the first launch and kept between launches; launches on one array are ordered. err: set when a wait gives up.
+// order 28.4 -> 28.6, of 380 000 28.6 -> 29.5: the line is 640 tiles. wait_limit: looks at a count not there yet before a
+// tile leaves its commands to the last one (at most kFusePatience, some milliseconds).
 constexpr uint32_t kFuseBlock = 256, kFuseItems = 2;
 constexpr uint32_t kFuseObjects = 5u << 16;
 constexpr uint32_t kFuseFirst = 16;  // (a cache line for the launch number)
 constexpr uint32_t kFuseTiles = kFuseObjects / (kFuseBlock * kFuseItems);
-constexpr uint32_t kFuseWords = kFuseFirst + kFuseTiles;
-hipError_t launch_fused(const CullJob& job, unsigned long long* words, uint32_t* err, hipStream_t st,
+constexpr uint32_t kFuseWords = kFuseFirst + 2u * kFuseTiles;
+constexpr uint32_t kFusePatience = 4096;
+// What launches of one stream hand over: the words are zero before the first launch and kept between launches; launches on
+// one set are ordered.
+struct FuseScratch {
+    unsigned long long* words;  // [kFuseWords]
+    uint2* left;                // [kFuseObjects] commands that tiles left to the last one
+    uint32_t* err;              // set when the last tile's wait gives up
+};
+hipError_t launch_fused(const CullJob& job, const FuseScratch& s, uint32_t wait_limit, hipStream_t st,
                         const FrameCacheDev* cache = nullptr);
 // Chunks of consecutive tiles: chunk c of a job holds tiles [t0, t1), the first n_long chunks tpc + 1 tiles and the
 // others tpc (so that as many chunks as workgroups fit at once take the whole job evenly).
@@ -194,10 +202,10 @@ void decide_inst_chunks(const CullJob& job, uint32_t block, uint32_t items, uint
                         uint32_t* tiles_per_chunk, uint32_t* n_long, uint32_t* n_chunks);
 
 // LATE pass from a frame cache recorded over the same range in tiles of `rec` objects (512, 1024 or 2048; job.n_tiles of
-// them): with an emit launch, or in one launch (a cache recorded by launch_fused; words, err: as there).
+// them): with an emit launch, or in one launch (a cache recorded by launch_fused; s, wait_limit: as there).
 hipError_t launch_late_cached(const CullJob& job, const CompactScratch& s, const FrameCacheDev& cache, uint32_t rec,
                               hipStream_t st);
-hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, unsigned long long* words, uint32_t* err,
+hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, const FuseScratch& s, uint32_t wait_limit,
                              hipStream_t st);
 // The first tiles of up to kArgJobs jobs, passed to the batched decide as a kernel argument (2 KiB of the 4 KiB
 // kernarg segment).
@@ -306,8 +314,8 @@ struct ClusterScratch {
 
 hipError_t launch_cluster_objects(const CullJob& job, const CompactScratch& s, uint32_t* ccounts, uint32_t block,
                                   uint32_t items, hipStream_t st);
-// words, err: as for launch_fused
+// s, wait_limit: as for launch_fused
 hipError_t launch_cluster_pass(const ClusterJob& job, const CompactScratch& cs, const ClusterScratch& xs,
-                               unsigned long long* words, uint32_t* err, hipStream_t st);
+                               const FuseScratch& s, uint32_t wait_limit, hipStream_t st);
 
 }  // namespace bz

@@ -97,7 +97,7 @@ uint64_t PyrPlan::tail_words() const
 
 StreamScratch::~StreamScratch()
 {
-    void* ps[] = { cs.counts, cs.staging, jobs_dev, pjobs_dev, err, fuse, xs.ccounts, xs.rbase, xs.scount, xs.sprefix,
+    void* ps[] = { cs.counts, cs.staging, jobs_dev, pjobs_dev, err, fuse, fuse_left, xs.ccounts, xs.rbase, xs.scount, xs.sprefix,
                    xs.survivors, inst_hist, inst_seg };
     for (void* p : ps)
         if (p) (void)hipFree(p);
@@ -117,13 +117,15 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
     if (!s.err) {
         hipError_t e = hipMalloc((void**)&s.fuse, kFuseWords * 8u);
         if (e == hipSuccess) e = hipMemset(s.fuse, 0, kFuseWords * 8u);
+        if (e == hipSuccess) e = hipMalloc((void**)&s.fuse_left, kFuseObjects * sizeof(uint2));
         if (e == hipSuccess) e = hipMalloc((void**)&s.err, 16);
         if (e == hipSuccess) e = hipMemset(s.err, 0, 16);
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // cleared before a launch on any stream
         if (e != hipSuccess) {
-            for (void* p : { (void*)s.fuse, (void*)s.err })
+            for (void* p : { (void*)s.fuse, (void*)s.fuse_left, (void*)s.err })
                 if (p) (void)hipFree(p);
             s.fuse = nullptr;
+            s.fuse_left = nullptr;
             s.err = nullptr;
             return hip_fail(e, "stream words");
         }
@@ -1023,7 +1025,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
             StreamScratch* sc = nullptr;
             s = words_for(st, &sc);
             if (s) return s;
-            e = launch_late_fused(job, d, sc->fuse, sc->err, st);
+            e = launch_late_fused(job, d, sc->fused(), wait_limit, st);
         } else {
             s = compact(job.n_tiles, (uint64_t)job.n_tiles * fc.block * fc.items, &cs);
             if (s) return s;
@@ -1039,7 +1041,7 @@ bz_status Ctx::cull(const bz_cull_args* a, hipStream_t st, const CompactScratch*
     else s = compact(job.n_tiles, (uint64_t)job.n_tiles * t.block * t.items, &cs);
     if (s) return s;
     auto launch = [&](const FrameCacheDev* d) {
-        return fuse ? launch_fused(job, fuse->fuse, fuse->err, st, d)
+        return fuse ? launch_fused(job, fuse->fused(), wait_limit, st, d)
                     : launch_cull(job, cs, t.block, t.items, n_cu, t.grid_per_cu, st, d);
     };
     if (cache && job.pass == PASS_EARLY) {
@@ -1252,7 +1254,7 @@ bz_status bz_cull_clusters(bz_ctx* ctx, const bz_cluster_cull_args* a, void* str
     cj.n_tiles = oj.n_tiles;
     cj.tile_size = t.block * t.items;
     hipError_t e = launch_cluster_objects(oj, sc->cs, sc->xs.ccounts, t.block, t.items, st);
-    if (e == hipSuccess) e = launch_cluster_pass(cj, sc->cs, sc->xs, sc->fuse, sc->err, st);
+    if (e == hipSuccess) e = launch_cluster_pass(cj, sc->cs, sc->xs, sc->fused(), ctx->wait_limit, st);
     if (e != hipSuccess) return ctx->hip_fail(e, "cluster cull launch");
     return BZ_OK;
 }
@@ -1392,7 +1394,8 @@ bz_status bz_check(bz_ctx* ctx, void* stream)
         if (e == hipSuccess && g.second->launched && g.second->last_stream == st) e = read_flags(g.second->err);
     if (e != hipSuccess) return ctx->hip_fail(e, "error flag read");
     if (flags[0]) {
-        // A workgroup of a one-launch pass that gave up may have published its count under a later launch's number
+        // One-launch passes that overlap on one stream's words (replays of a captured pass beside other passes of the
+        // stream) can also leave counts under a later launch's number: start again from zero.
         e = hipDeviceSynchronize();
         for (auto& x : ctx->scratch)
             if (e == hipSuccess && x.second->fuse) e = hipMemset(x.second->fuse, 0, kFuseWords * 8u);
@@ -1412,8 +1415,8 @@ bz_status bz_check(bz_ctx* ctx, void* stream)
     if (flags[0] || flags[1] || flags[2]) {
         if (flags[2] && !flags[0] && !flags[1])
             return ctx->fail(BZ_E_INVALID, "a staged transform update named a transform id out of range (skipped)");
-        return ctx->fail(BZ_E_INTERNAL, "a kernel gave up a bounded wait (the pyramid built then holds wrong values "
-                                        "until rebuilt)");
+        return ctx->fail(BZ_E_INTERNAL, "a kernel gave up a bounded wait (a cull's count and commands, or the pyramid "
+                                        "built then, are wrong until the call is made again)");
     }
     return BZ_OK;
 }

@@ -34,7 +34,7 @@ struct ExpandSmem {
     uint32_t obj[kXMaxTile];
     uint32_t lod[kXMaxTile];
     uint32_t coff[kXMaxTile];  // first cluster of the object's LOD
-    uint32_t red[kXWaves];
+    uint32_t red[2 * kXWaves];
     uint32_t lvl[kMaxMips];
     uint32_t last;  // FUSED: the number of the launch before
 };
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_expand_kernel(ClusterJob J, c
     // records in (objectId, clusterId) order; survivors compacted in the same order
     uint32_t surv = 0, surv0 = 0;  // survivors so far, of the first chunk
     bool keep0 = false;  // FUSED: the first chunk's record of this thread and its place among the survivors
-    uint32_t obj0 = 0, at0 = 0;
+    uint32_t obj0 = 0, cid0 = 0, at0 = 0;
     uint2 draw0 = make_uint2(0u, 0u);
     for (uint32_t r0 = 0; r0 < T; r0 += kXBlock) {
         const uint32_t r = r0 + tid;
@@ -219,6 +219,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_expand_kernel(ClusterJob J, c
         if (FUSED && r0 == 0) {
             keep0 = keep;
             obj0 = obj;
+            cid0 = cid;
             at0 = off + rank;
             if (keep) draw0 = J.cl_draw[cid];
         } else if (keep) {
@@ -233,17 +234,28 @@ __global__ __launch_bounds__(kXBlock) void cluster_expand_kernel(ClusterJob J, c
         return;
     }
     if (tid == 0) fuse_publish(fuse, launch, t, surv);
-    const uint32_t prefix = fuse_prefix<kXBlock>(fuse, launch, t, sm.red);
-    if (tid == 0 && t + 1u == J.n_tiles) {
-        *J.count = prefix + surv;
-        fuse_finish(fuse, launch);
-    }
+    const bool last_tile = t + 1u == J.n_tiles;
+    uint32_t prefix, left = 0;
+    const bool mine = fuse_prefix<kXBlock>(fuse, launch, t, last_tile, sm.red, prefix, left, [&] {
+        if (tid == 0) rbase[t] = base;
+        if (keep0) survivors[(size_t)base + at0] = make_uint2(obj0, cid0);
+    });
+    if (!mine) return;
+    if (tid == 0 && last_tile) *J.count = prefix + surv;
     if (keep0 && prefix + at0 < J.capacity) write_command(J.cmds, prefix + at0, obj0, draw0);
     // the survivors of later chunks, which are the last ones (written by this workgroup, behind a barrier)
     for (uint32_t e = surv0 + tid; e < surv; e += kXBlock) {
         const uint2 en = survivors[(size_t)base + e];
         if (prefix + e < J.capacity) write_command(J.cmds, prefix + e, en.x, J.cl_draw[en.y]);
     }
+    if (last_tile)
+        fuse_settle(fuse, launch, left, J.n_tiles, [&](uint32_t u, uint32_t first, uint32_t n) {
+            const size_t b = rbase[u];
+            for (uint32_t e = tid; e < n; e += 64u) {
+                const uint2 en = survivors[b + e];
+                if (first + e < J.capacity) write_command(J.cmds, first + e, en.x, J.cl_draw[en.y]);
+            }
+        });
 }
 
 constexpr uint32_t kCEmitTiles = kXBlock / 64;
@@ -303,7 +315,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_emit_kernel(ClusterJob J, con
 }  // namespace
 
 hipError_t launch_cluster_pass(const ClusterJob& job_in, const CompactScratch& cs, const ClusterScratch& xs,
-                               unsigned long long* words, uint32_t* err, hipStream_t st)
+                               const FuseScratch& s, uint32_t wait_limit, hipStream_t st)
 {
     if (job_in.n_tiles == 0 || job_in.tile_size > kXMaxTile) return hipErrorInvalidValue;
     ClusterJob job = job_in;
@@ -312,7 +324,7 @@ hipError_t launch_cluster_pass(const ClusterJob& job_in, const CompactScratch& c
     if (job.n_tiles <= kFuseTiles) {
         hipLaunchKernelGGL(cluster_expand_kernel<true>, g, b, 0, st, job, (const uint32_t*)cs.counts,
                            (const uint2*)cs.staging, (const uint32_t*)xs.ccounts, xs.rbase, xs.scount, xs.survivors,
-                           FuseDev{ words, err });
+                           FuseDev{ s.words, s.err, wait_limit < kFusePatience ? wait_limit : kFusePatience });
         return hipGetLastError();
     }
     hipError_t e = hipSuccess;

@@ -51,6 +51,7 @@ struct TileSmem {
     uint32_t ctot[2][BLOCK / 64];     // frame cache: per-wave totals of the survivors
     uint32_t csum[BLOCK / 64];        // cluster mode: per-wave sums of the emitting objects' cluster counts
     uint32_t last;                    // one-launch passes: the number of the launch before
+    uint32_t red[2 * (BLOCK / 64)];   // and the reduction of the earlier tiles' counts
 };
 
 // Pass families compiled separately so the visibility stream is loaded unconditionally where it is used.
@@ -216,13 +217,26 @@ struct NoPrefetch {
     __device__ __forceinline__ void operator()() const {}
 };
 
+// By the last tile of a one-launch pass: the commands of the tiles that left theirs, as (objectId, LOD) entries.
+__device__ __forceinline__ void settle_staged(const CullJob& J, uint32_t tile_size, const uint2* staging, const FuseDev& fuse,
+                                              uint32_t launch, uint32_t left)
+{
+    fuse_settle(fuse, launch, left, J.n_tiles, [&](uint32_t t, uint32_t first, uint32_t n) {
+        for (uint32_t e = threadIdx.x; e < n; e += 64u) {
+            const uint2 en = staging[(size_t)t * tile_size + e];
+            if (first + e < J.capacity) write_command(J.cmds, first + e, en.x, J.scene.lod_draw[en.y]);
+        }
+    });
+}
+
 // Decides one tile whose streams are in `s` (the decide kernel's body). Called by all threads of the workgroup.
 // `prefetch` is invoked once, after the tile's last global gather (the Hi-Z texels), so loads it issues stay in
 // flight through the rest of the tile (vmcnt retires in issue order: nothing later waits on them).
 // CL (cluster object pass): ccounts[gtile] also receives the sum of the emitting objects' LOD cluster counts.
 // CACHE (EARLY with all streams loaded): every frustum survivor of the tile is recorded in the frame cache `fc`.
 // INST (LOD-instanced output): each emitting object also adds 1 to its LOD's bin of the workgroup's LDS histogram.
-// FUSED (one tile per workgroup): the tile's commands are written here (fuse_emit) and not staged for an emit launch.
+// FUSED (one tile per workgroup): the tile's commands are written here and not staged for an emit launch (staged only
+// where the tile leaves them to the last one).
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool LDS_TAB, bool CL = false, bool CACHE = false, bool INST = false,
           bool FUSED = false, class Prefetch>
 __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_job, uint32_t gtile, uint32_t parity,
@@ -434,16 +448,22 @@ __device__ __forceinline__ void process_tile(const CullJob& J, uint32_t tile_in_
         uint2 d[ITEMS];
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) d[k] = emit[k] ? S.lod_draw[lod_abs[k]] : make_uint2(0u, 0u);
-        const uint32_t prefix = fuse_prefix<BLOCK>(fuse, launch, gtile, sm.wtot[parity ^ 1u]);
-        if (tid == 0 && gtile + 1u == J.n_tiles) {
-            *J.count = prefix + total;
-            fuse_finish(fuse, launch);
-        }
+        const bool last_tile = gtile + 1u == J.n_tiles;
+        uint32_t prefix, left = 0;
+        const bool mine = fuse_prefix<BLOCK>(fuse, launch, gtile, last_tile, sm.red, prefix, left, [&] {
+            uint2* stage = staging + (size_t)gtile * TILE + before;
+#pragma unroll
+            for (int k = 0; k < ITEMS; ++k)
+                if (emit[k]) stage[CACHE ? erank[k] : eslot[k]] = make_uint2(J.begin + i0 + 64u * k, lod_abs[k]);
+        });
+        if (!mine) return;
+        if (tid == 0 && last_tile) *J.count = prefix + total;
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k) {
             const uint32_t pos = prefix + before + (CACHE ? erank[k] : eslot[k]);
             if (emit[k] && pos < J.capacity) write_command(J.cmds, pos, J.begin + i0 + 64u * k, d[k]);
         }
+        if (last_tile) settle_staged(J, TILE, staging, fuse, launch, left);
     }
 }
 
@@ -526,7 +546,7 @@ __global__ __launch_bounds__(BLOCK) void decide_kernel(CullJob J, uint32_t* coun
 // EARLY too (the visibility's round trip costs more than the other objects' bytes here); the tables are read from global
 // memory, as for the batches.
 template <int BLOCK, int ITEMS, int MODE, bool HIZ, bool CACHE>
-__global__ __launch_bounds__(BLOCK) void fused_kernel(CullJob J, FrameCacheDev fc, FuseDev fuse)
+__global__ __launch_bounds__(BLOCK) void fused_kernel(CullJob J, FrameCacheDev fc, uint2* left, FuseDev fuse)
 {
     __shared__ TileSmem<BLOCK, ITEMS, false> sm;
     const uint32_t last = fuse_last(fuse);  // (no branch: its wait comes behind the streams' loads)
@@ -537,7 +557,7 @@ __global__ __launch_bounds__(BLOCK) void fused_kernel(CullJob J, FrameCacheDev f
     __syncthreads();
     const uint32_t launch = fuse_launch(sm.last);
     process_tile<BLOCK, ITEMS, MODE, HIZ, false, false, CACHE, false, true>(
-        J, blockIdx.x, blockIdx.x, 0u, s, nullptr, nullptr, nullptr, sm, NoPrefetch{}, fc, nullptr, fuse, launch);
+        J, blockIdx.x, blockIdx.x, 0u, s, nullptr, left, nullptr, sm, NoPrefetch{}, fc, nullptr, fuse, launch);
 }
 
 // Last entry of the ascending table `starts` that is <= t.
@@ -918,7 +938,7 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
                                                              uint2* staging, FuseDev fuse)
 {
     constexpr uint32_t NW = kLtBlock / 64, ROUNDS = TILE / kLtBlock;
-    __shared__ uint32_t s_new[TILE / 32], s_lvl[kMaxMips], s_tot[ROUNDS][NW], s_red[NW], s_last;
+    __shared__ uint32_t s_new[TILE / 32], s_lvl[kMaxMips], s_tot[ROUNDS][NW], s_red[2 * NW], s_last;
     const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t base = t * TILE, nt = J.n - base < TILE ? J.n - base : TILE, obj0 = J.begin + base;
     const uint32_t last = FUSED ? fuse_last(fuse) : 0u;
@@ -937,13 +957,11 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
     const uint32_t launch = FUSED ? fuse_launch(s_last) : 0u;
     uint32_t before = 0;      // the tile's commands of the rounds so far
     bool emit[ROUNDS];        // FUSED: a round's commands wait for the tile's first slot
-    uint32_t rank[ROUNDS], obj[ROUNDS];
-    uint2 d[ROUNDS];
+    uint32_t rank[ROUNDS], obj[ROUNDS], lod[ROUNDS];
 #pragma unroll
     for (uint32_t r = 0; r < ROUNDS; ++r) {
         emit[r] = false;
-        rank[r] = obj[r] = 0u;
-        d[r] = make_uint2(0u, 0u);
+        rank[r] = obj[r] = lod[r] = 0u;
         if (r * kLtBlock < n) {  // uniform
             const uint32_t e = r * kLtBlock + tid;
             if (r) {
@@ -963,7 +981,7 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
             const unsigned long long m = __ballot(emit[r]);
             rank[r] = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
             obj[r] = mt.x;
-            d[r].x = mt.y;
+            lod[r] = mt.y;
             if (lane == 0) s_tot[r][wave] = (uint32_t)__popcll(m);
             __syncthreads();
             uint32_t total = 0;
@@ -976,7 +994,7 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
             rank[r] += before;
             before += total;
             if constexpr (!FUSED)
-                if (emit[r]) staging[(size_t)t * TILE + rank[r]] = make_uint2(obj[r], d[r].x);
+                if (emit[r]) staging[(size_t)t * TILE + rank[r]] = make_uint2(obj[r], lod[r]);
         }
     }
     if (n == 0) __syncthreads();  // (s_new cleared; with survivors a round's barrier has followed its last bit)
@@ -997,19 +1015,24 @@ __global__ __launch_bounds__(kLtBlock) void late_tile_kernel(CullJob J, FrameCac
             __builtin_nontemporal_store((s_new[i >> 5] >> (i & 31u)) & 1u, J.vis_out + obj0 + i);
     }
     if constexpr (FUSED) {
+        uint2 d[ROUNDS];
 #pragma unroll
-        for (uint32_t r = 0; r < ROUNDS; ++r)
-            if (emit[r]) d[r] = J.scene.lod_draw[d[r].x];
-        const uint32_t prefix = fuse_prefix<kLtBlock>(fuse, launch, t, s_red);
-        if (tid == 0 && t + 1u == J.n_tiles) {
-            *J.count = prefix + before;
-            fuse_finish(fuse, launch);
-        }
+        for (uint32_t r = 0; r < ROUNDS; ++r) d[r] = emit[r] ? J.scene.lod_draw[lod[r]] : make_uint2(0u, 0u);
+        const bool last_tile = t + 1u == J.n_tiles;
+        uint32_t prefix, left = 0;
+        const bool mine = fuse_prefix<kLtBlock>(fuse, launch, t, last_tile, s_red, prefix, left, [&] {
+#pragma unroll
+            for (uint32_t r = 0; r < ROUNDS; ++r)
+                if (emit[r]) staging[(size_t)t * TILE + rank[r]] = make_uint2(obj[r], lod[r]);
+        });
+        if (!mine) return;
+        if (tid == 0 && last_tile) *J.count = prefix + before;
 #pragma unroll
         for (uint32_t r = 0; r < ROUNDS; ++r) {
             const uint32_t pos = prefix + rank[r];
             if (emit[r] && pos < J.capacity) write_command(J.cmds, pos, obj[r], d[r]);
         }
+        if (last_tile) settle_staged(J, TILE, staging, fuse, launch, left);
     }
 }
 
@@ -1096,11 +1119,17 @@ hipError_t launch_cull_t(const CullJob& job, const CompactScratch& s, uint32_t n
     return launch_emit(job, (uint32_t)(BLOCK * ITEMS), s, st);
 }
 
-hipError_t launch_fused_t(const CullJob& job, const FrameCacheDev& fc, bool record, const FuseDev& f, hipStream_t st)
+FuseDev fuse_dev(const FuseScratch& s, uint32_t wait_limit)
+{
+    return FuseDev{ s.words, s.err, wait_limit < kFusePatience ? wait_limit : kFusePatience };
+}
+
+hipError_t launch_fused_t(const CullJob& job, const FrameCacheDev& fc, bool record, uint2* left, const FuseDev& f,
+                          hipStream_t st)
 {
     const dim3 g(job.n_tiles), b(kFuseBlock);
 #define BZ_FUSED(M, HZ, CA) \
-    hipLaunchKernelGGL((fused_kernel<kFuseBlock, kFuseItems, M, HZ, CA>), g, b, 0, st, job, fc, f)
+    hipLaunchKernelGGL((fused_kernel<kFuseBlock, kFuseItems, M, HZ, CA>), g, b, 0, st, job, fc, left, f)
     const bool h = job.hiz != 0;
     if (job.pass == PASS_EARLY && record) {
         if (h) BZ_FUSED(MODE_EARLY, true, true);
@@ -1172,11 +1201,11 @@ hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t blo
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_fused(const CullJob& job, unsigned long long* words, uint32_t* err, hipStream_t st,
+hipError_t launch_fused(const CullJob& job, const FuseScratch& s, uint32_t wait_limit, hipStream_t st,
                         const FrameCacheDev* cache)
 {
     const FrameCacheDev fc = cache ? *cache : FrameCacheDev{};
-    return launch_fused_t(job, fc, cache != nullptr, FuseDev{ words, err }, st);
+    return launch_fused_t(job, fc, cache != nullptr, s.left, fuse_dev(s, wait_limit), st);
 }
 
 hipError_t launch_decide_only(const CullJob& job, const CompactScratch& s, uint32_t block, uint32_t items,
@@ -1216,11 +1245,11 @@ void decide_inst_chunks(const CullJob& job, uint32_t block, uint32_t items, uint
     }
 }
 
-hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, unsigned long long* words, uint32_t* err,
+hipError_t launch_late_fused(const CullJob& job, const FrameCacheDev& cache, const FuseScratch& s, uint32_t wait_limit,
                              hipStream_t st)
 {
     hipLaunchKernelGGL((late_tile_kernel<kFuseBlock * kFuseItems, true>), dim3(job.n_tiles), dim3(kLtBlock), 0, st, job,
-                       cache, (uint32_t*)nullptr, (uint2*)nullptr, FuseDev{ words, err });
+                       cache, (uint32_t*)nullptr, s.left, fuse_dev(s, wait_limit));
     return hipGetLastError();
 }
 

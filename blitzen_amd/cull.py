@@ -117,7 +117,7 @@ class Context:
         self.check(lib().bz_check(self.handle, stream), "bz_check")
 
     def set_wait_limit(self, sleeps: int):
-        """Sleeps a kernel's bounded wait may take before giving up (pyramid builds launched afterwards)."""
+        """Sleeps a kernel's bounded wait may take before giving up (launches made afterwards)."""
         self.check(lib().bz_set_wait_limit(self.handle, sleeps), "bz_set_wait_limit")
 
     def stream(self):

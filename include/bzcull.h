@@ -265,7 +265,8 @@ typedef struct bz_cull_args {
 /* One cull pass on `stream`. Replaces one vkCmdFillBuffer(count, 0) + vkCmdDispatch(N/64+1) of
  * DrawCullFirstPass / DrawCullOcclusionPass (vulkanDraw.cpp:119,145,180,213). Commands are written at
  * cmds_dev[0..min(count, capacity)); *count_dev = number of emitted commands. Overflow is detected by
- * the caller as *count_dev > capacity. */
+ * the caller as *count_dev > capacity.
+ * A pass captured from `stream` keeps that stream's scratch: order its replays with the stream's other passes. */
 BZ_API bz_status bz_cull(bz_ctx* ctx, const bz_cull_args* args, void* stream);
 
 /* bz_cull without any device allocation. No counterpart in the reference: it is for callers that cannot allocate
@@ -372,7 +373,8 @@ typedef struct bz_tuning {
  * capture a fixed batch with bz_batch_graph_create instead. Jobs that write one visibility buffer in overlapping ranges race. */
 BZ_API bz_status bz_cull_batch(bz_ctx* ctx, const bz_view_job* jobs, uint32_t n_jobs, void* stream);
 /* Synchronizes `stream` and reports BZ_E_INTERNAL if a kernel launched on it gave up a bounded wait
- * since the last check (the flag is then cleared). A pyramid build whose tail workgroup gave up waiting for a
+ * since the last check (the flag is then cleared): a pyramid build, the scan of bz_cull_instanced, or a bz_cull or
+ * bz_cull_clusters that runs in one launch (its count and commands are then wrong; run it again). A pyramid build whose tail workgroup gave up waiting for a
  * tile's hand-off word can leave such words set by tiles that finished later: the check then also waits for the
  * device and clears the hand-off words of every pyramid of the context, so the next build of each is correct
  * (the pyramid that was being built holds wrong values until rebuilt). */
@@ -381,6 +383,9 @@ BZ_API bz_status bz_check(bz_ctx* ctx, void* stream);
  * gives up; 0 gives up at the first word not yet handed over. Applies to launches made afterwards through this
  * context: pyramid builds (bz_pyramid_build, bz_pyramid_build_batch, bz_batch_graph_create) and the scan of
  * bz_cull_instanced. Default BZ_DEFAULT_WAIT_LIMIT.
+ * In a bz_cull or bz_cull_clusters that runs in one launch, a workgroup that waits longer than this (or than 4096
+ * sleeps) leaves its commands to the launch's last workgroup, with the same results; only that one's own wait, always
+ * of BZ_DEFAULT_WAIT_LIMIT, can be given up.
  * A small limit forces the give-up path for tests of the error handling; with the default the waits end in a few
  * microseconds. */
 #define BZ_DEFAULT_WAIT_LIMIT 1048576u
