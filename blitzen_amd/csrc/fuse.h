@@ -2,6 +2,7 @@
 // the counts that workgroups publish for the ones after them.
 #pragma once
 #include "bz_internal.h"
+#include "fuse_words.h"
 
 namespace bz {
 
@@ -14,7 +15,7 @@ __device__ __forceinline__ void write_command(uint32_t* cmds, uint32_t pos, uint
 }
 
 // The words that a launch's workgroups hand each other, each with the launch's number above its value: a word of another
-// launch is not taken, so nothing is cleared between launches.
+// launch is not taken, so nothing is cleared between launches (fuse_words.h).
 struct FuseDev {
     unsigned long long* words;  // [0] number of the last launch, [1] of the last one in which a tile left its commands
                                 // (32 bits each), [kFuseFirst + tile] the tiles' command counts, [kFuseFirst + kFuseTiles +
@@ -153,14 +154,15 @@ __device__ __forceinline__ uint32_t fuse_last(const FuseDev& fuse)
 }
 __device__ __forceinline__ uint32_t fuse_launch(uint32_t last)  // this launch's number
 {
-    return __builtin_amdgcn_readfirstlane(last) + 1u;
+    return fuse_next(__builtin_amdgcn_readfirstlane(last));
 }
 __device__ __forceinline__ void fuse_publish(const FuseDev& fuse, uint32_t launch, uint32_t tile, uint32_t count)
 {
     fuse_store(fuse, kFuseFirst + tile, launch, count);
 }
 // By the last tile, which has had every count: its first wave writes the commands of the tiles that left theirs
-// (write(tile, first command, commands), 64 lanes) and moves the launch's number on, which each workgroup has read.
+// (write(tile, first command, commands), 64 lanes), ages a word and moves the launch's number on, which each workgroup has
+// read.
 template <class Write>
 __device__ __forceinline__ void fuse_settle(const FuseDev& fuse, uint32_t launch, uint32_t left, uint32_t n_tiles,
                                             Write&& write)
@@ -179,8 +181,11 @@ __device__ __forceinline__ void fuse_settle(const FuseDev& fuse, uint32_t launch
             first += count;
         }
     }
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
+        const uint32_t aged = fuse_aged(launch, kFuseTiles);
+        if (aged >= n_tiles) fuse_store(fuse, kFuseFirst + aged, 0u, 0u);
         __hip_atomic_store(reinterpret_cast<uint32_t*>(fuse.words), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 }  // namespace bz
