@@ -156,17 +156,23 @@ bz_status Ctx::scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, Str
     return BZ_OK;
 }
 
-// The stream's words for a pass in one launch. A stream under capture whose first call this is has none yet.
+// The stream's words for a pass in one launch. A stream under capture whose first call this is has none yet. Outside a
+// capture, the first such pass also takes the least compaction scratch, as every other first pass does: one small pass is
+// enough before a pass of up to 2^20 objects is captured.
 bz_status Ctx::words_for(hipStream_t st, StreamScratch** out)
 {
     const auto it = scratch.find((uintptr_t)st);
-    if (it == scratch.end() || !it->second || !it->second->fuse) {
-        hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cst) == hipSuccess && cst != hipStreamCaptureStatusNone)
-            return fail(BZ_E_STATE, "the stream's words must be allocated, which is not allowed during stream capture; "
-                                    "run the call once before capturing");
+    const bool words = it != scratch.end() && it->second && it->second->fuse;
+    if (words && it->second->cs.capacity_tiles) {
+        *out = it->second.get();
+        return BZ_OK;
     }
-    return scratch_for(st, 0, 0, out);
+    hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
+    const bool capturing = hipStreamIsCapturing(st, &cst) == hipSuccess && cst != hipStreamCaptureStatusNone;
+    if (capturing && !words)
+        return fail(BZ_E_STATE, "the stream's words must be allocated, which is not allowed during stream capture; "
+                                "run the call once before capturing");
+    return scratch_for(st, capturing ? 0u : 1u, capturing ? 0u : 1u, out);
 }
 
 // Cluster-pass scratch: per-tile arrays for `tiles` object tiles and a survivor buffer of `records` entries.
