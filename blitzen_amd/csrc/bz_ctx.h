@@ -25,7 +25,11 @@ struct Scene {
     float4* xf_ps = nullptr;
     float4* xf_q = nullptr;
     float4* world = nullptr;           // world-space bounding spheres' centres and the scale, per object
-    uint8_t* xf_stamp = nullptr;       // [n_transforms] xf_version (mod 255, + 1) of each one's last update (obj_xf)
+    uint32_t *xf_first = nullptr, *xf_objs = nullptr;  // obj_xf: each transform's objects (XfTarget)
+    XfChunk* xf_chunks = nullptr;
+    uint32_t n_xf_chunks = 0, xf_per_block = 256;
+    hipError_t list_objects();
+    uint8_t* xf_stamp = nullptr;       // [n_transforms] xf_version (mod 255, + 1) of the last update (with xf_chunks)
     float4* surf_sphere = nullptr;
     uint2* surf_lod = nullptr;
     float* lod_error = nullptr;

@@ -245,13 +245,34 @@ hipError_t launch_pyramid_region(const PyrBuildJob& job, uint32_t* err, hipStrea
 hipError_t launch_pyramid_level(const float* src, uint32_t sw, uint32_t sh, float* dst, uint32_t dw, uint32_t dh,
                                 hipStream_t st);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t st);
+// The objects that use a transform follow its updates in the launch that scatters them, except lists so long that one would
+// keep a workgroup busy: those are cut into pieces, for a launch of their own.
+constexpr uint32_t kXfChunk = 256;
+struct XfChunk {
+    uint32_t xf, begin, end;    // objs[begin, end) use transform xf
+};
+constexpr uint32_t xf_inline(uint32_t per_block) { return per_block > 16u ? 16384u / per_block : 1024u; }
+constexpr uint64_t xf_pieces_most(uint64_t n_objects) { return n_objects / 65u + n_objects / kXfChunk + 1u; }
+// first[n_xf + 1], objs[n]: the lists. work: n_xf + 1 words; work[n_xf] = lists that are not empty.
+hipError_t launch_list_objects(const uint32_t* obj_xf, uint32_t n, uint32_t n_xf, uint32_t* work, uint32_t* first,
+                               uint32_t* objs, hipStream_t st);
+// The lists of more than `most` objects (64 at least), in pieces; *n_chunks: their number.
+hipError_t launch_list_chunks(const uint32_t* first, uint32_t n_xf, uint32_t most, XfChunk* chunks, uint32_t* n_chunks,
+                              hipStream_t st);
 // Where a transform update writes: the transform streams, and what of the objects' world-space spheres follows from
 // them.
 struct XfTarget {
     SceneDev scene;
     float4 *xf_ps, *xf_q, *world;
     uint32_t* winner;           // [n_transforms] zero before and after the launches
-    uint8_t* stamp;             // [n_transforms] the last update of each transform (scenes with obj_xf; else nullptr)
+    // scenes with obj_xf: the objects that use transform t are objs[first[t], first[t + 1])
+    const uint32_t* first;      // [n_transforms + 1]
+    const uint32_t* objs;       // [n_objects]
+    // and the lists of more than xf_inline(per_block) objects, in pieces
+    const XfChunk* chunks;      // [n_chunks]
+    uint32_t n_chunks;
+    uint32_t per_block;         // updates per workgroup of 256 threads
+    uint8_t* stamp;             // [n_transforms] the last update of each of those (nullptr without chunks)
     uint8_t version;            // this update's stamp (not 0)
 };
 // Staged updates: ids[i] and the 32-byte MeshTransform record i (pos.xyz, scale | quaternion) scattered into the SoA

@@ -1419,41 +1419,135 @@ __device__ __forceinline__ float4 object_surface(const SceneDev& S, uint32_t obj
     return S.surf_sphere[S.obj_surf16 ? (uint32_t)S.obj_surf16[obj] : S.obj_surf[obj]];
 }
 
+// The spheres of the objects that use the workgroup's updated transforms (scenes with obj_xf): thread i's transform is used
+// by `len` objects, listed from objs[first]. The lists, end to end, are dealt to the threads, so that one of many objects does
+// not hold a thread up; four objects of a thread in flight. An update then costs what it moves: a launch that looked at the
+// stamp of every object's transform instead took, for 41 943 of 4 194 304 transforms in random order, 31 us besides.
+struct SpreadSmem {
+    float4 ps[256], q[256];
+    uint32_t end[256], off[256];  // of each list: its end in the sequence, and what takes a place in it to its index in objs
+    uint32_t wsum[4];
+};
+__device__ __forceinline__ void spread_spheres(const XfTarget& to, uint32_t first, uint32_t len, const float4& ps,
+                                               const float4& q, SpreadSmem& sm)
+{
+    constexpr uint32_t U = 4;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    uint32_t end = wave_incl_scan(len, tid & 63u);
+    if ((tid & 63u) == 63u) sm.wsum[wave] = end;
+    sm.ps[tid] = ps;
+    sm.q[tid] = q;
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; ++w) end += sm.wsum[w];
+    sm.end[tid] = end;
+    sm.off[tid] = first - (end - len);
+    __syncthreads();
+    const uint32_t total = sm.end[255];
+    for (uint32_t r0 = 0; r0 < total; r0 += U * 256u) {
+        uint32_t j[U], obj[U];
+        float4 sph[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t r = r0 + u * 256u + tid;
+            j[u] = 0;  // the first list that ends behind r
+#pragma unroll
+            for (uint32_t step = 128; step; step >>= 1)
+                if (sm.end[j[u] + step - 1u] <= r) j[u] += step;
+            obj[u] = r < total ? to.objs[sm.off[j[u]] + r] : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) sph[u] = object_surface(to.scene, obj[u]);
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (r0 + u * 256u + tid < total) to.world[obj[u]] = world_sphere(sph[u], sm.ps[j[u]], sm.q[j[u]]);
+    }
+}
+// The list of an updated transform; a long one is left to the next launch.
+__device__ __forceinline__ void spread_list(const XfTarget& to, uint32_t id, bool updated, uint32_t& first, uint32_t& len)
+{
+    first = updated ? to.first[id] : 0u;
+    len = updated ? to.first[id + 1u] - first : 0u;
+    if (len > xf_inline(to.per_block)) {
+        to.stamp[id] = to.version;
+        len = 0u;
+    }
+}
+
+template <bool SHARED>
 __global__ __launch_bounds__(256) void scatter_staged_transforms_kernel(const uint32_t* __restrict__ dev_ids,
                                                                         const float4* __restrict__ records, uint32_t n,
                                                                         XfTarget to)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = dev_ids[i];
-    if (id >= to.scene.n_transforms || to.winner[id] != i + 1u) return;
-    const bool sphere = !to.scene.obj_xf && id < to.scene.n_objects;
-    const float4 sph = sphere ? object_surface(to.scene, id) : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 ps = records[2u * i], q = records[2u * i + 1u];
-    to.xf_ps[id] = ps;
-    to.xf_q[id] = q;
-    to.winner[id] = 0u;
-    if (sphere) to.world[id] = world_sphere(sph, ps, q);
-    else if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
+    if constexpr (SHARED) {
+        __shared__ SpreadSmem sm;
+        const uint32_t i = blockIdx.x * to.per_block + threadIdx.x;
+        const uint32_t id = threadIdx.x < to.per_block && i < n ? dev_ids[i] : 0xffffffffu;
+        const bool wins = id < to.scene.n_transforms && to.winner[id] == i + 1u;
+        float4 ps = make_float4(0.f, 0.f, 0.f, 0.f), q = ps;
+        if (wins) {
+            ps = records[2u * i];
+            q = records[2u * i + 1u];
+        }
+        uint32_t first, len;
+        spread_list(to, id, wins, first, len);  // (its loads behind the records')
+        if (wins) {
+            to.xf_ps[id] = ps;
+            to.xf_q[id] = q;
+            to.winner[id] = 0u;
+        }
+        spread_spheres(to, first, len, ps, q, sm);
+    } else {
+        const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+        if (i >= n) return;
+        const uint32_t id = dev_ids[i];
+        if (id >= to.scene.n_transforms || to.winner[id] != i + 1u) return;
+        const bool sphere = id < to.scene.n_objects;
+        const float4 sph = sphere ? object_surface(to.scene, id) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 ps = records[2u * i], q = records[2u * i + 1u];
+        to.xf_ps[id] = ps;
+        to.xf_q[id] = q;
+        to.winner[id] = 0u;
+        if (sphere) to.world[id] = world_sphere(sph, ps, q);
+    }
 }
 
 // Updates that name every id once (and in range), up to kDistinctUpdates of them: straight from the pinned slot to the
 // streams in one launch. Calls with 4096 updates 11.5 us against 14.3 in two launches, 10 485 16.2 against 18.6, 16 384 21.1
 // against 22.8, 24 576 27.7 against 28.7, but 41 943 51.5 against 39.1: ids and records read over the link at once slow each
 // other down when there are many.
+template <bool SHARED>
 __global__ __launch_bounds__(256) void scatter_distinct_transforms_kernel(const uint32_t* __restrict__ ids,
                                                                           const float4* __restrict__ records,
                                                                           uint32_t n, XfTarget to)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = ids[i];
-    const float4 ps = records[2u * i], q = records[2u * i + 1u];
-    if (id >= to.scene.n_transforms) return;  // (the caller has looked: only a caller's race on its ids gets here)
-    to.xf_ps[id] = ps;
-    to.xf_q[id] = q;
-    if (to.scene.obj_xf) to.stamp[id] = to.version;  // its objects follow in the next launch
-    else if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), ps, q);
+    if constexpr (SHARED) {
+        __shared__ SpreadSmem sm;
+        const uint32_t i = blockIdx.x * to.per_block + threadIdx.x;
+        const bool mine = threadIdx.x < to.per_block && i < n;
+        const uint32_t id = mine ? ids[i] : 0xffffffffu;
+        float4 ps = make_float4(0.f, 0.f, 0.f, 0.f), q = ps;
+        if (mine) {
+            ps = records[2u * i];
+            q = records[2u * i + 1u];
+        }
+        uint32_t first, len;
+        const bool valid = id < to.scene.n_transforms;
+        spread_list(to, id, valid, first, len);
+        if (valid) {
+            to.xf_ps[id] = ps;
+            to.xf_q[id] = q;
+        }
+        spread_spheres(to, first, len, ps, q, sm);
+    } else {
+        const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+        if (i >= n) return;
+        const uint32_t id = ids[i];
+        const float4 ps = records[2u * i], q = records[2u * i + 1u];
+        if (id >= to.scene.n_transforms) return;  // (the caller has looked: only a caller's race on its ids gets here)
+        to.xf_ps[id] = ps;
+        to.xf_q[id] = q;
+        if (id < to.scene.n_objects) to.world[id] = world_sphere(object_surface(to.scene, id), ps, q);
+    }
 }
 
 // World-space spheres of all the scene's objects.
@@ -1465,27 +1559,112 @@ __global__ __launch_bounds__(256) void world_spheres_kernel(SceneDev S, float4* 
     world[i] = world_sphere(object_surface(S, i), S.xf_ps[x], S.xf_q[x]);
 }
 
-// The spheres of the objects whose transform carries the stamp of the update just scattered. By object, so that the cost
-// does not depend on how many share one transform (a list of objects per transform would be walked serially by the
-// transform's thread). Nearly all of the work is looking at the stamps, one gather per object: a byte each, so that
-// they stay in the L2s, four in flight per thread (update of 41 943 of 4 194 304 transforms in random order 99 us with
-// 32-bit stamps and one object per thread, 69 now; of 10 485 of 1 048 576 23.3, 22.9).
-constexpr uint32_t kStampItems = 4;
-__global__ __launch_bounds__(256) void stamped_spheres_kernel(SceneDev S, float4* __restrict__ world,
-                                                              const uint8_t* __restrict__ stamp, uint8_t version)
+// The spheres of the objects of a transform that many use, a wave per piece of at most kXfChunk of them: those whose
+// transform carries the stamp of the update just scattered.
+__global__ __launch_bounds__(256) void chunk_spheres_kernel(XfTarget to)
 {
-    const uint32_t i0 = blockIdx.x * 256u * kStampItems + threadIdx.x;
-    uint32_t x[kStampItems];
-    bool hit[kStampItems];
+    const uint32_t c = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (c >= to.n_chunks) return;
+    const XfChunk ck = to.chunks[c];
+    if (to.stamp[ck.xf] != to.version) return;
+    const float4 ps = to.xf_ps[ck.xf], q = to.xf_q[ck.xf];
+    constexpr uint32_t U = kXfChunk / 64u;
+    uint32_t obj[U];
+    float4 sph[U];
 #pragma unroll
-    for (uint32_t k = 0; k < kStampItems; ++k) x[k] = i0 + k * 256u < S.n_objects ? S.obj_xf[i0 + k * 256u] : 0u;
-#pragma unroll
-    for (uint32_t k = 0; k < kStampItems; ++k) hit[k] = stamp[x[k]] == version;
-#pragma unroll
-    for (uint32_t k = 0; k < kStampItems; ++k) {
-        const uint32_t i = i0 + k * 256u;
-        if (hit[k] && i < S.n_objects) world[i] = world_sphere(object_surface(S, i), S.xf_ps[x[k]], S.xf_q[x[k]]);
+    for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t k = ck.begin + u * 64u + lane;
+        obj[u] = to.objs[k < ck.end ? k : ck.begin];
     }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) sph[u] = object_surface(to.scene, obj[u]);
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+        if (ck.begin + u * 64u + lane < ck.end) to.world[obj[u]] = world_sphere(sph[u], ps, q);
+}
+
+// Adds 1 to counter[x] for every active lane and gives each lane the count before it. The lanes of the first two transforms
+// met are added together: where one transform is many objects', they would otherwise queue up at its counter.
+__device__ __forceinline__ uint32_t count_up(uint32_t* counter, uint32_t x, bool active)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t place = 0;
+    for (uint32_t round = 0; round < 2u; ++round) {
+        const unsigned long long todo = __ballot(active);
+        if (!todo) return place;
+        const uint32_t x0 = __shfl(x, __ffsll(todo) - 1, 64);
+        const unsigned long long same = __ballot(active && x == x0);
+        uint32_t base = 0;
+        if (lane == (uint32_t)__ffsll(same) - 1u) base = atomicAdd(&counter[x0], (uint32_t)__popcll(same));
+        base = __shfl(base, __ffsll(same) - 1, 64);
+        if (active && x == x0) {
+            place = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            active = false;
+        }
+    }
+    return active ? atomicAdd(&counter[x], 1u) : place;
+}
+
+__global__ __launch_bounds__(256) void list_count_kernel(const uint32_t* __restrict__ obj_xf, uint32_t n, uint32_t* counts)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    count_up(counts, i < n ? obj_xf[i] : 0u, i < n);
+}
+
+__global__ __launch_bounds__(256) void list_fill_kernel(const uint32_t* __restrict__ obj_xf, uint32_t n, uint32_t* next,
+                                                        uint32_t* __restrict__ objs)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t place = count_up(next, i < n ? obj_xf[i] : 0u, i < n);
+    if (i < n) objs[place] = i;
+}
+
+// next[t] = first[t], the number of lists that are not empty
+__global__ __launch_bounds__(256) void list_start_kernel(const uint32_t* __restrict__ first, uint32_t n_xf, uint32_t* next,
+                                                         uint32_t* used)
+{
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t < n_xf) next[t] = first[t];
+    const unsigned long long m = __ballot(t < n_xf && first[t + 1u] != first[t]);
+    if ((threadIdx.x & 63u) == 0 && m) atomicAdd(used, (uint32_t)__popcll(m));
+}
+
+__global__ __launch_bounds__(256) void list_chunks_kernel(const uint32_t* __restrict__ first, uint32_t n_xf, uint32_t most,
+                                                          XfChunk* __restrict__ chunks, uint32_t* n_chunks)
+{
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= n_xf) return;
+    const uint32_t b = first[t], e = first[t + 1u];
+    if (e - b <= most) return;
+    const uint32_t n = (e - b + kXfChunk - 1u) / kXfChunk, slot = atomicAdd(n_chunks, n);
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint32_t k0 = b + k * kXfChunk;
+        chunks[slot + k] = XfChunk{ t, k0, e - k0 < kXfChunk ? e : k0 + kXfChunk };
+    }
+}
+
+hipError_t launch_list_objects(const uint32_t* obj_xf, uint32_t n, uint32_t n_xf, uint32_t* work, uint32_t* first,
+                               uint32_t* objs, hipStream_t st)
+{
+    const dim3 go((n + 255u) / 256u), gt((n_xf + 255u) / 256u), b(256);
+    hipError_t e = launch_fill_u32(work, 0u, (uint64_t)n_xf + 1u, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(list_count_kernel, go, b, 0, st, obj_xf, n, work);
+    e = launch_scan_counts(work, n_xf, first, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(list_start_kernel, gt, b, 0, st, (const uint32_t*)first, n_xf, work, work + n_xf);
+    hipLaunchKernelGGL(list_fill_kernel, go, b, 0, st, obj_xf, n, work, objs);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_chunks(const uint32_t* first, uint32_t n_xf, uint32_t most, XfChunk* chunks, uint32_t* n_chunks,
+                              hipStream_t st)
+{
+    const hipError_t e = launch_fill_u32(n_chunks, 0u, 1u, st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(list_chunks_kernel, dim3((n_xf + 255u) / 256u), dim3(256), 0, st, first, n_xf, most, chunks,
+                       n_chunks);
+    return hipGetLastError();
 }
 
 hipError_t launch_world_spheres(const SceneDev& scene, float4* world, hipStream_t st)
@@ -1499,21 +1678,24 @@ hipError_t launch_scatter_staged_transforms(const uint32_t* ids, const float4* r
                                             const XfTarget& to, uint32_t* dev_ids, uint32_t* err, hipStream_t st)
 {
     if (n == 0) return hipSuccess;
-    const dim3 g((n + 255u) / 256u), b(256);
+    const bool shared = to.scene.obj_xf != nullptr && to.scene.n_objects != 0;
+    const uint32_t per = shared ? to.per_block : 256u;
+    const dim3 g((uint32_t)(((uint64_t)n + per - 1u) / per)), g256((n + 255u) / 256u), b(256);
     if (distinct && n <= kDistinctUpdates) {
-        hipLaunchKernelGGL(scatter_distinct_transforms_kernel, g, b, 0, st, ids, records, n, to);
+        if (shared) hipLaunchKernelGGL(scatter_distinct_transforms_kernel<true>, g, b, 0, st, ids, records, n, to);
+        else hipLaunchKernelGGL(scatter_distinct_transforms_kernel<false>, g, b, 0, st, ids, records, n, to);
     } else {
-        hipLaunchKernelGGL(mark_staged_transforms_kernel, g, b, 0, st, ids, n, to.scene.n_transforms, dev_ids, to.winner,
+        hipLaunchKernelGGL(mark_staged_transforms_kernel, g256, b, 0, st, ids, n, to.scene.n_transforms, dev_ids, to.winner,
                            err);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(scatter_staged_transforms_kernel, g, b, 0, st, (const uint32_t*)dev_ids, records, n, to);
+        const uint32_t* di = dev_ids;
+        if (shared) hipLaunchKernelGGL(scatter_staged_transforms_kernel<true>, g, b, 0, st, di, records, n, to);
+        else hipLaunchKernelGGL(scatter_staged_transforms_kernel<false>, g, b, 0, st, di, records, n, to);
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !to.scene.obj_xf || to.scene.n_objects == 0) return e;
-    constexpr uint32_t per = 256u * kStampItems;
-    hipLaunchKernelGGL(stamped_spheres_kernel, dim3((to.scene.n_objects + per - 1u) / per), b, 0, st, to.scene, to.world,
-                       (const uint8_t*)to.stamp, to.version);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || to.n_chunks == 0) return e;
+    hipLaunchKernelGGL(chunk_spheres_kernel, dim3((to.n_chunks + 3u) / 4u), b, 0, st, to);
     return hipGetLastError();
 }
 
