@@ -123,7 +123,7 @@ def bench_batched(ctx, stream, steps: int, warmup: int):
     if not np.array_equal(c_graph, c_plain):
         raise RuntimeError("batched and per-view draw counts differ")
     ctx.graph_destroy(graph)
-    ctx.set_tuning(0, single_view.block, single_view.items, single_view.grid_per_cu)
+    ctx.set_tuning(0, single_view.block, single_view.items, single_view.grid_per_cu, single_view.reserved)
     n_views = len(plan)
     cmds = int(c_graph.sum())
     alg = W.algorithmic_bytes_batched(plan, cmds)

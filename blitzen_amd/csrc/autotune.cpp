@@ -2,6 +2,7 @@
 // every candidate on the caller's own jobs (every candidate gives identical results; only the time differs).
 // Results can be cached in a small JSON file keyed by device name, kernel and object-count bucket, one entry per
 // line:   "<device>|k<kernel>|b<floor(log2(objects))>": {"block": B, "items": I, "grid_per_cu": G, "us": T},
+// and "by_size": 1 behind T where the choice is the built-in one by the number of objects.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -29,9 +30,11 @@ std::map<std::string, CacheEntry> read_cache(const char* path)
     while (std::fgets(line, sizeof line, f)) {
         char key[256];
         CacheEntry e{};
-        if (std::sscanf(line, " \"%255[^\"]\": {\"block\": %u, \"items\": %u, \"grid_per_cu\": %u, \"us\": %lf}", key,
-                        &e.t.block, &e.t.items, &e.t.grid_per_cu, &e.us) == 5)
-            m[key] = e;
+        const int got = std::sscanf(line,
+                                    " \"%255[^\"]\": {\"block\": %u, \"items\": %u, \"grid_per_cu\": %u, \"us\": %lf, "
+                                    "\"by_size\": %u}",
+                                    key, &e.t.block, &e.t.items, &e.t.grid_per_cu, &e.us, &e.t.reserved);
+        if (got == 5 || got == 6) m[key] = e;
     }
     std::fclose(f);
     return m;
@@ -45,9 +48,9 @@ bool write_cache(const char* path, const std::map<std::string, CacheEntry>& m)
     std::fprintf(f, "{\n");
     size_t k = 0;
     for (const auto& kv : m) {
-        std::fprintf(f, "  \"%s\": {\"block\": %u, \"items\": %u, \"grid_per_cu\": %u, \"us\": %.3f}%s\n",
+        std::fprintf(f, "  \"%s\": {\"block\": %u, \"items\": %u, \"grid_per_cu\": %u, \"us\": %.3f%s}%s\n",
                      kv.first.c_str(), kv.second.t.block, kv.second.t.items, kv.second.t.grid_per_cu, kv.second.us,
-                     ++k < m.size() ? "," : "");
+                     kv.second.t.reserved == BZ_TUNING_BY_SIZE ? ", \"by_size\": 1" : "", ++k < m.size() ? "," : "");
     }
     std::fprintf(f, "}\n");
     const bool ok = std::fclose(f) == 0;
@@ -116,6 +119,7 @@ extern "C" bz_status bz_autotune(bz_ctx* ctx, uint32_t kernel, const bz_view_job
     };
 
     std::vector<bz_tuning> cands;
+    if (kernel == 0) cands.push_back(kBuiltInTuning);
     const uint32_t per_cu[] = { 0, 1, 2, 4 };
     for (uint32_t b : { 256u, 512u })
         for (uint32_t i : { 2u, 4u })

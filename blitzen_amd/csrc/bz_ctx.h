@@ -154,6 +154,8 @@ struct ExtSem {
     ~ExtSem();  // interop.cpp
 };
 
+constexpr bz_tuning kBuiltInTuning{ 512, 2, 0, BZ_TUNING_BY_SIZE };  // kernel 0
+
 struct Ctx {
     int device = 0;
     uint32_t n_cu = 0;
@@ -172,7 +174,6 @@ struct Ctx {
     bz_tuning tune[2] = {};
     // The tuning of one single-view pass over n objects: tune[0], or where that is the built-in one, the choice by n.
     bz_tuning pass_tuning(uint32_t n) const;
-    bool built_in_tuning() const;
     bool one_launch(uint32_t n) const;  // such a pass goes in one launch (launch_fused)
     std::unique_ptr<Server> server;
     void* noalloc_scratch = nullptr;  // device address of this device's fixed scratch (bz_cull_noalloc)

@@ -318,25 +318,17 @@ uint32_t tiles_for(uint32_t n, uint32_t block, uint32_t items)
     return t ? (uint32_t)t : 1u;
 }
 
-constexpr bz_tuning kBuiltInTuning{ 512, 2, 0, 0 };
-
 // Two objects a thread up to 2^21 objects, four above. Four are better where the streams bound the pass and the objects
 // in view are spread over all tiles: a wave's compacted LOD selection then runs on twice the lanes (4 194 304 objects at
 // random with the frame cache 59.2 against 62.8 us, PLAIN of 12 000 000 57.9 against 73.3; 2 000 000 only 41.8 against 42.8).
 // Where neighbouring ids are neighbours in space, a tile is all in view or not at all, and a wave works through its
 // survivors 64 at a time: half as many per wave spread them better (2 000 000 in region order 41.7 against 49.9 us, 1 048 576
 // 34.0 against 38.7, 600 000 30.7 against 34.3).
-bool Ctx::built_in_tuning() const
-{
-    const bz_tuning &t = tune[0], &d = kBuiltInTuning;
-    return t.block == d.block && t.items == d.items && t.grid_per_cu == d.grid_per_cu;
-}
-
-bool Ctx::one_launch(uint32_t n) const { return n <= kFuseObjects && built_in_tuning(); }
+bool Ctx::one_launch(uint32_t n) const { return n <= kFuseObjects && tune[0].reserved == BZ_TUNING_BY_SIZE; }
 
 bz_tuning Ctx::pass_tuning(uint32_t n) const
 {
-    if (!built_in_tuning()) return tune[0];
+    if (tune[0].reserved != BZ_TUNING_BY_SIZE) return tune[0];
     if (one_launch(n)) return bz_tuning{ kFuseBlock, kFuseItems, 0, 0 };
     return n <= (1u << 21) ? bz_tuning{ 256, 2, 0, 0 } : bz_tuning{ 256, 4, 0, 0 };
 }

@@ -289,8 +289,9 @@ class Context:
         cap = cmds.nbytes // 24 if capacity is None else capacity
         return cmds.download(INDIRECT_DRAW, min(n, cap), stream), n
 
-    def set_tuning(self, kernel: int, block: int, items: int, grid_per_cu: int = 0):
-        t = A.Tuning(block=block, items=items, grid_per_cu=grid_per_cu)
+    def set_tuning(self, kernel: int, block: int, items: int, grid_per_cu: int = 0, reserved: int = 0):
+        """`reserved`: A.TUNING_BY_SIZE puts kernel 0's built-in choice by the number of objects back in force."""
+        t = A.Tuning(block=block, items=items, grid_per_cu=grid_per_cu, reserved=reserved)
         self.check(lib().bz_set_tuning(self.handle, kernel, C.byref(t)), "bz_set_tuning")
 
     def autotune(self, kernel: int, jobs: list[A.ViewJob], cache_path: str | None = None, stream=None) -> A.Tuning:

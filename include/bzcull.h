@@ -364,8 +364,12 @@ typedef struct bz_tuning {
     uint32_t block;           /* threads per workgroup: 256 or 512 */
     uint32_t items;           /* objects per thread:    2 or 4     */
     uint32_t grid_per_cu;     /* workgroups per CU for the persistent decide kernel; 0 = as many as fit */
-    uint32_t reserved;
+    uint32_t reserved;        /* BZ_TUNING_BY_SIZE, or 0 */
 } bz_tuning;
+/* Kernel 0's built-in tuning: bz_cull chooses by the number of objects (the other passes use block, items and
+ * grid_per_cu). bz_get_tuning reports it as {512, 2, 0, BZ_TUNING_BY_SIZE}; set with this value it is in force again.
+ * Without it a tuning is taken as it is. */
+#define BZ_TUNING_BY_SIZE 1u
 
 /* Culls every job in one launch pair (decide + emit over the jobs' concatenated tiles). Each job's output
  * equals what bz_cull gives for it alone. Jobs with no objects only get their count zeroed. The job table
@@ -391,11 +395,11 @@ BZ_API bz_status bz_check(bz_ctx* ctx, void* stream);
 #define BZ_DEFAULT_WAIT_LIMIT 1048576u
 BZ_API bz_status bz_set_wait_limit(bz_ctx* ctx, uint32_t sleeps);
 /* Tuning used by bz_cull (kernel 0) and bz_cull_batch (kernel 1); defaults are built in, bz_autotune
- * replaces them. With the built-in one for kernel 0 (512, 2, 0), bz_cull chooses by the number of objects. */
+ * replaces them. */
 BZ_API bz_status bz_get_tuning(bz_ctx* ctx, uint32_t kernel /* 0 = single view, 1 = batched */, bz_tuning* out);
 BZ_API bz_status bz_set_tuning(bz_ctx* ctx, uint32_t kernel, const bz_tuning* t);
 /* Times every candidate tuning (block 256/512 x items 2/4, and for kernel 0 a persistent grid of 0, 1, 2
- * or 4 workgroups per CU) on the given jobs with HIP events and keeps the fastest; results are identical for
+ * or 4 workgroups per CU, and the built-in choice by the number of objects) on the given jobs with HIP events and keeps the fastest; results are identical for
  * every candidate. The jobs run repeatedly, so a LATE job should write its visibility out of place. If
  * cache_path is not NULL the choice is read from / written to that JSON file, keyed by device name, kernel
  * and floor(log2(total objects)); a cached entry is used without timing. */
