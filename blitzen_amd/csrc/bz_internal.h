@@ -89,6 +89,7 @@ constexpr uint32_t kRegionTile = 2;         // texels of the last level per work
 constexpr uint32_t kRegionLevels = 5;       // at most this many levels in the regions
 constexpr uint32_t kRegionMax = 48;         // a region's widest levels 0, 2, 4 (half of it: levels 1, 3)
 constexpr uint32_t kRegionTail = 8192;      // texels of the last level, held by the tail workgroup
+constexpr uint32_t kRegionFew = 6400;       // and with fewer than ten levels (plan_pyramid)
 struct PyrRegion {
     uint32_t begin, end, need;
 };

@@ -298,10 +298,15 @@ bool plan_pyramid(uint32_t base_w, uint32_t base_h, uint32_t mips, PyrPlan* p)
     // single pass: power-of-two extent, and the tile image's first reduction fits the tail workgroup's LDS tile
     const uint64_t tail_texels = (uint64_t)std::max(1u, p->tiles_x / 2u) * std::max(1u, p->tiles_y / 2u);
     p->single_pass = pow2 && (p->tile_levels >= mips || tail_texels <= kPyrTailTexels);
-    if (!p->single_pass) {  // the regions of the last level must all reach one workgroup's LDS
+    // Regions: the texels of the last level must all reach one workgroup's LDS, and there are a quarter as many workgroups.
+    // With many of them a build is slower than a launch per level unless that takes ten (1920 x 1080, 8040 texels: 6
+    // levels 25.4 us against 20.7, 8 levels 26.5 against 24.6, 11 levels 28.0 against 30; 960 x 540, 4 levels 12.9
+    // against 12.4; 1700 x 950, 6254 texels: 5 levels 18.2 against 20.9, 8 levels 24.0 against 26.7). One level is one
+    // launch either way (120 x 68: 5.7 us by regions, 3.4 by texels).
+    if (!p->single_pass && mips > 1u) {
         const uint32_t K = std::min(kRegionLevels, mips) - 1u;
         const uint32_t w = level_dim(base_w, K), h = level_dim(base_h, K);
-        if ((uint64_t)w * h <= kRegionTail) {
+        if ((uint64_t)w * h <= (mips < 10u ? kRegionFew : kRegionTail)) {
             p->region = true;
             p->tile_levels = K + 1u;
             p->tiles_x = (w + kRegionTile - 1u) / kRegionTile;
