@@ -27,6 +27,7 @@ __device__ __forceinline__ float min4(float a, float b, float c, float d)
 }
 
 typedef float float4_unaligned __attribute__((ext_vector_type(4), aligned(4)));  // one 16-byte load at any dword
+typedef float float2_unaligned __attribute__((ext_vector_type(2), aligned(4)));  // one 8-byte load at any dword
 
 // A quad_perm of the four lanes of each quad.
 template <int A, int B, int C, int D>
@@ -129,9 +130,26 @@ __device__ __forceinline__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile
             b1 = pick(p, e.x1 - xs);
             b2 = pick(q, e.x0 - xs);
             b3 = pick(q, e.x1 - xs);
-        } else {
-            a0 = r0[f.x0], a1 = r0[f.x1], a2 = r1[f.x0], a3 = r1[f.x1];
-            b0 = r0[e.x0], b1 = r0[e.x1], b2 = r1[e.x0], b3 = r1[e.x1];
+        } else if (J.w >= 2u) {
+            // More depth texels per base texel: each footprint's two texels of a row as one 8-byte load, which starts a
+            // texel early where the footprint is the row's last one. With eight 4-byte loads a 4096 x 4096 depth onto
+            // 1024 x 1024 took 13.2 us, and 10.4 for one level only; now 9.2 and 5.8.
+            const uint32_t xa = f.x0 < J.w - 2u ? f.x0 : J.w - 2u, xe = e.x0 < J.w - 2u ? e.x0 : J.w - 2u;
+            const float2_unaligned p = *reinterpret_cast<const float2_unaligned*>(r0 + xa);
+            const float2_unaligned q = *reinterpret_cast<const float2_unaligned*>(r1 + xa);
+            const float2_unaligned u = *reinterpret_cast<const float2_unaligned*>(r0 + xe);
+            const float2_unaligned v = *reinterpret_cast<const float2_unaligned*>(r1 + xe);
+            a0 = f.x0 > xa ? p.y : p.x;
+            a1 = f.x1 > xa ? p.y : p.x;
+            a2 = f.x0 > xa ? q.y : q.x;
+            a3 = f.x1 > xa ? q.y : q.x;
+            b0 = e.x0 > xe ? u.y : u.x;
+            b1 = e.x1 > xe ? u.y : u.x;
+            b2 = e.x0 > xe ? v.y : v.x;
+            b3 = e.x1 > xe ? v.y : v.x;
+        } else {  // a depth image one texel wide
+            a0 = a1 = b0 = b1 = r0[0];
+            a2 = a3 = b2 = b3 = r1[0];
         }
         if (x0 < bw && y0 < bh) ta = min4(a0, a1, a2, a3);
         if (x0 + 1u < bw && y0 < bh) tb = min4(b0, b1, b2, b3);
