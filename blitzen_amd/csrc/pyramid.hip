@@ -158,6 +158,7 @@ __device__ __forceinline__ void pyramid_tile(const PyrBuildJob& J, uint32_t tile
         if (x0 + 1u < bw) *reinterpret_cast<float2*>(J.texels + (size_t)y0 * bw + x0) = make_float2(ta, tb);
         else if (x0 < bw) J.texels[(size_t)y0 * bw + x0] = ta;  // a base one texel wide
     }
+    if (J.mips == 1u) return;
     // ---- levels 1 and 2: (x1, y0 / 2) >> (L - 1) is the lane's texel of level L, stored by the first lane of its group
     const uint32_t levels = J.tile_levels;
     auto store = [&](uint32_t L, uint32_t x, uint32_t y, float t) {
