@@ -217,6 +217,7 @@ inline bz_status upload_table(Ctx* ctx, T*& dev, T*& host, uint32_t& cap, hipEve
 {
     (void)hipEventSynchronize(wait);
     if (cap < n) {
+        (void)hipStreamSynchronize(st);  // `wait` is behind the last copy, not behind the kernels that read the table
         if (dev) (void)hipFree(dev);
         if (host) (void)hipHostFree(host);
         dev = nullptr;
