@@ -57,3 +57,23 @@ def test_few_jobs(views, graph):
             j.check(ctx, None if j.pyr is None else oracle_pyramid(buf, bw, bh, mips, w, hh))
     finally:
         ctx.close()
+
+
+def test_table_grows_behind_a_running_batch():
+    """A batch of large jobs, and without waiting for it one of far more jobs, whose table has to grow."""
+    ctx = bz.Context(0)
+    try:
+        n = 600000
+        sc = H.as_tuple(H.c1_scene(n, seed=3))
+        h = ctx.scene_create(*sc)
+        s = ctx.stream()
+        large = [Job(ctx, h, sc, H.view(yaw=0.3 * k), A.PASS_PLAIN, begin=0, count=n) for k in range(13)]
+        small = [Job(ctx, h, sc, H.view(yaw=0.01 * k), A.PASS_PLAIN, begin=11 * k, count=300 + k) for k in range(300)]
+        ctx.sync()
+        for jobs in (large, small):
+            ctx.cull_batch([j.vj for j in jobs], stream=s)
+        ctx.check_kernels(s)
+        for j in large[::4] + small[::29]:
+            j.check(ctx, None)
+    finally:
+        ctx.close()
