@@ -183,7 +183,6 @@ struct Ctx {
 
     bz_status fail(bz_status s, const std::string& what);
     bz_status hip_fail(hipError_t e, const char* what);
-    void free_later(void* p);
     Scene* scene(bz_scene h);
     Pyramid* pyramid(bz_pyramid h);
     bz_status scratch_for(hipStream_t st, uint32_t tiles, uint64_t entries, StreamScratch** out);
@@ -195,7 +194,6 @@ struct Ctx {
     // Jobs with objects go to `out` (tile_start set); the count buffers of jobs with none go to `empty`.
     bz_status make_batch(const bz_view_job* jobs, uint32_t n_jobs, const bz_tuning& t, std::vector<CullJob>& out,
                          std::vector<uint32_t*>& empty, uint32_t* total_tiles);
-    uint32_t batch_grid(const bz_tuning& t, uint32_t total_tiles) const;
     bz_status upload_jobs(StreamScratch* sc, const CullJob* jobs, uint32_t n, hipStream_t st);
     bz_status upload_pjobs(StreamScratch* sc, const PyrBuildJob* jobs, uint32_t n, hipStream_t st);
     bz_status build_pyramid(Pyramid* p, const float* depth, uint32_t w, uint32_t h, hipStream_t st);

@@ -50,11 +50,6 @@ bz_status Ctx::hip_fail(hipError_t e, const char* what)
     return fail(e == hipErrorOutOfMemory ? BZ_E_OOM : BZ_E_HIP, m);
 }
 
-void Ctx::free_later(void* p)
-{
-    if (p) (void)hipFree(p);
-}
-
 Scene* Ctx::scene(bz_scene h)
 {
     auto it = scenes.find(h);
@@ -1343,13 +1338,6 @@ static hipError_t zero_counts(const std::vector<uint32_t*>& empty, hipStream_t s
     for (uint32_t* c : empty)
         if (e == hipSuccess) e = launch_fill_u32(c, 0u, 1, st);
     return e;
-}
-
-uint32_t Ctx::batch_grid(const bz_tuning& t, uint32_t total_tiles) const
-{
-    uint64_t g = (uint64_t)n_cu * std::max<uint32_t>(t.grid_per_cu, 1u);
-    if (g > total_tiles) g = total_tiles;
-    return g ? (uint32_t)g : 1u;
 }
 }  // namespace bz
 

@@ -302,12 +302,7 @@ __global__ __launch_bounds__(kXBlock) void cluster_emit_kernel(ClusterJob J, con
         for (uint32_t u = 0; u < kCEmitUnroll; ++u) {
             const uint32_t e = e0 + u * 64u + lane;
             const uint32_t pos = out0 + e;
-            if (e < c && pos < J.capacity) {
-                uint2* cmd = reinterpret_cast<uint2*>(J.cmds + (size_t)pos * 6u);
-                cmd[0] = make_uint2(ent[u].x, d[u].x);  // objectId, indexCount
-                cmd[1] = make_uint2(1u, d[u].y);         // instanceCount, firstIndex
-                cmd[2] = make_uint2(0u, 0u);             // vertexOffset, firstInstance
-            }
+            if (e < c && pos < J.capacity) write_command(J.cmds, pos, ent[u].x, d[u]);
         }
     }
 }
