@@ -34,9 +34,12 @@ DEPTH_W, DEPTH_H, OCCLUDERS = 1920, 1080, 512
 PYR_W, PYR_H, PYR_MIPS = 1024, 512, 11
 SEED = 0xB1172E01
 HBM_PEAK_GBS = 8000.0
+# the frame's algorithmic bytes, of the reference's records:
 LATE_BYTES_PER_OBJECT = 48  # RenderObject 8 + MeshTransform 32 + visibility read 4 + write 4
 EARLY_BYTES_PER_OBJECT = 4  # visibility read; + 40 B per last-frame-visible object
 CMD_BYTES = 24
+# the other legs': what a pass reads of an object here, its world-space sphere and its (16-bit) surface id
+OBJECT_BYTES = 18
 
 
 def log(msg: str):
@@ -253,9 +256,9 @@ def bench_clusters(ctx, stream, steps: int, warmup: int):
     ctx.sync(stream)
     ctx.check_kernels(stream)
     cull_ms = c0.elapsed_ms(c1) / steps
-    # algorithmic bytes of the cull: object pass 40 B per object (RenderObject 8 + transform 32), per record 12 B
+    # algorithmic bytes of the cull: object pass 18 B per object (sphere, surface id), per record 12 B
     # written and 12 B read back + 20 B of cluster data (sphere, cone), 24 B per draw, two counts
-    cull_bytes = cf.n_objects * 40 + records * (12 + 12 + 20) + draws * 24 + 8
+    cull_bytes = cf.n_objects * OBJECT_BYTES + records * (12 + 12 + 20) + draws * 24 + 8
     out = {"workload": "1,048,576 objects over 128 surfaces x 8 LODs with 16-128 clusters of 64 triangles (LOD k "
                        "owns max(1, c >> 2k)); per frame 1% seeded transform updates (10,485 x 32 B uploaded) + object "
                        "pass (frustum + LOD, as PreClusterDrawCull) + expansion + cluster frustum/Hi-Z/cone tests "
@@ -308,7 +311,7 @@ def bench_next_rows(ctx, stream, scenes, view, transforms, steps: int):
         ms, _ = timed(lambda k: ctx.cull(scenes[k % len(scenes)], view, pass_, cmds, cnt, capacity=N_OBJECTS,
                                          stream=stream))
         n = int(cnt.download(np.uint32, 1, stream)[0])
-        out[name] = row(ms, N_OBJECTS * 40 + n * CMD_BYTES + 4, {"commands": n})
+        out[name] = row(ms, N_OBJECTS * OBJECT_BYTES + n * CMD_BYTES + 4, {"commands": n})
     # LOD-instanced: every LOD's list has room for 8192 instances (the largest list here holds a few thousand)
     n_lods = N_SURFACES * N_LODS
     per_lod = 8192
@@ -319,7 +322,7 @@ def bench_next_rows(ctx, stream, scenes, view, transforms, steps: int):
     k_cmds = int(icnt.download(np.uint32, 1, stream)[0])
     ctr = counters.download(np.uint32, n_lods * 2, stream).reshape(-1, 2)
     inst = int(ctr[:, 1].sum())
-    out["instanced"] = row(ms, N_OBJECTS * 40 + inst * 4 + n_lods * 8 + k_cmds * 32 + 4,
+    out["instanced"] = row(ms, N_OBJECTS * OBJECT_BYTES + inst * 4 + n_lods * 8 + k_cmds * 32 + 4,
                            {"instances": inst, "lod_commands": k_cmds, "instances_per_lod": per_lod,
                             "largest_list": int(ctr[:, 1].max())})
     # transform streaming: 1% of the transforms per call (ids + 32-byte transforms from host arrays)
@@ -355,9 +358,9 @@ def bench_next_rows(ctx, stream, scenes, view, transforms, steps: int):
 
 def bench_size_scaling(ctx, stream, view, steps: int, copies: int = 2):
     """The PLAIN pass of one job at 4, 8 and 16 M objects (ranges [0, n) of two resident 16 M-object scenes, used
-    in turn so that a range is not cache-resident between launches). The pass is decide + emit; a job of more than
-    4096 tiles also scans its tile counts, so that every emit workgroup reads its output offset instead of re-summing
-    the earlier tiles' counts. Time per million objects stays flat when the emit is linear in the object count."""
+    in turn so that a range is not cache-resident between launches). The pass is decide + emit, whose workgroups add up
+    the earlier tiles' counts; a job of more than 32 768 tiles scans them instead. Time per million objects stays flat
+    when the emit is linear in the object count."""
     import numpy as np
 
     from blitzen_amd import _capi as A
@@ -386,7 +389,7 @@ def bench_size_scaling(ctx, stream, view, steps: int, copies: int = 2):
         ctx.check_kernels(stream)
         us = e0.elapsed_ms(e1) / steps * 1e3
         n_cmd = int(cnt.download(np.uint32, 1, stream)[0])
-        alg = n * 40 + n_cmd * CMD_BYTES + 4
+        alg = n * OBJECT_BYTES + n_cmd * CMD_BYTES + 4
         out["sizes"].append({"objects": n, "tiles": n // 1024, "scanned_prefix": n // 1024 > 32768,
                              "us": round(us, 2), "us_per_mobject": round(us / (n / 1048576), 3), "commands": n_cmd,
                              "achieved_gbs": round(alg / (us * 1e-6) / 1e9, 1)})

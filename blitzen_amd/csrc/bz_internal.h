@@ -71,10 +71,12 @@ inline void set_prefix(CompactScratch& s, bool batches)
     s.tile_job = s.counts && batches ? s.prefix + s.capacity_tiles + 1u : nullptr;
 }
 
-// An emit workgroup adds the counts of its job's earlier tiles itself when there are at most kScanTiles of them (one
-// round of loads), and in a launch of its own shape also beyond (kEmitSumTiles). Batches and cluster passes with more
-// tiles get their exclusive prefix from one scan launch between the decide and the emit instead, so that the work per
-// workgroup stays constant and the pass stays linear in the object count.
+// The counts of a job's earlier tiles are added up where its commands are written when there are at most kScanTiles of them
+// (one round of loads of a workgroup; four of a wave, in the batched emit), and in a launch of its own shape also beyond
+// (kEmitSumTiles). Batches and cluster passes with more tiles get their exclusive prefix from one scan launch between the
+// decide and the emit instead, so that the work per workgroup stays constant and the pass stays linear in the object count.
+// Batches with the scan / without, us: 13 jobs of 1024 tiles 82.0 / 77.8, of 2048 153.7 / 147.1, of 4096 308.4 / 300.9;
+// 4 jobs of 5860 tiles 137.5 / 138.3, of 8192 185.6 / 191.7: the lines cross between 4096 and 5860.
 constexpr uint32_t kScanTiles = 4096;
 // Exclusive prefix of counts[0, n) into prefix[0, n], prefix[n] = the total (one workgroup, linear in n).
 hipError_t launch_scan_counts(const uint32_t* counts, uint32_t n, uint32_t* prefix, hipStream_t st);
@@ -130,9 +132,9 @@ hipError_t launch_cull(const CullJob& job, const CompactScratch& s, uint32_t blo
                        uint32_t per_cu, hipStream_t st, const FrameCacheDev* cache = nullptr);
 // One launch for the whole pass over at most kFuseObjects objects, tiles of kFuseBlock x kFuseItems: each workgroup adds
 // up the counts that the tiles before it publish, instead of an emit launch. That trades a launch (about 2 us, and as long
-// on the host) for a wait on the slowest earlier tile, which grows with the tiles: PLAIN of 131 072 objects 9.3 -> 6.9 us,
-// of 330 000 10.5 -> 8.7; EARLY + pyramid + LATE of 1000 objects 20 -> 15.7, of 262 144 27.5 -> 26.0, of 330 000 in region
-// order 28.4 -> 28.6, of 380 000 28.6 -> 29.5: the line is 640 tiles. wait_limit: looks at a count not there yet before a
+// on the host) for a wait on the slowest earlier tile, which grows with the tiles: PLAIN of 131 072 objects 9.4 -> 6.9 us,
+// of 327 680 10.1 -> 8.6; EARLY + pyramid + LATE of 1000 objects 25.0 -> 21.9, of 262 144 27.7 -> 24.4, of 327 680 28.4 ->
+// 26.0, in region order 30.0 -> 29.6 (of 380 000 in region order one launch lost, 28.6 against 29.5): the line is 640 tiles. wait_limit: looks at a count not there yet before a
 // tile leaves its commands to the last one (at most kFusePatience, some milliseconds).
 constexpr uint32_t kFuseBlock = 256, kFuseItems = 2;
 constexpr uint32_t kFuseObjects = 5u << 16;

@@ -372,9 +372,9 @@ typedef struct bz_tuning {
 #define BZ_TUNING_BY_SIZE 1u
 
 /* Culls every job in one launch pair (decide + emit over the jobs' concatenated tiles). Each job's output
- * equals what bz_cull gives for it alone. Jobs with no objects only get their count zeroed. The job table
- * of more than a dozen jobs is staged through a context-owned pinned buffer, so this call cannot be stream-captured:
- * capture a fixed batch with bz_batch_graph_create instead. Jobs that write one visibility buffer in overlapping ranges race. */
+ * equals what bz_cull gives for it alone. Jobs with no objects only get their count zeroed. The call cannot be
+ * stream-captured (BZ_E_STATE), whatever the number of jobs: the job table of a larger batch goes through a
+ * context-owned pinned buffer. Capture a fixed batch with bz_batch_graph_create instead. Jobs that write one visibility buffer in overlapping ranges race. */
 BZ_API bz_status bz_cull_batch(bz_ctx* ctx, const bz_view_job* jobs, uint32_t n_jobs, void* stream);
 /* Synchronizes `stream` and reports BZ_E_INTERNAL if a kernel launched on it gave up a bounded wait
  * since the last check (the flag is then cleared): a pyramid build, the scan of bz_cull_instanced, or a bz_cull or
