@@ -126,9 +126,14 @@ __device__ __forceinline__ bool fuse_prefix(const FuseDev& fuse, uint32_t launch
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_s_waitcnt(0);
         left = __hip_atomic_load(mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == 0) {  // each workgroup has read the launch's number: it moves on, and a word ages
+            const uint32_t aged = fuse_aged(launch, kFuseTiles);
+            if (aged > tile) fuse_store(fuse, kFuseFirst + aged, 0u, 0u);
+            __hip_atomic_store(reinterpret_cast<uint32_t*>(fuse.words), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         return true;
     }
-    if (here) return true;
+    if (__builtin_expect(here, 1)) return true;
     const uint32_t word = kFuseFirst + kFuseTiles + tile;
     stage();
     __threadfence();
@@ -161,30 +166,22 @@ __device__ __forceinline__ void fuse_publish(const FuseDev& fuse, uint32_t launc
     fuse_store(fuse, kFuseFirst + tile, launch, count);
 }
 // By the last tile, which has had every count: its first wave writes the commands of the tiles that left theirs
-// (write(tile, first command, commands), 64 lanes), ages a word and moves the launch's number on, which each workgroup has
-// read.
+// (write(tile, first command, commands), 64 lanes).
 template <class Write>
 __device__ __forceinline__ void fuse_settle(const FuseDev& fuse, uint32_t launch, uint32_t left, uint32_t n_tiles,
                                             Write&& write)
 {
-    if (threadIdx.x >= 64u) return;
-    if (__builtin_amdgcn_readfirstlane(left) == launch) {
-        uint32_t first = 0;
-        for (uint32_t t = 0; t + 1u < n_tiles; ++t) {
-            const uint32_t count = (uint32_t)fuse_load(fuse, kFuseFirst + t);
-            uint32_t mine = 0;
-            if (threadIdx.x == 0) mine = fuse_claim(fuse, kFuseFirst + kFuseTiles + t, launch) ? 1u : 0u;
-            if (__builtin_amdgcn_readfirstlane(mine)) {
-                __threadfence();
-                write(t, first, count);
-            }
-            first += count;
+    if (threadIdx.x >= 64u || __builtin_expect(__builtin_amdgcn_readfirstlane(left) != launch, 1)) return;
+    uint32_t first = 0;
+    for (uint32_t t = 0; t + 1u < n_tiles; ++t) {
+        const uint32_t count = (uint32_t)fuse_load(fuse, kFuseFirst + t);
+        uint32_t mine = 0;
+        if (threadIdx.x == 0) mine = fuse_claim(fuse, kFuseFirst + kFuseTiles + t, launch) ? 1u : 0u;
+        if (__builtin_amdgcn_readfirstlane(mine)) {
+            __threadfence();
+            write(t, first, count);
         }
-    }
-    if (threadIdx.x == 0) {
-        const uint32_t aged = fuse_aged(launch, kFuseTiles);
-        if (aged >= n_tiles) fuse_store(fuse, kFuseFirst + aged, 0u, 0u);
-        __hip_atomic_store(reinterpret_cast<uint32_t*>(fuse.words), launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        first += count;
     }
 }
 
