@@ -632,6 +632,7 @@ def main():
                       "late": round(late_ms * 1e3, 2),
                       "frame_events": round(statistics.mean(t_frame) * 1e3, 2),
                       "frame_timed_region": round(frame_ms * 1e3, 2)},
+        "pass_gbs_bytes": "of the reference's records (the cached late pass reads its survivors' records instead)",
         "pass_gbs": {"pyramid": round(pyr_bytes / (statistics.mean(t_pyr) * 1e-3) / 1e9, 1),
                      "early": round(early_bytes / (statistics.mean(t_early) * 1e-3) / 1e9, 1),
                      "late": round(late_bytes / (late_ms * 1e-3) / 1e9, 1)},
